@@ -10,14 +10,18 @@ state resident in HBM.  Prints one JSON line:
 
   value        vertex-steps/s = N * K / (time of K steps), HIP events on the
                stream the kernels run on
-  roofline     for the dominant kernel (cg_spmv): algorithmic bytes per
-               launch (88N + 32P, the spmv share of the per-iteration model
-               160N + 32P) / its average launch time inside the step's launch
-               sequence (an event attached to every dispatch of the same
-               steps, oc_cloth_profile_steps), against 8 TB/s; the same over
-               300 back-to-back launches beside it; traffic = HBM bytes per
-               launch from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE
-               summary, and its fraction beside the model's
+  roofline     for the dominant kernel, the resident solve (one launch per CG
+               solve, matrix and vectors on chip): the bytes a solve cannot do
+               without (24P + 62N: blocks, masks, r, d, dv in, dv out) / its
+               average launch time inside the step's launch sequence (an
+               event attached to every dispatch of the same steps,
+               oc_cloth_profile_steps), against 8 TB/s.  The launch is bound
+               by its two device-wide exchanges per iteration, so beside it
+               stand the time per iteration and the per-iteration model's
+               bytes, K(160N + 32P), over the same time.  cg_spmv: the kernel
+               that larger cloths launch per iteration, over 300 back-to-back
+               launches, its algorithmic bytes (88N + 32P) and its HBM bytes
+               from the committed rocprofv3 summary
   config       the kernel split per step, and the same workload with the
                single-reduction CG
   batch        4096 uneven cloths, 200 steps, one graph-replayed launch per
@@ -55,6 +59,13 @@ def spmv_bytes(N: int, P: int) -> int:
     """Algorithmic bytes of one cg_spmv launch: symmetric blocks 24N+24P,
     topology 8P+4N, d in / q out 24N, direction update d = r + beta d 36N."""
     return 88 * N + 32 * P
+
+
+def solve_bytes(N: int, P: int) -> int:
+    """Bytes one resident solve cannot do without: blocks 24P, mask and pin
+    3N (rounded up), r, d, dv in and dv out 48N, partials and halo 11N at
+    most."""
+    return 62 * N + 24 * P
 
 
 def step_bytes(N: int, S: int, P: int, K: int) -> int:
@@ -592,10 +603,10 @@ def main():
 
         # the same steps again with every dispatch timed (same state path)
         split = kernel_split(cl, args.steps)
-        # the dominant kernel's launch time inside the step's launch sequence
-        spmv_avg_s = split["in_sequence_launch_us"]["cg_spmv"] * 1e-6
+        # the solve's launch time inside the step's launch sequence
+        solve_s = split["in_sequence_launch_us"]["cg_spmv"] * 1e-6
         spmv_b2b_s = cl.time_cg_spmv(300) * 1e-6
-        achieved = spmv_bytes(N, P) / spmv_avg_s / 1e9
+        achieved = solve_bytes(N, P) / solve_s / 1e9
         traffic = read_profile_value(os.path.join(ROOT, "profiles", "cg_spmv_512x512_pmc.txt"),
                                      "cg_spmv_hbm_bytes_per_launch")
         out.update({
@@ -621,19 +632,23 @@ def main():
                 "kernel_ms_per_step": split,
             },
             "roofline": {
-                "bound": "hbm",
-                "kernel": "cg_spmv",
+                "bound": "latency",
+                "kernel": "cg_resident (one launch per solve)",
                 "achieved": achieved,
                 "peak": HBM_PEAK_GBS,
                 "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS,
-                "traffic": traffic,
-                "algorithmic_bytes_per_launch": spmv_bytes(N, P),
-                "avg_launch_us": spmv_avg_s * 1e6,
+                "traffic": None,
+                "algorithmic_bytes_per_launch": solve_bytes(N, P),
+                "avg_launch_us": solve_s * 1e6,
+                "us_per_iteration": solve_s * 1e6 / max(K, 1),
+                "iteration_model_GBps": K * (160 * N + 32 * P) / solve_s / 1e9,
+            },
+            "cg_spmv": {
                 "avg_launch_us_back_to_back": spmv_b2b_s * 1e6,
+                "algorithmic_bytes_per_launch": spmv_bytes(N, P),
                 "frac_back_to_back": spmv_bytes(N, P) / spmv_b2b_s / 1e9 / HBM_PEAK_GBS,
-                "traffic_GBps": None if traffic is None else traffic / spmv_avg_s / 1e9,
-                "traffic_frac": None if traffic is None else traffic / spmv_avg_s / 1e9 / HBM_PEAK_GBS,
+                "traffic": traffic,
             },
         })
         cl.close()

@@ -59,7 +59,10 @@ typedef enum {
 #define OC_FLAG_CG_PERSISTENT 2 /* run all CG iterations of a solve in one cooperative
                                    launch, resident blocks serving several tiles each
                                    (same arithmetic and results, grid barriers between
-                                   phases); ignored where cooperative launch is absent */
+                                   phases); ignored where cooperative launch is absent.
+                                   Cloths whose pairs follow the reference's stencil and
+                                   that fit the device (about 512 tiles of 64x8 on MI355X)
+                                   are solved in one launch with or without it */
 #define OC_FLAG_JACOBI 4        /* Jacobi-preconditioned CG: Baraff and Witkin's modified PCG
                                    with P = diag(A), the intent of BW:308-330 and BW:784-785;
                                    the stopping tests then measure r.(P^-1 r) */
@@ -395,9 +398,9 @@ int oc_cloth_rollout_backward(oc_cloth cloth, const float* grad_x, const float* 
  * frame counter, IE:562-584): runs nsteps exactly as oc_cloth_step does
  * (same launches, same results), each kernel launched with a start and a
  * stop event attached to its own dispatch, and returns per kernel class
- * (0 assembly, 1 first CG launch of an iteration (cg_spmv), 2 second
- * (cg_axpy), 3 other solver launches, 4 update) the summed kernel
- * milliseconds and the launch counts.  ms[5], launches[5]; synchronises. */
+ * (0 assembly, 1 first CG launch of an iteration (cg_spmv) or the one launch
+ * of a whole solve, 2 second (cg_axpy), 3 other solver launches, 4 update)
+ * the summed kernel milliseconds and the launch counts.  ms[5], launches[5]; synchronises. */
 int oc_cloth_profile_steps(oc_cloth cloth, int32_t nsteps, float* ms, int32_t* launches);
 
 /* Introspection of the assembled system (for tests and tools).

@@ -158,6 +158,8 @@ namespace oc {
 
 int cloth_device(const oc_cloth_s* c) { return c->device; }
 
+const DevCloth& cloth_view(const oc_cloth_s* c) { return c->dc; }
+
 size_t cloth_partial_floats(const oc_cloth_s* c) {
     const size_t it = (size_t)std::max(c->prm.cg_max_iters, 1), nt = (size_t)c->dc.nt;
     return 2 * (it + 1) * nt + 2 * (it + 2);
@@ -309,7 +311,14 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     const size_t amask = st_asm ? align_up(sizeof(uint32_t) * N) : 0;
     const size_t cst = st_asm ? align_up(sizeof(float) * oc::kCstPlanes * N) : 0;
     const size_t scst = st_asm ? align_up(sizeof(int32_t) * S) : 0;
-    const size_t total = 17 * vec + blocks + ainc_s + ainc_m + pair_m + pair_k + 3 * sp + pin + amask + cst + scst;
+    d.stencil = t.stencil ? 1 : 0;
+    d.res_vt = oc::resident_cg_tiles(d);
+    const size_t xch = d.res_vt ? align_up(sizeof(uint64_t) * oc::resident_words(d.ntx, d.nty, d.res_vt, oc::kTileX,
+                                                                                 oc::kTileY))
+                                : 0;
+    const size_t sync = align_up(sizeof(unsigned) * 4);
+    const size_t total = 17 * vec + blocks + ainc_s + ainc_m + pair_m + pair_k + 3 * sp + pin + amask + cst + scst +
+                         xch + sync;
     if (hipMalloc(&c->arena, total) != hipSuccess) {
         delete c;
         return fail(OC_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(total) + " bytes failed");
@@ -336,7 +345,6 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     d.ainc_m = (const uint16_t*)take(ainc_m);
     d.pair_m = (const uint16_t*)take(pair_m);
     d.pair_mask = (const uint16_t*)take(pair_k);
-    d.stencil = t.stencil ? 1 : 0;
     for (int k = 0; k < oc::kStencil; k++) d.stencil_plane[k] = t.stencil_plane[k];
     d.L0 = (const float*)take(sp);
     d.ks = (const float*)take(sp);
@@ -352,6 +360,10 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     d.q2 = (float*)take(vec);
     d.s1 = (float*)take(vec);
     d.s2 = (float*)take(vec);
+    d.xslots = d.res_vt ? oc::resident_slots(d.ntx, d.nty) : 0;
+    d.xstride = d.res_vt ? oc::resident_stride(d.ntx, d.nty) : 0;
+    d.xch = d.res_vt ? (uint64_t*)take(xch) : nullptr;
+    d.sync = (unsigned*)take(sync);
 
     auto cleanup = [&](int code) {
         (void)hipFree(c->arena);

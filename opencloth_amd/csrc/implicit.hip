@@ -112,6 +112,20 @@ __device__ inline void cg_finish_block(const DevCloth& c, const StepScalars& s, 
 // ---------------------------------------------------------------------------
 // assembly + CG start
 // ---------------------------------------------------------------------------
+// Control words of the solve that follows an assembly (one thread): not done,
+// no status; for the resident solve a new roll call, barrier counter and
+// epoch base (past every tag the last resident solve used).
+__device__ inline void start_solve(const DevCloth& c) {
+    c.ctl[0] = 0;
+    c.ctl[1] = 0;
+    c.ctl[2] = 0;
+    if (c.res_vt) {
+        c.sync[0] = c.sync[3];
+        c.sync[1] = 0;
+        c.sync[2] = 0;
+    }
+}
+
 // Constants of one incident spring (gathered by spring id).
 struct SpringC {
     float L0, ks, kd;
@@ -162,11 +176,7 @@ __global__ __launch_bounds__(TX* TY) void k_assemble(DevCloth c, StepScalars s) 
         // sticky word before the control block is cleared (with UPD that
         // solve had no update launch to record them)
         if (UPD) cg_finish_block(c, s, &sh.bc);
-        if (threadIdx.x == 0) {
-            c.ctl[0] = 0;
-            c.ctl[1] = 0;
-            c.ctl[2] = 0;
-        }
+        if (threadIdx.x == 0) start_solve(c);
     }
     // own slot tables and the first springs' constants, then the window
     int sps[WA];
@@ -354,11 +364,7 @@ __global__ __launch_bounds__(TX* TY, 4) void k_assemble_st(DevCloth c, StepScala
     const int N = c.N, nx = c.nx, i = gj * nx + gi;
     if (blockIdx.x == 0) {
         if (UPD) cg_finish_block(c, s, &sh.bc);
-        if (threadIdx.x == 0) {
-            c.ctl[0] = 0;
-            c.ctl[1] = 0;
-            c.ctl[2] = 0;
-        }
+        if (threadIdx.x == 0) start_solve(c);
     }
     auto own_cst = [&](int m, int o, int q, int g) {
         return ldo(c.cst, (uint32_t)(((m * kOwned + o) * 3 + q) * N + g));
@@ -609,7 +615,9 @@ struct SpmvShared {
 // cloth's pairs follow the kStencil order (c.stencil), so a 12-bit mask per
 // vertex replaces the WP slot metas and every slot's offset, owner and plane
 // are constants; the sums run in the same pair order either way.
-template <int TX, int TY, int WP, bool STENCIL = false>
+// LEAN (stencil form): the blocks are read as they are used instead of up
+// front, for a kernel whose registers the hoisted form would spill.
+template <int TX, int TY, int WP, bool STENCIL = false, bool LEAN = false>
 __device__ inline bool spmv_phase(const DevCloth& c, const StepScalars& s, int k, bool read_done,
                                   SpmvShared<TX, TY>& sh, int vb) {
     constexpr int NT = TX * TY;
@@ -652,24 +660,25 @@ __device__ inline bool spmv_phase(const DevCloth& c, const StepScalars& s, int k
             }
         }
     }
-    constexpr int NS = STENCIL ? kStencil : WP;
+    constexpr int NS = LEAN ? 1 : STENCIL ? kStencil : WP;
     uint16_t m[NS];
     float C[NS][6];
-    if constexpr (STENCIL) {
+    auto stencil_block = [&](int k, float (&b)[6]) {
+        const int di = stencil_di(k), dj = stencil_dj(k);
+        const uint32_t blk = stencil_owner(k) ? (uint32_t)i : (uint32_t)(i + dj * c.nx + di);
+        const uint32_t off = blk + (uint32_t)c.stencil_plane[k] * 6u * (uint32_t)N;
+        if ((mask >> k) & 1u) {
 #pragma unroll
-        for (int k = 0; k < kStencil; k++) {
-            const int di = stencil_di(k), dj = stencil_dj(k);
-            const uint32_t blk = stencil_owner(k) ? (uint32_t)i : (uint32_t)(i + dj * c.nx + di);
-            const uint32_t off = blk + (uint32_t)c.stencil_plane[k] * 6u * (uint32_t)N;
-            if ((mask >> k) & 1u) {
+            for (int q = 0; q < 6; q++) b[q] = ldo(c.blocks, off + (uint32_t)(q * N));
+        } else {
 #pragma unroll
-                for (int q = 0; q < 6; q++) C[k][q] = ldo(c.blocks, off + (uint32_t)(q * N));
-            } else {
-#pragma unroll
-                for (int q = 0; q < 6; q++) C[k][q] = 0.0f;
-            }
+            for (int q = 0; q < 6; q++) b[q] = 0.0f;
         }
-    } else {
+    };
+    if constexpr (STENCIL && !LEAN) {
+#pragma unroll
+        for (int k = 0; k < kStencil; k++) stencil_block(k, C[k]);
+    } else if constexpr (!STENCIL) {
 #pragma unroll
         for (int sl = 0; sl < WP; sl++) {
             m[sl] = (own && sl < c.wp) ? ldo(c.pair_m, (uint32_t)(sl * N + i)) : kEmptySlot;
@@ -739,7 +748,8 @@ __device__ inline bool spmv_phase(const DevCloth& c, const StepScalars& s, int k
                 if (!((mask >> k) & 1u)) continue;
                 const int wy = ly + H + stencil_dj(k), wx = lx + H + stencil_di(k);
                 V3 w = {sh.wd[0][wy][wx] - di.x, sh.wd[1][wy][wx] - di.y, sh.wd[2][wy][wx] - di.z};
-                V3 a = symmv(C[k], w);
+                if constexpr (LEAN) stencil_block(k, C[0]);
+                V3 a = symmv(C[LEAN ? 0 : k], w);
                 acc = {acc.x + a.x, acc.y + a.y, acc.z + a.z};
             }
         } else {
@@ -1089,12 +1099,96 @@ __global__ __launch_bounds__(TX* TY) void k_cg_axpy(DevCloth c, StepScalars s, i
     axpy_phase<TX, TY>(c, s, k, true, ws, bc, blockIdx.x);
 }
 
-// Grid barrier of the persistent solve: every block adds 1 to *bar and waits
-// until it reaches target.  The add is a release (the block's writes reach
-// the device-coherent level first); the wait polls with relaxed agent-scope
-// loads, which read the coherent value without invalidating caches, and a
-// single acquire fence follows.  The wait is bounded; on time-out the block
-// sets ctl[4] and the caller ends the kernel, so every wave exits.
+// ---------------------------------------------------------------------------
+// resident CG: a whole solve in one launch, the pair blocks in registers
+// ---------------------------------------------------------------------------
+// Every block keeps a region of TX x (TY VT) vertices for the whole solve:
+// each thread holds VT vertices' pair blocks, r, q and solution in registers
+// and the region's d with its halo sits in LDS, so an iteration reads no
+// matrix and no vector from memory.  What blocks tell each other goes
+// through memory as 8-byte words (value, tag) that are stored and polled with
+// relaxed device-scope accesses: a word is its own flag, so no fence (which
+// on MI355X writes back the XCD's L2) and no barrier counter is needed.
+// Two exchanges per iteration, as the recurrence has two reductions:
+//   alpha : the tiles' d.q partials
+//   beta  : the tiles' r.z partials, and z of the region's outer two rows and
+//           columns, from which the neighbours form their halo's d
+// The tag of exchange n of a solve is the solve's epoch base + n + 1.  A block
+// publishes exchange n + 1 only after it has read all of exchange n, and
+// every exchange needs every block's partials; so when a block publishes
+// n + 2 all have read n, and two sets of partials and one set of rims are
+// enough.  Partials are stored once per XCD (8 copies, 8 lanes) in tile
+// order, and a block polls its own XCD's copy.
+// The partials are summed in tile order exactly as the per-iteration launches
+// sum them.
+//
+// The blocks wait for each other, so they must run at the same time.  They
+// are launched one per CU at most, but another stream's or process's work may
+// hold some CUs: thread 0 of each block signs in, and the blocks take the
+// resident path once all have.  If they have not within kRollCallTicks, the
+// roll is closed; the blocks signed in by then run the solve with the
+// per-iteration code below (memory-based phases, a barrier between them) and
+// later ones leave.  So the launch needs no cooperative launch (20 us each,
+// measured) and cannot wait for a block that never starts.
+//
+// Measured per iteration (30 to 40 iterations, two launches per iteration
+// before): 512x512 16.3 -> 7.1 us, 256x256 about 9 -> 4.3, 128x128 9.7 -> 3.9,
+// 21x21 7.1 -> 3.6.  An exchange takes 1.0 us between a few blocks and 1.7 to
+// 2.4 us among 256 (store to the coherence point, then polled loads of 512
+// words); the rest at 512x512, 2.9 us, is the arithmetic: 16 waves per CU
+// issue about 200 instructions each per iteration.
+constexpr unsigned kRollClosed = 1u << 15;       // count in bits 0-14, team size in bits 16-30
+constexpr unsigned long long kRollCallTicks = 50000;  // 0.5 ms of the 100 MHz counter
+constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
+
+// v, opaque to the compiler: what is computed from it is not moved ahead of
+// the iteration loop, where the exchange's few dozen addresses would spill.
+__device__ inline unsigned here(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// Word i of the exchange, from a uniform base and a 32-bit offset.
+__device__ inline uint64_t xch_load(const uint64_t* p, unsigned i) {
+    return __hip_atomic_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(p) + here(i * 8u)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void xch_store(uint64_t* p, unsigned i, unsigned tag, float v) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(p) + here(i * 8u)),
+                       ((uint64_t)tag << 32) | (uint64_t)__float_as_uint(v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sign in (one thread per block); returns this block's rank, or -1 when the
+// roll is closed.
+__device__ inline int roll_call_sign(unsigned* roll) {
+    const unsigned w = __hip_atomic_fetch_add(roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return (w & kRollClosed) ? -1 : (int)(w & (kRollClosed - 1));
+}
+// Team size once decided: all nb blocks, or those signed in when the roll was
+// closed.  The word decides: a close only succeeds on a word whose count is
+// below nb, and once the count has reached nb no block closes it.
+__device__ inline int roll_call_wait(unsigned* roll, int nb) {
+    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+    for (;;) {
+        unsigned w = __hip_atomic_load(roll, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (w & kRollClosed) return (int)(w >> 16);
+        const unsigned n = w & (kRollClosed - 1);
+        if ((int)n >= nb) return nb;
+        if (__builtin_amdgcn_s_memrealtime() - t0 > kRollCallTicks)
+            __hip_atomic_compare_exchange_strong(roll, &w, w | kRollClosed | (n << 16), __ATOMIC_RELAXED,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+// Grid barrier of the blocks of a team (also the persistent solve): every
+// block adds 1 to *bar and waits until it reaches target.  The add is a
+// release (the block's writes reach the device-coherent level first); the
+// wait polls with relaxed agent-scope loads, which read the coherent value
+// without invalidating caches, and a single acquire fence follows.  The wait
+// is bounded; on time-out the block sets ctl[4] and the caller ends the
+// kernel, so every wave exits.
 __device__ inline bool grid_barrier(unsigned* bar, unsigned target, int* err) {
     __syncthreads();
     __shared__ int ok;
@@ -1117,32 +1211,440 @@ __device__ inline bool grid_barrier(unsigned* bar, unsigned target, int* err) {
     return ok != 0;
 }
 
-// All CG iterations in one cooperative launch: the spmv and axpy phases of
-// the multi-kernel form, separated by grid barriers instead of kernel
-// boundaries.  Each resident block serves tiles blockIdx.x, +gridDim.x, ...
-// with the same per-tile code.  Every block owns at least one tile and so
-// takes the same stop decisions as the others: all blocks pass the same
-// barriers.
+// All CG iterations by a team of co-resident blocks: the spmv and axpy phases
+// of the multi-kernel form, separated by grid barriers instead of kernel
+// boundaries.  Block `rank` of `team` serves tiles rank, rank + team, ... with
+// the same per-tile code.  Every block owns at least one tile and so takes
+// the same stop decisions as the others: all blocks pass the same barriers.
+// Returns false when a barrier timed out.
+template <int TX, int TY, int WP, bool STENCIL>
+__device__ inline bool cg_team(const DevCloth& c, const StepScalars& s, unsigned* bar, int rank, int team,
+                               SpmvShared<TX, TY>& sh, float* ws, float& bc) {
+    unsigned target = 0;
+    for (int k = 0; k < s.max_it; k++) {
+        bool stop = false;
+        for (int vb = rank; vb < c.nt && !stop; vb += team)
+            stop = spmv_phase<TX, TY, WP, STENCIL, STENCIL>(c, s, k, false, sh, vb);
+        if (stop) break;
+        target += (unsigned)team;
+        if (!grid_barrier(bar, target, c.ctl + 4)) return false;
+        for (int vb = rank; vb < c.nt && !stop; vb += team)
+            stop = axpy_phase<TX, TY>(c, s, k, false, ws, bc, vb);
+        if (stop) break;
+        target += (unsigned)team;
+        if (!grid_barrier(bar, target, c.ctl + 4)) return false;
+    }
+    return true;
+}
+
+// Region r of block b: blocks go to XCDs round-robin and each XCD takes a
+// contiguous run of regions.
+__device__ inline int region_of_block(int b, int nb) {
+    const int x = b & 7, q = nb >> 3, r = nb & 7;
+    return x * q + min(x, r) + (b >> 3);
+}
+
+// HY rows per region, one thread per vertex.  An iteration evaluates every
+// pair once: a vertex computes a = C (d_j - d_i) of the six pairs it owns
+// (those owned outside the region whose partner is inside, the strips, are
+// computed by the last threads) and leaves them in LDS, where the partner
+// takes them negated; swapping a pair's ends negates w and a exactly, and
+// both ends add in stencil order, so the sums are the SpMV's bits (as in
+// the spring-once assembly).  That halves the arithmetic and the registers
+// for blocks (36 floats) against every vertex computing its 12 pairs.
+// Component planes in LDS are whole multiples of 64 words apart, so that two
+// components move in one LDS instruction without bank conflicts.
+template <int TX, int HY>
+struct ResidentShared {
+    static constexpr int WX = TX + 2 * H, WY = HY + 2 * H, NT = TX * HY;
+    static constexpr int NS = (strip_total<TX, HY>() + 63) / 64 * 64;  // strip pairs, padded
+    static constexpr int WP = (WX * WY + 63) / 64 * 64;
+    float wd[3][WP];                // d on the region and its halo (z between two iterations)
+    float res[3][kOwned * NT + NS];  // a of the owned pairs, direction by direction, then the strips'
+    float sc[6][NS];                // the strip pairs' blocks
+    float x[3][NT];                 // the solution
+    float ws[NT / 64];
+    float bc;       // alpha or beta of the exchange just read
+    int go;         // kGo, kStop, kBreakdown or kTimeout, after the same exchange
+    int late;       // a halo vertex's z did not come
+    int team, rank;
+};
+constexpr int kGo = 0, kStop = 1, kBreakdown = 2, kTimeout = 4;
+
+template <int TX, int HY>
+__global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars s, int nb, int finish) {
+    constexpr int TY = kTileY, VT = HY / TY;            // tiles per region
+    constexpr int NT = TX * HY, NWT = TX * TY / 64;     // threads; waves per tile
+    using SH = ResidentShared<TX, HY>;
+    constexpr int WX = SH::WX;
+    constexpr int E = resident_rim(TX, HY);             // rim entries of a region
+    constexpr int NH = 2 * H * TX + 2 * H * HY + 4;     // halo vertices read by the stencil
+    constexpr int NJ = kResidentTiles / 64;             // partials per lane of wave 0
+    constexpr int S0 = NT - SH::NS;                     // first strip thread
+    static_assert(TX == 64 && HY % TY == 0, "one row per wave, whole tiles");
+    static_assert(E <= NH && NH <= NT - 64 && S0 >= 0, "rims and halo by waves 1.., strips by the last waves");
+    union Shared {
+        SH r;
+        struct {
+            SpmvShared<TX, TY> sp;
+            float ws[NWT];
+            float bc;
+        } t;
+    };
+    __shared__ Shared lds;
+    SH& sh = lds.r;
+    const int tid = threadIdx.x, lx = tid % TX, ly = tid / TX;
+    // sign in, unless the solve is already done (a second solve of one
+    // assembly); all blocks read ctl[0] before any can finish
+    int rank = 0;
+    if (tid == 0) rank = c.ctl[0] ? -1 : roll_call_sign(c.sync + 1);
+
+    const int N = c.N, nx = c.nx, ny = c.ny, ntx = c.ntx;
+    const int reg = region_of_block(blockIdx.x, nb);
+    const int rx = reg % ntx, ry = reg / ntx;
+    const int x0 = rx * TX, y0 = ry * HY;
+    const int gi = x0 + lx, gj = y0 + ly, i = gj * nx + gi;
+    const bool own = gi < nx && gj < ny;
+    const bool jac = (s.flags & OC_FLAG_JACOBI) != 0;
+    const unsigned base = c.sync[0];
+
+    // ---- this thread's vertex: mask, vectors, owned blocks
+    const uint32_t mask = own ? ldo(c.pair_mask, (uint32_t)i) : 0u;
+    float pv[kPartialRegs];
+    if (tid < 64) partial_load(c.del_part, c.nt, pv);
+    V3 r = {0.0f, 0.0f, 0.0f}, pn = r, d = r;
+    bool pinned = true;
+    if (own) {
+        r = ld3o(c.r, N, i);
+        const V3 x = ld3o(c.dv, N, i);
+        sh.x[0][tid] = x.x;
+        sh.x[1][tid] = x.y;
+        sh.x[2][tid] = x.z;
+        d = ld3o(c.d0, N, i);
+        if (jac) pn = ld3o(c.pinv, N, i);
+        pinned = ldo(c.pin, (uint32_t)i) != 0;
+    }
+    auto block_of = [&](float (&C)[6], int plane, int g, bool have) {
+        const uint32_t off = (uint32_t)g + (uint32_t)plane * 6u * (uint32_t)N;
+#pragma unroll
+        for (int q = 0; q < 6; q++) C[q] = have ? ldo(c.blocks, off + (uint32_t)(q * N)) : 0.0f;
+    };
+    float C[kOwned][6];
+#pragma unroll
+    for (int o = 0; o < kOwned; o++) block_of(C[o], c.stencil_plane[owned_k(o)], i, (mask >> owned_k(o)) & 1u);
+    // where the partner of this vertex's pairs finds the owner's a (two
+    // 16-bit places per register)
+    unsigned place[kOwned / 2] = {};
+#pragma unroll
+    for (int o = 0; o < kOwned; o++) {
+        const int wx = lx - own_dx(o), wy = ly - own_dy(o);
+        const int w = (wx >= 0 && wx < TX && wy >= 0)
+                          ? o * NT + wy * TX + wx
+                          : kOwned * NT + strip_base<TX, HY>(o) + strip_index<TX, HY>(o, wx, wy);
+        place[o / 2] |= (unsigned)w << (16 * (o & 1));
+    }
+    // this thread's strip pair: the owner's window entry and its partner's
+    int sown = 0, spar = 0;
+    bool strip = false;
+    if (tid >= S0 && tid - S0 < strip_total<TX, HY>()) {
+        int o, q, wx, wy;
+        strip_of_column<TX, HY>(tid - S0, o, q);
+        strip_owner<TX, HY>(o, q, wx, wy);
+        const int gx = x0 + wx, gy = y0 + wy, g = gy * nx + gx;
+        strip = gx >= 0 && gx < nx && gy >= 0 && gy < ny && ((ldo(c.pair_mask, (uint32_t)g) >> owned_k(o)) & 1u);
+        sown = (wy + H) * WX + wx + H;
+        spar = sown + own_dy(o) * WX + own_dx(o);
+        float SC[6];
+        block_of(SC, c.stencil_plane[owned_k(o)], g, strip);
+#pragma unroll
+        for (int e = 0; e < 6; e++) sh.sc[e][tid - S0] = SC[e];
+    }
+    // this thread's halo vertex: where its d lives in the window, and the rim
+    // entry its owner publishes z in
+    int hx = 0, hy = 0, hreg = 0, hent = 0;
+    bool halo = false;
+    if (const int e = tid - 64; e >= 0 && e < NH) {
+        if (e < 2 * TX) {  // two rows above
+            hx = e % TX, hy = e / TX - 2;
+            hreg = reg - ntx, hent = 2 * TX + e;
+        } else if (e < 4 * TX) {  // two rows below
+            hx = e % TX, hy = HY + e / TX - 2;
+            hreg = reg + ntx, hent = e - 2 * TX;
+        } else if (e < 4 * TX + 2 * HY) {  // two columns left
+            const int q = e - 4 * TX;
+            hx = q / HY - 2, hy = q % HY;
+            hreg = reg - 1, hent = 4 * TX + 2 * HY + q;
+        } else if (e < 4 * TX + 4 * HY) {  // two columns right
+            const int q = e - 4 * TX - 2 * HY;
+            hx = TX + q / HY, hy = q % HY;
+            hreg = reg + 1, hent = 4 * TX + q;
+        } else {  // the four corners next to the region
+            const int q = e - 4 * TX - 4 * HY;
+            hx = (q & 1) ? TX : -1, hy = (q & 2) ? HY : -1;
+            hreg = reg + ((q & 1) ? 1 : -1) + ((q & 2) ? ntx : -ntx);
+            hent = ((q & 2) ? 0 : 3 * TX) + ((q & 1) ? 0 : TX - 1);
+        }
+        const int gx = x0 + hx, gy = y0 + hy;
+        halo = gx >= 0 && gx < nx && gy >= 0 && gy < ny;
+    }
+    const int hw = (hy + H) * WX + hx + H;
+    V3 hd = {0.0f, 0.0f, 0.0f}, hz = hd;
+    if (halo) hd = ld3o(c.d0, N, (y0 + hy) * nx + x0 + hx);
+    // this thread's rim entry: the window cell whose z it publishes
+    int rw = 0;
+    if (const int e = tid - 64; e >= 0 && e < E) {
+        const int q = e - 4 * TX, qx = q / HY;
+        rw = e < 4 * TX ? ((e < 2 * TX ? e / TX : HY - 4 + e / TX) + H) * WX + e % TX + H
+                        : (q % HY + H) * WX + (qx < H ? qx : TX - 2 * H + qx) + H;
+    }
+    uint64_t* const rim = c.xch + resident_part_words(c.xstride);
+    const unsigned hsrc = (unsigned)(hreg * 3 * E + hent), rout = (unsigned)(reg * 3 * E);
+    // this XCD's copy of the tiles' partials
+    unsigned xcc;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+    const uint64_t* const near = c.xch + (size_t)(xcc & 7u) * c.xstride;
+
+    // Sum of the tiles' partials of exchange n (wave 0): polled until every
+    // tag is the exchange's, then added as partial_finish does.
+    auto poll_sum = [&](unsigned n, float& sum) -> bool {
+        const uint64_t* p = near + (n & 1u) * c.xslots;
+        const unsigned tag = base + n + 1u;
+        uint64_t w[NJ];
+        for (int spin = 0;; spin++) {
+            bool ok = true;
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                w[j] = tid + 64 * j < c.nt ? xch_load(p, (unsigned)(tid + 64 * j)) : (uint64_t)tag << 32;
+#pragma unroll
+            for (int j = 0; j < NJ; j++) ok = ok && (unsigned)(w[j] >> 32) == tag;
+            if (__all(ok)) break;
+            if (spin > kPollLimit) return false;
+        }
+        float t = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) t += __uint_as_float((unsigned)w[j]);
+        sum = wave_sum(t);
+        return true;
+    };
+    // The tiles' sums of t (tile_sum's order), published as exchange n.
+    auto publish = [&](unsigned n, float t) {
+        const float w = wave_sum(t);
+        if ((tid & 63) == 0) sh.ws[tid >> 6] = w;
+        __syncthreads();
+        if (tid < 8 * VT && ry * VT + (tid >> 3) < c.nty) {  // 8 copies of each tile's partial
+            const float* const q = sh.ws + (tid >> 3) * NWT;
+            float p = q[0];
+#pragma unroll
+            for (int k = 1; k < NWT; k++) p = p + q[k];
+            xch_store(c.xch, (tid & 7) * c.xstride + (n & 1u) * c.xslots + (ry * VT + (tid >> 3)) * ntx + rx, base + n + 1u,
+                      p);
+        }
+    };
+    // ---- d0 on the region and its halo; r.z of the start
+    const int cw = (ly + H) * WX + lx + H;
+    auto put = [&](int w, V3 v) {
+        sh.wd[0][w] = v.x;
+        sh.wd[1][w] = v.y;
+        sh.wd[2][w] = v.z;
+    };
+    auto get = [&](int w) { return V3{sh.wd[0][w], sh.wd[1][w], sh.wd[2][w]}; };
+    put(cw, d);
+    if (halo) put(hw, hd);
+    // r.z of the iteration at hand and of the one before, the stopping test's
+    // threshold: kept by thread 0, which decides for the block (every block's
+    // thread 0 decides alike) and hands on alpha and beta
+    float delta = 0.0f, delta_old = 0.0f, delta0 = 0.0f, thresh = 0.0f;
+    auto stopped = [&]() { return s.tol_mode != 2 && !(delta > thresh); };
+    if (tid < 64) {
+        delta = delta0 = partial_finish(c.del_part, c.nt, pv);
+        thresh = s.tol_mode == 1 ? s.tol2 * delta0 : s.tol2;
+    }
+    if (tid == 0) {
+        sh.go = stopped() ? kStop : kGo;
+        sh.late = 0;
+        sh.rank = rank;
+        sh.team = rank < 0 ? 0 : roll_call_wait(c.sync + 1, nb);
+    }
+    __syncthreads();
+    const int team = sh.team;
+    rank = sh.rank;
+    if (rank < 0) return;
+    if (team < nb) {
+        __syncthreads();  // (the shared words above have been read)
+        if (tid >= TX * TY) return;
+        if (!cg_team<TX, TY, kStencil, true>(c, s, c.sync + 2, rank, team, lds.t.sp, lds.t.ws, lds.t.bc)) return;
+        __syncthreads();
+        if (finish && rank == 0) cg_finish_block(c, s, &lds.t.bc);
+        return;
+    }
+
+    // ---- iterations
+    const bool full = __all(mask == 0xFFFu);  // every lane of the wave has all 12 neighbours
+    int it = s.max_it, go = sh.go;
+    float beta = 0.0f;
+    for (int k = 0; k < s.max_it; k++) {
+        if (go != kGo) {
+            it = k;
+            break;
+        }
+        if (k > 0) {  // d = z + beta d
+            const V3 z = jac ? V3{pn.x * r.x, pn.y * r.y, pn.z * r.z} : r;
+            d = {z.x + beta * d.x, z.y + beta * d.y, z.z + beta * d.z};
+            put(cw, d);
+            if (halo) {
+                hd = {hz.x + beta * hd.x, hz.y + beta * hd.y, hz.z + beta * hd.z};
+                put(hw, hd);
+            }
+            __syncthreads();
+        }
+        // q = S A d: the owned pairs, then every vertex's sum.  Pairs that do
+        // not exist have a zero block; what they give is not added.
+        V3 a[kOwned];
+#pragma unroll
+        for (int o = 0; o < kOwned; o++) a[o] = get(cw + own_dy(o) * WX + own_dx(o));
+#pragma unroll
+        for (int o = 0; o < kOwned; o++) {
+            a[o] = symmv(C[o], V3{a[o].x - d.x, a[o].y - d.y, a[o].z - d.z});
+            sh.res[0][o * NT + tid] = a[o].x;
+            sh.res[1][o * NT + tid] = a[o].y;
+            sh.res[2][o * NT + tid] = a[o].z;
+        }
+        if (strip) {
+            const int t = tid - S0;
+            const V3 e = get(sown), f = get(spar);
+            float SC[6];
+#pragma unroll
+            for (int q = 0; q < 6; q++) SC[q] = sh.sc[q][t];
+            const V3 b = symmv(SC, V3{f.x - e.x, f.y - e.y, f.z - e.z});
+            sh.res[0][kOwned * NT + t] = b.x;
+            sh.res[1][kOwned * NT + t] = b.y;
+            sh.res[2][kOwned * NT + t] = b.z;
+        }
+        __syncthreads();
+        V3 acc = {s.md * d.x, s.md * d.y, s.md * d.z};
+        V3 p[kOwned];
+#pragma unroll
+        for (int o = 0; o < kOwned; o++) {
+            const unsigned w = (here(place[o / 2]) >> (16 * (o & 1))) & 0xFFFFu;
+            p[o] = {sh.res[0][w], sh.res[1][w], sh.res[2][w]};
+        }
+        auto add = [&](int kk) {
+            const int o = owned_index(kk);
+            return stencil_owner(kk) ? V3{acc.x + a[o].x, acc.y + a[o].y, acc.z + a[o].z}
+                                     : V3{acc.x - p[o].x, acc.y - p[o].y, acc.z - p[o].z};
+        };
+        if (full) {
+#pragma unroll
+            for (int kk = 0; kk < kStencil; kk++) acc = add(kk);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < kStencil; kk++) {
+                const V3 n = add(kk);
+                const bool have = (mask >> kk) & 1u;
+                acc = {have ? n.x : acc.x, have ? n.y : acc.y, have ? n.z : acc.z};
+            }
+        }
+        const V3 q = pinned ? V3{0.0f, 0.0f, 0.0f} : acc;
+        publish(2u * k, own ? dot3(d, q) : 0.0f);
+        if (tid < 64) {
+            float sigma = 0.0f;
+            const bool got = poll_sum(2u * k, sigma);
+            // sigma == 0 only after r (hence d) underflowed: no update, no 0/0
+            const float alpha = sigma == 0.0f ? 0.0f : delta / sigma;
+            if (tid == 0) {
+                sh.bc = alpha;
+                sh.go = !got ? kTimeout : sigma < 0.0f || !isfinite(sigma) ? kBreakdown : kGo;
+            }
+        }
+        __syncthreads();
+        const float alpha = sh.bc;
+        go = sh.go;
+        if (go != kGo) {
+            it = k;
+            break;
+        }
+        const bool last = k + 1 == s.max_it;
+        r = {r.x - alpha * q.x, r.y - alpha * q.y, r.z - alpha * q.z};
+        const V3 z = jac ? V3{pn.x * r.x, pn.y * r.y, pn.z * r.z} : r;
+        put(cw, z);
+        publish(2u * k + 1u, own ? dot3(r, z) : 0.0f);
+        const unsigned tag = base + 2u * k + 2u;
+        if (!last && tid >= 64 && tid < 64 + E) {
+            const V3 v = get(rw);
+            const unsigned e = rout + tid - 64;
+            xch_store(rim, e, tag, v.x);
+            xch_store(rim, e + E, tag, v.y);
+            xch_store(rim, e + 2 * E, tag, v.z);
+        }
+        sh.x[0][tid] = sh.x[0][tid] + alpha * d.x;
+        sh.x[1][tid] = sh.x[1][tid] + alpha * d.y;
+        sh.x[2][tid] = sh.x[2][tid] + alpha * d.z;
+        if (last && blockIdx.x != 0) break;  // nothing more is read: block 0 records the status
+        if (tid < 64) {
+            float sum = 0.0f;
+            const bool got = poll_sum(2u * k + 1u, sum);
+            delta_old = delta;
+            delta = sum;
+            // beta = 0 once r.r has underflowed to 0 (fixed iteration counts)
+            const float b = delta_old != 0.0f ? delta / delta_old : 0.0f;
+            if (tid == 0) {
+                sh.bc = b;
+                sh.go = !got ? kTimeout : stopped() ? kStop : kGo;
+            }
+        } else if (halo && !last) {
+            uint64_t w[3];
+            for (int spin = 0;; spin++) {
+#pragma unroll
+                for (int e = 0; e < 3; e++) w[e] = xch_load(rim, hsrc + e * E);
+                if ((unsigned)(w[0] >> 32) == tag && (unsigned)(w[1] >> 32) == tag && (unsigned)(w[2] >> 32) == tag)
+                    break;
+                if (spin > kPollLimit) {
+                    sh.late = 1;
+                    break;
+                }
+            }
+            hz = {__uint_as_float((unsigned)w[0]), __uint_as_float((unsigned)w[1]), __uint_as_float((unsigned)w[2])};
+        }
+        // (a stop after the last iteration leaves it = max_it)
+        __syncthreads();
+        beta = sh.bc;
+        go = sh.late ? kTimeout : last ? sh.go & kTimeout : sh.go;
+    }
+
+    if (blockIdx.x == 0 && tid == 0) c.sync[3] = base + 2u * (unsigned)s.max_it;  // the next solve's base
+    if (go == kTimeout) {  // an exchange timed out: report it, leave dv as it was
+        if (tid == 0) {
+            __hip_atomic_fetch_or(c.ctl + 4, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (blockIdx.x == 0) c.ctl[0] = 1;
+        }
+        return;
+    }
+    if (own) st3o(c.dv, N, i, V3{sh.x[0][tid], sh.x[1][tid], sh.x[2][tid]});
+    if (blockIdx.x == 0 && tid == 0) {
+        // as a stopped solve of the per-iteration launches leaves them; the
+        // status bits follow as cg_finish_block derives them
+        c.scal[0] = delta0;
+        c.scal[it] = delta;
+        c.ctl[0] = 1;
+        c.ctl[1] = it;
+        int st = c.ctl[2] | (go == kBreakdown ? OC_SOLVE_BREAKDOWN : 0);
+        if (finish) {
+            if (s.tol_mode != 2 && delta > thresh && !(st & OC_SOLVE_BREAKDOWN)) st |= OC_SOLVE_NOT_CONVERGED;
+            if (!isfinite(delta)) st |= OC_SOLVE_NONFINITE;
+            atomicOr(c.ctl + 3, st);
+        }
+        c.ctl[2] = st;
+    }
+}
+
+// All CG iterations of any topology in one cooperative launch (each resident
+// block serves tiles blockIdx.x, + gridDim.x, ...).
 template <int TX, int TY, int WP>
 __global__ __launch_bounds__(TX* TY) void k_cg_persistent(DevCloth c, StepScalars s, unsigned* bar) {
     __shared__ SpmvShared<TX, TY> sh;
     __shared__ float ws[TX * TY / 64];
     __shared__ float bc;
-    const unsigned nb = gridDim.x;
-    unsigned target = 0;
-    for (int k = 0; k < s.max_it; k++) {
-        bool stop = false;
-        for (int vb = blockIdx.x; vb < c.nt && !stop; vb += gridDim.x)
-            stop = spmv_phase<TX, TY, WP>(c, s, k, false, sh, vb);
-        if (stop) break;
-        target += nb;
-        if (!grid_barrier(bar, target, c.ctl + 4)) break;
-        for (int vb = blockIdx.x; vb < c.nt && !stop; vb += gridDim.x)
-            stop = axpy_phase<TX, TY>(c, s, k, false, ws, bc, vb);
-        if (stop) break;
-        target += nb;
-        if (!grid_barrier(bar, target, c.ctl + 4)) break;
-    }
+    (void)cg_team<TX, TY, WP, false>(c, s, bar, blockIdx.x, gridDim.x, sh, ws, bc);
 }
 
 __global__ void k_reset_barrier(unsigned* bar) {
@@ -1379,8 +1881,30 @@ int persistent_cg_grid(const DevCloth& c) {
     return std::min(grid, c.nt);
 }
 
+int resident_cg_tiles(const DevCloth& c) {
+    int dev = 0, cus = 0;
+    if (!c.stencil || c.nt > kResidentTiles || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    if (c.nt <= cus) return 1;
+    return c.ntx * ((c.nty + 1) / 2) <= cus ? 2 : 0;
+}
+
+hipError_t launch_cg_resident(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish, int blocks) {
+    const dim3 grid(blocks), block(kTileX * kTileY * c.res_vt);
+    const int nb = resident_blocks(c.ntx, c.nty, c.res_vt);
+    if (blocks < 1 || blocks > nb || s.max_it < 1) return hipErrorInvalidValue;
+    if (c.res_vt == 1)
+        return launch_k(1, k_cg_resident<kTileX, kTileY>, grid, block, st, c, s, nb, finish ? 1 : 0);
+    if (c.res_vt == 2)
+        return launch_k(1, k_cg_resident<kTileX, 2 * kTileY>, grid, block, st, c, s, nb, finish ? 1 : 0);
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_cg(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish) {
     hipError_t e;
+    if (c.res_vt && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION))
+        return launch_cg_resident(c, s, st, finish, resident_blocks(c.ntx, c.nty, c.res_vt));
     if (c.persistent && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION)) {
         if (c.persistent > c.nt) return hipErrorInvalidValue;  // a block without a tile
         unsigned* bar = reinterpret_cast<unsigned*>(c.ctl + 6);

@@ -119,10 +119,23 @@ __device__ inline V3 spring_force(V3 x1, V3 x2, V3 v1, V3 v2, float L0, float Ks
     return {s * (dp.x * inv), s * (dp.y * inv), s * (dp.z * inv)};
 }
 
-// Wave tree: lane l += lane l+off for off = 32..1; lane 0 ends with the sum.
+// Wave tree: lane l += lane l+off for off = 32..1; lane 0 ends with the sum
+// (the other lanes' values are not the tree's).  Offsets 32 and 16 by gfx950's
+// lane-swap instructions, the rest by row shifts inside 16 lanes: register
+// moves of a few cycles, where each __shfl_down is an LDS round trip.
+template <int N>
+__device__ inline float row_down(float t) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(t), 0x100 + N, 0xF, 0xF, true));
+}
 __device__ inline float wave_sum(float t) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) t += __shfl_down(t, off, 64);
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+    t += __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+    t += __uint_as_float(b[1]);
+    t += row_down<8>(t);
+    t += row_down<4>(t);
+    t += row_down<2>(t);
+    t += row_down<1>(t);
     return t;
 }
 

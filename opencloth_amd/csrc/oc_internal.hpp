@@ -220,13 +220,47 @@ struct DevCloth {
     float* s1;
     float* s2;
     int cg1_alpha;
+    // resident solve: tiles per block (0: not used), the exchange words
+    // (resident_words of them) with xslots slots per set of partials and
+    // xstride words from one copy of the partials to the next, and its
+    // control words: [0] epoch base of the tags, [1] roll call, [2] barrier
+    // counter of a partial team, [3] the next solve's epoch base
+    int res_vt;
+    int xslots, xstride;
+    uint64_t* xch;
+    unsigned* sync;
 };
+
+// Resident solve (k_cg_resident): one block per region of kTileX x (kTileY
+// tiles) vertices, one block per CU.  Registers hold a thread's pair blocks
+// (72 floats per vertex), so a CU takes two tiles and 256 CUs take 512.
+constexpr int kResidentTiles = 512;
+__host__ __device__ constexpr int resident_rim(int tx, int hy) { return 2 * kHalo * tx + 2 * kHalo * hy; }
+__host__ __device__ constexpr int resident_blocks(int ntx, int nty, int tiles) {
+    return ntx * ((nty + tiles - 1) / tiles);
+}
+// Slots per set of partials (one per tile, in whole 512-byte lines), words
+// between the partials' copies, words of all 8 copies, and words with the
+// rims.  The copies of many tiles are 64 KB apart: an exchange among 256
+// blocks waited 4519 cycles so, 4739 at 32 KB, 5084 at 16 KB and 5575 at 8 KB
+// (back to back); a few tiles' copies may lie closer.
+__host__ __device__ constexpr int resident_slots(int ntx, int nty) { return (ntx * nty + 63) / 64 * 64; }
+__host__ __device__ constexpr int resident_stride(int ntx, int nty) { return ntx * nty > 64 ? 8192 : 512; }
+__host__ __device__ constexpr size_t resident_part_words(int xstride) { return (size_t)8 * xstride; }
+constexpr size_t resident_words(int ntx, int nty, int tiles, int tx, int ty) {
+    return resident_part_words(resident_stride(ntx, nty)) +
+           (size_t)resident_blocks(ntx, nty, tiles) * 3 * resident_rim(tx, ty * tiles);
+}
+// Tiles per block of the resident solve for this cloth on the current
+// device, 0 where it does not fit (or the pairs have no stencil form).
+int resident_cg_tiles(const DevCloth& c);
 
 // Implicit steps of a cloth handle, the body of oc_cloth_step (capi.cpp).
 // partials: NULL for the handle's own CG partials and scalars, else a device
 // buffer of cloth_partial_floats(c) floats used in their place.
 size_t cloth_partial_floats(const ::oc_cloth_s* c);
 int cloth_device(const ::oc_cloth_s* c);  // the device the handle was created on
+const DevCloth& cloth_view(const ::oc_cloth_s* c);
 int cloth_step(::oc_cloth_s* c, int nsteps, float* partials);
 
 // Blocks of the persistent CG launch (all resident at once), 0 if unsupported.
@@ -244,8 +278,8 @@ struct StepScalars {
 // implicit.hip starts its kernel with hipExtLaunchKernelGGL and the next
 // start/stop event pair of the profile, so every kernel's own duration is
 // recorded inside the real launch sequence, with no event packets between
-// the launches.  kind: 0 assembly, 1 CG iteration (part 1), 2 CG part 2,
-// 3 other solver launches, 4 update.
+// the launches.  kind: 0 assembly, 1 CG iteration (part 1) or a whole solve,
+// 2 CG part 2, 3 other solver launches, 4 update.
 struct LaunchProfile {
     hipEvent_t* start;
     hipEvent_t* stop;
@@ -269,6 +303,9 @@ hipError_t launch_scatter_cst(const DevCloth& c, const int32_t* spring_cst, int 
 // finish = false leaves the iteration count and status to launch_update(...,
 // finish = true), the step's last launch.
 hipError_t launch_cg(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish = true);
+// The resident solve with `blocks` blocks: all of resident_blocks(), or fewer
+// to run the partial team's code.
+hipError_t launch_cg_resident(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish, int blocks);
 hipError_t launch_cg_spmv(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_axpy(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_finish(const DevCloth& c, const StepScalars& s, hipStream_t st);
