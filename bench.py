@@ -148,12 +148,13 @@ def bench_entries(steps: int = 100) -> dict:
     nd_col, nb_col = pc.num_colors()
     ms = timed(lambda k: pc.step(k), steps)
     ns = sc.params.solver_iterations
-    b = ns * (72 * len(sc.distance) + 108 * len(sc.bending)) + 132 * N
+    # x, v, w in and x, v out once, a record per constraint and solver iteration
+    b = ns * 12 * (len(sc.distance) + len(sc.bending)) + 52 * N
     out["pbd"] = {"workload": f"{n}x{n} PBD step, {len(sc.distance)} distance and {len(sc.bending)} "
                               f"bending constraints, {ns} solver iterations",
                   "ms_per_step": ms, "vertex_steps_per_s": N / (ms * 1e-3),
                   "colours": [nd_col, nb_col],
-                  "launches_per_step": 5 + ns * (nd_col + nb_col + int(sc.params.ground)) + 1,
+                  "launches_per_step": 2 + ns,
                   "algorithmic_bytes": b, "roofline_frac": b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
     pc.close()
 

@@ -2,8 +2,11 @@
 // (OpenCloth_PositionBasedDynamics/.../main.cpp) over caller-given distance
 // and bending constraint lists.  Constraints are coloured on the host
 // (greedy, in list order: a constraint takes the lowest colour not yet used
-// at any of its particles) and stored colour by colour; one launch projects
-// one colour.  With OC_FLAG_LIST_ORDER they are stored level by level
+// at any of its particles) and laid out for the tiled solver (pbd_plan.cpp):
+// one launch per step for a cloth of up to kPbdSmall particles, one per
+// solver iteration and two for the sums beyond; constraints that reach too
+// far for it are stored colour by colour and one launch projects one colour.
+// With OC_FLAG_LIST_ORDER they are stored level by level
 // instead (a constraint's level is one more than the highest level among the
 // earlier constraints sharing a particle with it) and one single-workgroup
 // launch projects all levels of a step in order: the reference's sequential
@@ -13,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstring>
 #include <new>
 #include <string>
 #include <vector>
@@ -53,12 +57,10 @@ void bucket(int n, int arity, const std::vector<int32_t>& p, const std::vector<i
         });
 }
 
-// Greedy colouring in list order (see bucket for the order inside a colour).
-// Returns the colour count, -1 past 64.
-int colour(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<int32_t>& order,
-           std::vector<int32_t>& ptr) {
+// Greedy colouring in list order.  Returns the colour count, -1 past 64.
+int colour(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<int>& col) {
     std::vector<uint64_t> used((size_t)N, 0);
-    std::vector<int> col((size_t)n);
+    col.assign((size_t)n, 0);
     int ncol = 0;
     for (int c = 0; c < n; c++) {
         uint64_t m = 0;
@@ -69,7 +71,6 @@ int colour(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<i
         for (int a = 0; a < arity; a++) used[p[(size_t)arity * c + a]] |= uint64_t(1) << k;
         ncol = std::max(ncol, k + 1);
     }
-    bucket(n, arity, p, col, ncol, order, ptr);
     return ncol;
 }
 
@@ -96,12 +97,13 @@ int levels(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<i
 }  // namespace
 
 struct oc_pbd_s {
-    int N = 0, nd = 0, nb = 0;
+    int N = 0;
     oc_pbd_params prm{};
     hipStream_t stream = nullptr;
     void* arena = nullptr;
     oc::DevPbd dev{};
-    std::vector<int32_t> d_ptr, b_ptr;  // colour offsets
+    std::vector<int32_t> d_ptr, b_ptr;  // colour (or level) offsets, not with the tiled solver
+    int n_dcol = 0, n_bcol = 0;         // colours (or levels)
 };
 
 namespace {
@@ -119,6 +121,11 @@ oc::PbdScalars pscalars(const oc_pbd_s* p) {
     s.global_k = s.gd * 0.01f;  // PBD:712
     s.inv_dt = 1.0f / p->prm.dt;
     s.flags = p->prm.flags;
+    s.w = 1.0f / p->prm.mass;
+    const float wsum = s.w + s.w + 2.0f * s.w;
+    s.inv_2w = 1.0f / (s.w + s.w);
+    s.bend_2w = (2.0f * s.w) / wsum;
+    s.bend_4w = (4.0f * s.w) / wsum;
     return s;
 }
 
@@ -206,117 +213,161 @@ int oc_pbd_create(int32_t n_vertices, const float* x0, const uint8_t* pinned,
     if (!p) return set_error(OC_ERR_OUT_OF_MEMORY, "host allocation failed");
     std::vector<int32_t> d_order, b_order;
     const bool list_order = (params->flags & OC_FLAG_LIST_ORDER) != 0;
+    oc::PbdPlan plan;
     if (list_order) {
-        levels(N, n_distance, 2, dp, d_order, p->d_ptr);
-        levels(N, n_bending, 3, bp, b_order, p->b_ptr);
-    } else if (colour(N, n_distance, 2, dp, d_order, p->d_ptr) < 0 ||
-               colour(N, n_bending, 3, bp, b_order, p->b_ptr) < 0) {
-        delete p;
-        return set_error(OC_ERR_UNSUPPORTED_TOPOLOGY, "constraints need more than 64 colours");
+        p->n_dcol = levels(N, n_distance, 2, dp, d_order, p->d_ptr);
+        p->n_bcol = levels(N, n_bending, 3, bp, b_order, p->b_ptr);
+    } else {
+        std::vector<int> dcol, bcol;
+        p->n_dcol = colour(N, n_distance, 2, dp, dcol);
+        p->n_bcol = colour(N, n_bending, 3, bp, bcol);
+        if (p->n_dcol < 0 || p->n_bcol < 0) {
+            delete p;
+            return set_error(OC_ERR_UNSUPPORTED_TOPOLOGY, "constraints need more than 64 colours");
+        }
+        // the tiled solver where its closures stay small: at most 4 times
+        // the constraints (they are 1.7 times on a 512x512 grid of the
+        // reference's lists, where a solver iteration takes 10 us against 77
+        // us for a launch per colour)
+        int dev = 0, lds = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+            lds = 0;
+        const int local = std::min(oc::kPbdLocal, (lds - 4096) / 16);
+        const oc::PbdFamily df{n_distance, 2, p->n_dcol, dp.data(), dcol.data()};
+        const oc::PbdFamily bf{n_bending, 3, p->n_bcol, bp.data(), bcol.data()};
+        const bool small = N <= oc::kPbdSmall;
+        if (!oc::build_pbd_plan(N, x0, df, bf, small ? oc::kPbdSmall : oc::kPbdOwned, local, 4.0f, &plan)) {
+            bucket(n_distance, 2, dp, dcol, p->n_dcol, d_order, p->d_ptr);
+            bucket(n_bending, 3, bp, bcol, p->n_bcol, b_order, p->b_ptr);
+        }
     }
-    const size_t nd = n_distance, nb = n_bending;
-    std::vector<int32_t> d1(nd), d2(nd), b1(nb), b2(nb), b3(nb);
-    std::vector<float> drest(nd), dkp(nd), brest(nb), bw(nb), bkp(nb);
-    for (size_t j = 0; j < nd; j++) {
-        const int c = d_order[j];
-        const int a = dp[2 * c], b = dp[2 * c + 1];
-        d1[j] = a;
-        d2[j] = b;
+    // rest lengths and k' of every constraint, in list order (PBD:148-178)
+    std::vector<float> drest_of((size_t)n_distance), dkp_of((size_t)n_distance), brest_of((size_t)n_bending),
+        bkp_of((size_t)n_bending);
+    bool d_same = true, b_same = true;  // one k' for the whole family
+    auto k_of = [&](float k, size_t c, std::vector<float>& kp, float before, bool& same) {
+        kp[c] = c > 0 && k == before ? kp[c - 1] : k_prime(clamp01(k), ns);
+        same = same && (c == 0 || std::memcmp(&kp[c], &kp[0], sizeof(float)) == 0);
+    };
+    for (int c = 0; c < n_distance; c++) {
+        const int a = dp[2 * (size_t)c], b = dp[2 * (size_t)c + 1];
         const float dx = x0[3 * a] - x0[3 * b], dy = x0[3 * a + 1] - x0[3 * b + 1],
                     dz = x0[3 * a + 2] - x0[3 * b + 2];
-        drest[j] = sqrtf(dx * dx + dy * dy + dz * dz);
-        dkp[j] = k_prime(clamp01(distance[c].k), ns);
+        drest_of[c] = sqrtf(dx * dx + dy * dy + dz * dz);
+        k_of(distance[c].k, c, dkp_of, c ? distance[c - 1].k : 0.0f, d_same);
     }
-    for (size_t j = 0; j < nb; j++) {
-        const int c = b_order[j];
-        const int a = bp[3 * c], b = bp[3 * c + 1], d = bp[3 * c + 2];
-        b1[j] = a;
-        b2[j] = b;
-        b3[j] = d;
-        bw[j] = W[a] + W[b] + 2.0f * W[d];
+    for (int c = 0; c < n_bending; c++) {
+        const int a = bp[3 * (size_t)c], b = bp[3 * (size_t)c + 1], d = bp[3 * (size_t)c + 2];
         float dc[3];
         for (int k = 0; k < 3; k++) {
             const float ctr = 0.3333f * ((x0[3 * a + k] + x0[3 * b + k]) + x0[3 * d + k]);
             dc[k] = x0[3 * d + k] - ctr;
         }
-        brest[j] = sqrtf(dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
-        bkp[j] = k_prime(clamp01(bending[c].k), ns);
+        brest_of[c] = sqrtf(dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
+        k_of(bending[c].k, c, bkp_of, c ? bending[c - 1].k : 0.0f, b_same);
     }
 
     p->N = N;
-    p->nd = n_distance;
-    p->nb = n_bending;
     p->prm = *params;
     const int nblk = (N + oc::kPbdBlock - 1) / oc::kPbdBlock;
-    const size_t vec = align_up(sizeof(float) * 3 * N);
-    const size_t sN = align_up(sizeof(float) * N);
-    const size_t sd = align_up(4 * std::max<size_t>(nd, 1)), sb = align_up(4 * std::max<size_t>(nb, 1));
-    const size_t spart = align_up(sizeof(float) * oc::kPbdSums * nblk);
-    const size_t ssum = align_up(sizeof(float) * oc::kPbdSums);
-    const size_t sdl = align_up(4 * p->d_ptr.size()), sbl = align_up(4 * p->b_ptr.size());
-    const size_t total = 3 * vec + sN + 4 * sd + 6 * sb + spart + ssum + sdl + sbl;
+    oc::DevPbd& d = p->dev;
+    d.N = N;
+    d.nblk = nblk;
+    // device arrays: where each goes, its bytes and its contents (none: zeros)
+    struct Array {
+        const void** dst;
+        size_t bytes;
+        const void* src;
+    };
+    std::vector<Array> arrays;
+    auto add = [&](auto*& dst, size_t bytes, const void* src) {
+        arrays.push_back({(const void**)(const void*)&dst, std::max<size_t>(bytes, 4), bytes ? src : nullptr});
+    };
+    const size_t vec = sizeof(float) * 3 * (size_t)N;
+    add(d.x, vec, nullptr);
+    add(d.v, vec, nullptr);
+    add(d.t, vec, nullptr);
+    add(d.w, sizeof(float) * (size_t)N, W.data());
+    add(d.part, sizeof(float) * oc::kPbdSums * (size_t)nblk, nullptr);
+    add(d.sums, sizeof(float) * oc::kPbdSums, nullptr);
+    // the constraints in the order they are stored: the plan's records (a
+    // constraint once for every block that projects it), or colour by colour
+    std::vector<int32_t> d1, d2, b1, b2, b3;
+    std::vector<float> drest, dkp, brest, bw, bkp, kp;
+    auto bytes_of = [](const auto& v) { return v.size() * sizeof(v[0]); };
+    if (plan.nb > 0) {
+        d.nb = plan.nb;
+        d.nd_col = p->n_dcol;
+        d.nb_col = p->n_bcol;
+        d.max_local = plan.max_local;
+        const int ncol = p->n_dcol + p->n_bcol;
+        const bool uniform = d_same && b_same;
+        if (!uniform) kp.resize(plan.rec.size());
+        for (int b = 0; b < plan.nb; b++)
+            for (int c = 0; c < ncol; c++) {
+                const int32_t* at = plan.cptr.data() + (size_t)b * (ncol + 1) + c;
+                for (int32_t j = at[0]; j < at[1]; j++) {
+                    const int32_t e = plan.id[j];
+                    plan.rec[j].rest = c < p->n_dcol ? drest_of[e] : brest_of[e];
+                    if (!uniform) kp[j] = c < p->n_dcol ? dkp_of[e] : bkp_of[e];
+                }
+            }
+        if (plan.rec.empty()) plan.rec.push_back({0u, 0.0f, 0u});  // (what an idle thread loads)
+        d.n_rec = (int)plan.rec.size();
+        add(d.t_off, bytes_of(plan.off), plan.off.data());
+        add(d.t_own, bytes_of(plan.own), plan.own.data());
+        add(d.t_ids, bytes_of(plan.ids), plan.ids.data());
+        add(d.t_cptr, bytes_of(plan.cptr), plan.cptr.data());
+        add(d.t_rec, bytes_of(plan.rec), plan.rec.data());
+        if (!uniform) add(d.t_kp, bytes_of(kp), kp.data());
+        d.d_kp_all = n_distance > 0 ? dkp_of[0] : 0.0f;
+        d.b_kp_all = n_bending > 0 ? bkp_of[0] : 0.0f;
+        if (plan.nb > 1) add(d.t2, vec, nullptr);
+    } else {
+        for (int32_t c : d_order) {
+            drest.push_back(drest_of[c]);
+            dkp.push_back(dkp_of[c]);
+            d1.push_back(dp[2 * (size_t)c]);
+            d2.push_back(dp[2 * (size_t)c + 1]);
+        }
+        for (int32_t c : b_order) {
+            brest.push_back(brest_of[c]);
+            bkp.push_back(bkp_of[c]);
+            const int a = bp[3 * (size_t)c], b = bp[3 * (size_t)c + 1], e = bp[3 * (size_t)c + 2];
+            b1.push_back(a);
+            b2.push_back(b);
+            b3.push_back(e);
+            bw.push_back(W[a] + W[b] + 2.0f * W[e]);
+        }
+        add(d.d_p1, bytes_of(d1), d1.data());
+        add(d.d_p2, bytes_of(d2), d2.data());
+        add(d.d_rest, bytes_of(drest), drest.data());
+        add(d.d_kp, bytes_of(dkp), dkp.data());
+        add(d.b_p1, bytes_of(b1), b1.data());
+        add(d.b_p2, bytes_of(b2), b2.data());
+        add(d.b_p3, bytes_of(b3), b3.data());
+        add(d.b_rest, bytes_of(brest), brest.data());
+        add(d.b_w, bytes_of(bw), bw.data());
+        add(d.b_kp, bytes_of(bkp), bkp.data());
+        add(d.d_lv, bytes_of(p->d_ptr), p->d_ptr.data());
+        add(d.b_lv, bytes_of(p->b_ptr), p->b_ptr.data());
+        d.nd_lv = (int)p->d_ptr.size() - 1;
+        d.nb_lv = (int)p->b_ptr.size() - 1;
+    }
+    size_t total = 0;
+    for (const Array& a : arrays) total += align_up(a.bytes);
     if (hipMalloc(&p->arena, total) != hipSuccess) {
         delete p;
         return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc failed");
     }
+    bool ok = hipMemset(p->arena, 0, total) == hipSuccess;
     char* q = (char*)p->arena;
-    auto take = [&](size_t bytes) {
-        char* r = q;
-        q += bytes;
-        return r;
-    };
-    oc::DevPbd& d = p->dev;
-    d.N = N;
-    d.nblk = nblk;
-    d.x = (float*)take(vec);
-    d.v = (float*)take(vec);
-    d.t = (float*)take(vec);
-    float* w = (float*)take(sN);
-    int32_t* dd1 = (int32_t*)take(sd);
-    int32_t* dd2 = (int32_t*)take(sd);
-    float* ddr = (float*)take(sd);
-    float* ddk = (float*)take(sd);
-    int32_t* bb1 = (int32_t*)take(sb);
-    int32_t* bb2 = (int32_t*)take(sb);
-    int32_t* bb3 = (int32_t*)take(sb);
-    float* bbr = (float*)take(sb);
-    float* bbw = (float*)take(sb);
-    float* bbk = (float*)take(sb);
-    d.part = (float*)take(spart);
-    d.sums = (float*)take(ssum);
-    int32_t* dlv = (int32_t*)take(sdl);
-    int32_t* blv = (int32_t*)take(sbl);
-    d.d_lv = dlv;
-    d.b_lv = blv;
-    d.nd_lv = (int)p->d_ptr.size() - 1;
-    d.nb_lv = (int)p->b_ptr.size() - 1;
-    d.w = w;
-    d.d_p1 = dd1;
-    d.d_p2 = dd2;
-    d.d_rest = ddr;
-    d.d_kp = ddk;
-    d.b_p1 = bb1;
-    d.b_p2 = bb2;
-    d.b_p3 = bb3;
-    d.b_rest = bbr;
-    d.b_w = bbw;
-    d.b_kp = bbk;
-    bool ok = hipMemset(p->arena, 0, total) == hipSuccess &&
-              hipMemcpy(w, W.data(), 4 * (size_t)N, hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(dlv, p->d_ptr.data(), 4 * p->d_ptr.size(), hipMemcpyHostToDevice) == hipSuccess &&
-              hipMemcpy(blv, p->b_ptr.data(), 4 * p->b_ptr.size(), hipMemcpyHostToDevice) == hipSuccess;
-    if (ok && nd)
-        ok = hipMemcpy(dd1, d1.data(), 4 * nd, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(dd2, d2.data(), 4 * nd, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(ddr, drest.data(), 4 * nd, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(ddk, dkp.data(), 4 * nd, hipMemcpyHostToDevice) == hipSuccess;
-    if (ok && nb)
-        ok = hipMemcpy(bb1, b1.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(bb2, b2.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(bb3, b3.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(bbr, brest.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(bbw, bw.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess &&
-             hipMemcpy(bbk, bkp.data(), 4 * nb, hipMemcpyHostToDevice) == hipSuccess;
+    for (const Array& a : arrays) {
+        *a.dst = q;
+        if (ok && a.src) ok = hipMemcpy(q, a.src, a.bytes, hipMemcpyHostToDevice) == hipSuccess;
+        q += align_up(a.bytes);
+    }
     if (!ok) {
         (void)hipFree(p->arena);
         delete p;
@@ -367,8 +418,8 @@ int oc_pbd_get_state(oc_pbd p, float* x, float* v) {
 
 int oc_pbd_num_colors(oc_pbd p, int32_t* n_distance_colors, int32_t* n_bending_colors) {
     if (!p) return set_error(OC_ERR_INVALID_ARGUMENT, "pbd is NULL");
-    if (n_distance_colors) *n_distance_colors = (int32_t)p->d_ptr.size() - 1;
-    if (n_bending_colors) *n_bending_colors = (int32_t)p->b_ptr.size() - 1;
+    if (n_distance_colors) *n_distance_colors = p->n_dcol;
+    if (n_bending_colors) *n_bending_colors = p->n_bcol;
     return OC_OK;
 }
 
@@ -377,7 +428,17 @@ int oc_pbd_step(oc_pbd p, int32_t nsteps, const oc_ellipsoid* e) {
     if (nsteps < 0) return set_error(OC_ERR_INVALID_ARGUMENT, "nsteps < 0");
     const oc::PbdScalars s = pscalars(p);
     const oc::DevPbd& d = p->dev;
-    const int nd_col = (int)p->d_ptr.size() - 1, nb_col = (int)p->b_ptr.size() - 1;
+    if (d.nb == 1) {
+        const int most = 1024 / p->prm.solver_iterations + 1;  // steps of one launch: up to some 10 ms
+        for (int left = nsteps; left > 0; left -= most)
+            OC_HIP(oc::launch_pbd_small(d, s, std::min(most, left), p->prm.solver_iterations, e, p->stream));
+        return OC_OK;
+    }
+    if (d.nb > 1) {
+        for (int n = 0; n < nsteps; n++) OC_HIP(oc::launch_pbd_tiled(d, s, p->prm.solver_iterations, e, p->stream));
+        return OC_OK;
+    }
+    const int nd_col = p->n_dcol, nb_col = p->n_bcol;
     for (int n = 0; n < nsteps; n++) {
         if (p->prm.flags & OC_FLAG_LIST_ORDER) {
             OC_HIP(oc::launch_pbd_predict_seq(d, s, p->stream));
@@ -387,7 +448,7 @@ int oc_pbd_step(oc_pbd p, int32_t nsteps, const oc_ellipsoid* e) {
             OC_HIP(oc::launch_pbd_predict(d, s, p->stream));
             for (int it = 0; it < p->prm.solver_iterations; it++) {
                 for (int c = 0; c < nd_col; c++)
-                    OC_HIP(oc::launch_pbd_distance(d, p->d_ptr[c], p->d_ptr[c + 1] - p->d_ptr[c], p->stream));
+                    OC_HIP(oc::launch_pbd_distance(d, s, p->d_ptr[c], p->d_ptr[c + 1] - p->d_ptr[c], p->stream));
                 for (int c = 0; c < nb_col; c++)
                     OC_HIP(oc::launch_pbd_bending(d, s, p->b_ptr[c], p->b_ptr[c + 1] - p->b_ptr[c], p->stream));
                 if (p->prm.flags & OC_FLAG_GROUND_CLAMP) OC_HIP(oc::launch_pbd_ground(d, p->stream));

@@ -184,6 +184,33 @@ __device__ inline float partial_sum(const float* part, int nt, float* bc) {
     return *bc;
 }
 
+// EllipsoidCollision (OpenCloth_ImplicitEuler/.../main.cpp:727-751) of one
+// point: its place on the surface when p is inside, p otherwise.
+__device__ __forceinline__ V3 ellipsoid_push(const oc_ellipsoid& e, V3 p, bool& inside) {
+    float d0[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        const float t = e.inverse[0 * 4 + r] * p.x + e.inverse[1 * 4 + r] * p.y +
+                        e.inverse[2 * 4 + r] * p.z + e.inverse[3 * 4 + r] * 1.0f;
+        d0[r] = t - e.center[r];
+    }
+    const float dist = sqrtf(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
+    inside = dist < 1.0f;
+    if (!inside) return p;
+#pragma unroll
+    for (int c = 0; c < 3; c++) d0[c] = ((e.radius - dist) * d0[c]) / dist;
+    float delta[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        float t[3] = {e.transform[0 * 4 + a], e.transform[1 * 4 + a], e.transform[2 * 4 + a]};
+        const float tt = t[0] * t[0] + t[1] * t[1] + t[2] * t[2];
+#pragma unroll
+        for (int c = 0; c < 3; c++) t[c] = t[c] / tt;
+        delta[a] = d0[0] * t[0] + d0[1] * t[1] + d0[2] * t[2];
+    }
+    return {p.x + delta[0], p.y + delta[1], p.z + delta[2]};
+}
+
 // Per-spring adjoint terms (oracle.c spring_adjoint, same expression order):
 // derivative of h mu.f + h^2 mu.K v' + h mu.D dv with respect to e = x1-x2
 // (ge), to v1 (gvv) and to ks (gk).

@@ -377,10 +377,40 @@ struct VgridScalars {
 };
 hipError_t launch_vgrid(const DevVgrid& c, const VgridScalars& s, hipStream_t st);
 
-// Position-based dynamics (pbd.hip).  Particle vectors are SoA planes;
-// constraints are stored colour by colour (list order inside a colour).
+// Tiled PBD solver's plan (pbd_plan.cpp).  A constraint family: n constraints
+// of `arity` particles (p) and their colours.
+struct PbdFamily {
+    int n = 0, arity = 2, ncol = 0;
+    const int32_t* p = nullptr;
+    const int* col = nullptr;
+};
+// A constraint as a block projects it: the places of its particles in the
+// block's list (16 bits each; c only of a bending constraint).
+struct PbdRecord {
+    uint32_t ab;
+    float rest;
+    uint32_t c;
+};
+struct PbdPlan {
+    int nb = 0, max_local = 0;
+    std::vector<int32_t> off, own, ids;  // block b's particles: ids[off[b], off[b+1]), the first own[b] its own
+    std::vector<int32_t> cptr;           // per block, record offsets of the colours (distance, then bending) + 1
+    std::vector<PbdRecord> rec;          // rest is filled by the caller
+    std::vector<int32_t> id;             // constraint of each record, in its family
+};
+bool build_pbd_plan(int N, const float* x0, const PbdFamily& dist, const PbdFamily& bend, int owned, int max_local,
+                    float max_work, PbdPlan* out);
+
+// Position-based dynamics (pbd.hip).  Particle vectors are SoA planes.
 constexpr int kPbdBlock = 256;     // particles per reduction block
 constexpr int kPbdSums = 16;       // reduced scalars: [0..6] pass A, [7..15] pass B
+// A cloth of up to kPbdSmall particles is stepped by one workgroup (40x40: 27
+// us per step, tiled 31); beyond it a workgroup of the tiled solver owns up to
+// kPbdOwned particles (64x64: 37 us, one workgroup 54) and holds at most
+// kPbdLocal (16 bytes each in LDS).
+constexpr int kPbdSmall = 2048;
+constexpr int kPbdOwned = 1024;
+constexpr int kPbdLocal = 9216;
 struct DevPbd {
     int N, nblk;
     float* x;
@@ -404,13 +434,27 @@ struct DevPbd {
     const int32_t* d_lv;
     const int32_t* b_lv;
     int nd_lv, nb_lv;
+    // tiled solver (nb > 0): the plan's arrays; t_kp NULL: each family has
+    // one k'
+    int nb, nd_col, nb_col, max_local, n_rec;
+    const int32_t* t_off;
+    const int32_t* t_own;
+    const int32_t* t_ids;
+    const int32_t* t_cptr;
+    const PbdRecord* t_rec;
+    const float* t_kp;
+    float d_kp_all, b_kp_all;
+    float* t2;  // the other predicted positions
 };
 struct PbdScalars {
     float mass, gx, gy, gz, dt, gd, kdamp, global_k, inv_dt;
     int flags;
+    // what the projections divide by between free particles, which all have
+    // the inverse mass w: 1 / (w + w), 2w / (w + w + 2w), 4w / (w + w + 2w)
+    float w, inv_2w, bend_2w, bend_4w;
 };
 hipError_t launch_pbd_predict(const DevPbd& c, const PbdScalars& s, hipStream_t st);
-hipError_t launch_pbd_distance(const DevPbd& c, int first, int count, hipStream_t st);
+hipError_t launch_pbd_distance(const DevPbd& c, const PbdScalars& s, int first, int count, hipStream_t st);
 hipError_t launch_pbd_bending(const DevPbd& c, const PbdScalars& s, int first, int count,
                               hipStream_t st);
 hipError_t launch_pbd_ground(const DevPbd& c, hipStream_t st);
@@ -423,6 +467,16 @@ hipError_t launch_pbd_predict_seq(const DevPbd& c, const PbdScalars& s, hipStrea
 hipError_t launch_pbd_levels(const DevPbd& c, const PbdScalars& s, int iterations, int ground,
                              hipStream_t st);
 hipError_t launch_pbd_integrate(const DevPbd& c, const PbdScalars& s, hipStream_t st);
+// nsteps whole steps of a cloth with one block (nb == 1) in one launch; e may
+// be NULL.
+hipError_t launch_pbd_small(const DevPbd& c, const PbdScalars& s, int nsteps, int iterations, const oc_ellipsoid* e,
+                            hipStream_t st);
+// One step by the tiled solver (nb > 1): the sums, then one launch per solver
+// iteration, the first with the prediction, the last with the collider (e may
+// be NULL) and the velocities.  A single iteration, whose blocks still read
+// their surroundings' x and v, leaves these to launches of their own.
+hipError_t launch_pbd_tiled(const DevPbd& c, const PbdScalars& s, int iterations, const oc_ellipsoid* e,
+                            hipStream_t st);
 
 // Tile shape of the implicit kernels (one workgroup per tile; a multiple of
 // 64 threads).  The reduction order depends on it; oc_cloth_tile_shape

@@ -25,27 +25,9 @@ __global__ __launch_bounds__(256) void k_ellipsoid(float* x, float* w, int N, oc
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= N) return;
     const V3 p = ld3(x, N, i);
-    float d0[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++) {
-        const float t = e.inverse[0 * 4 + r] * p.x + e.inverse[1 * 4 + r] * p.y +
-                        e.inverse[2 * 4 + r] * p.z + e.inverse[3 * 4 + r] * 1.0f;
-        d0[r] = t - e.center[r];
-    }
-    const float dist = sqrtf(d0[0] * d0[0] + d0[1] * d0[1] + d0[2] * d0[2]);
-    if (!(dist < 1.0f)) return;
-#pragma unroll
-    for (int c = 0; c < 3; c++) d0[c] = ((e.radius - dist) * d0[c]) / dist;
-    float delta[3];
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        float t[3] = {e.transform[0 * 4 + a], e.transform[1 * 4 + a], e.transform[2 * 4 + a]};
-        const float tt = t[0] * t[0] + t[1] * t[1] + t[2] * t[2];
-#pragma unroll
-        for (int c = 0; c < 3; c++) t[c] = t[c] / tt;
-        delta[a] = d0[0] * t[0] + d0[1] * t[1] + d0[2] * t[2];
-    }
-    const V3 q = {p.x + delta[0], p.y + delta[1], p.z + delta[2]};
+    bool inside;
+    const V3 q = ellipsoid_push(e, p, inside);
+    if (!inside) return;
     st3(x, N, i, q);
     st3(w, N, i, mode == 1 ? q : V3{0.0f, 0.0f, 0.0f});
 }
