@@ -80,8 +80,8 @@ class ClothBatch:
         check(lib().oc_batch_set_state(self.h, ptr(Xa), ptr(Va)))
 
     def get_state(self):
-        X = np.zeros((self.N, 3), np.float32)
-        V = np.zeros((self.N, 3), np.float32)
+        X = np.empty((self.N, 3), np.float32)
+        V = np.empty((self.N, 3), np.float32)
         check(lib().oc_batch_get_state(self.h, ptr(X), ptr(V)))
         return X, V
 

@@ -96,8 +96,8 @@ class ImplicitCloth:
         check(lib().oc_cloth_set_state(self.h, ptr(Xa), ptr(Va)))
 
     def get_state(self):
-        X = np.zeros((self.N, 3), np.float32)
-        V = np.zeros((self.N, 3), np.float32)
+        X = np.empty((self.N, 3), np.float32)
+        V = np.empty((self.N, 3), np.float32)
         check(lib().oc_cloth_get_state(self.h, ptr(X), ptr(V)))
         return X, V
 
@@ -110,7 +110,7 @@ class ImplicitCloth:
         return self.get_state()[1]
 
     def get_dv(self):
-        dv = np.zeros((self.N, 3), np.float32)
+        dv = np.empty((self.N, 3), np.float32)
         check(lib().oc_cloth_get_dv(self.h, ptr(dv)))
         return dv
 
@@ -277,7 +277,7 @@ class VerletCloth:
             pass
 
     def get_state(self):
-        X = np.zeros((self.N, 3), np.float32); XL = np.zeros((self.N, 3), np.float32)
+        X = np.empty((self.N, 3), np.float32); XL = np.empty((self.N, 3), np.float32)
         check(lib().oc_verlet_get_state(self.h, ptr(X), ptr(XL)))
         return X, XL
 
@@ -350,8 +350,8 @@ class VerletGrid:
         check(lib().oc_vgrid_set_stream(self.h, stream))
 
     def get_state(self):
-        X = np.zeros((self.N, 4), np.float32)
-        XL = np.zeros((self.N, 4), np.float32)
+        X = np.empty((self.N, 4), np.float32)
+        XL = np.empty((self.N, 4), np.float32)
         check(lib().oc_vgrid_get_state(self.h, ptr(X), ptr(XL)))
         return X, XL
 
@@ -422,7 +422,7 @@ class PBDCloth:
         check(lib().oc_pbd_set_state(self.h, ptr(Xa), ptr(Va)))
 
     def get_state(self):
-        X = np.zeros((self.N, 3), np.float32); V = np.zeros((self.N, 3), np.float32)
+        X = np.empty((self.N, 3), np.float32); V = np.empty((self.N, 3), np.float32)
         check(lib().oc_pbd_get_state(self.h, ptr(X), ptr(V)))
         return X, V
 

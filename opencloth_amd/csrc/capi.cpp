@@ -35,6 +35,7 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 struct oc_cloth_s {
     oc::GridTopology topo;
     oc_params prm{};
+    oc::StateIo io;
     hipStream_t stream = nullptr;
     int device = 0;
     int max_it_alloc = 0;
@@ -121,34 +122,24 @@ int ensure_scratch(oc_cloth_s* c, int max_iters) {
     return OC_OK;
 }
 
-void aos_to_soa(const float* a, int N, std::vector<float>& out) {
-    out.resize(3 * (size_t)N);
-    for (int i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) out[(size_t)k * N + i] = a[3 * (size_t)i + k];
-}
-void soa_to_aos(const std::vector<float>& s, int N, float* a) {
-    for (int i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) a[3 * (size_t)i + k] = s[(size_t)k * N + i];
-}
-
-int upload_vec(oc_cloth_s* c, float* dst, const float* host_aos) {
-    std::vector<float> tmp;
-    if (host_aos)
-        aos_to_soa(host_aos, c->dc.N, tmp);
-    else
-        tmp.assign(3 * (size_t)c->dc.N, 0.0f);
-    OC_HIP(hipMemcpyAsync(dst, tmp.data(), tmp.size() * sizeof(float), hipMemcpyHostToDevice,
-                          c->stream));
-    OC_HIP(hipStreamSynchronize(c->stream));
+// A host array of vertices (NULL: zeros) into the planes dst, and back.
+int upload_vec(oc_cloth_s* c, float* dst, const float* host) {
+    OC_HIP(c->io.write({{dst, (size_t)c->dc.N, const_cast<float*>(host)}}, c->stream));
     return OC_OK;
 }
-
-int download_vec(oc_cloth_s* c, const float* src, float* host_aos) {
-    std::vector<float> tmp(3 * (size_t)c->dc.N);
-    OC_HIP(hipMemcpyAsync(tmp.data(), src, tmp.size() * sizeof(float), hipMemcpyDeviceToHost,
-                          c->stream));
-    OC_HIP(hipStreamSynchronize(c->stream));
-    soa_to_aos(tmp, c->dc.N, host_aos);
+int download_vec(oc_cloth_s* c, float* src, float* host) {
+    OC_HIP(c->io.read({{src, (size_t)c->dc.N, host}}, c->stream));
+    return OC_OK;
+}
+// Two at a time, either may be absent (planes NULL, or no host array to read to).
+int upload_vecs(oc_cloth_s* c, float* d0, const float* host0, float* d1, const float* host1) {
+    const size_t N = (size_t)c->dc.N;
+    OC_HIP(c->io.write({{d0, N, const_cast<float*>(host0)}, {d1, N, const_cast<float*>(host1)}}, c->stream));
+    return OC_OK;
+}
+int download_vecs(oc_cloth_s* c, float* s0, float* host0, float* s1, float* host1) {
+    const size_t N = (size_t)c->dc.N;
+    OC_HIP(c->io.read({{s0, N, host0}, {s1, N, host1}}, c->stream));
     return OC_OK;
 }
 
@@ -407,8 +398,7 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     if (hipHostMalloc((void**)&c->ctl_host, sizeof(int) * 8) != hipSuccess)
         return cleanup(fail(OC_ERR_OUT_OF_MEMORY, "hipHostMalloc failed"));
     if ((rc = ensure_scratch(c, params->cg_max_iters)) != OC_OK) return cleanup(rc);
-    if ((rc = upload_vec(c, d.x, x0)) != OC_OK) return cleanup(rc);
-    if ((rc = upload_vec(c, d.v, v0)) != OC_OK) return cleanup(rc);
+    if ((rc = upload_vecs(c, d.x, x0, d.v, v0)) != OC_OK) return cleanup(rc);
     *out = c;
     return OC_OK;
 }
@@ -448,19 +438,15 @@ int oc_cloth_get_params(oc_cloth c, oc_params* p) {
 
 int oc_cloth_set_state(oc_cloth c, const float* x, const float* v) {
     if (!c) return fail(OC_ERR_INVALID_ARGUMENT, "cloth is NULL");
-    int rc;
-    if (x && (rc = upload_vec(c, c->dc.x, x)) != OC_OK) return rc;
-    if (v && (rc = upload_vec(c, c->dc.v, v)) != OC_OK) return rc;
+    const int rc = upload_vecs(c, x ? c->dc.x : nullptr, x, v ? c->dc.v : nullptr, v);
+    if (rc != OC_OK) return rc;
     c->assembled = false;
     return OC_OK;
 }
 
 int oc_cloth_get_state(oc_cloth c, float* x, float* v) {
     if (!c) return fail(OC_ERR_INVALID_ARGUMENT, "cloth is NULL");
-    int rc;
-    if (x && (rc = download_vec(c, c->dc.x, x)) != OC_OK) return rc;
-    if (v && (rc = download_vec(c, c->dc.v, v)) != OC_OK) return rc;
-    return OC_OK;
+    return download_vecs(c, c->dc.x, x, c->dc.v, v);
 }
 
 int oc_cloth_get_dv(oc_cloth c, float* dv) {
@@ -883,8 +869,7 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
     float* gx[2] = {rv.vec[7], rv.vec[8]};
     float* gv[2] = {rv.vec[9], rv.vec[10]};
     int rc;
-    if ((rc = upload_vec(c, gx[0], grad_x)) != OC_OK) return rc;
-    if ((rc = upload_vec(c, gv[0], grad_v)) != OC_OK) return rc;
+    if ((rc = upload_vecs(c, gx[0], grad_x, gv[0], grad_v)) != OC_OK) return rc;
     OC_HIP(hipMemsetAsync(rv.gks, 0, sizeof(float) * std::max(c->topo.S, 1), c->stream));
     const oc::StepScalars s = scalars(c, c->prm.dt);
     oc::StepScalars s_cold = s;
@@ -937,8 +922,7 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
                               c->stream));
         OC_HIP(hipStreamSynchronize(c->stream));
     }
-    if (grad_x0 && (rc = download_vec(c, gx[cur], grad_x0)) != OC_OK) return rc;
-    if (grad_v0 && (rc = download_vec(c, gv[cur], grad_v0)) != OC_OK) return rc;
+    if ((rc = download_vecs(c, gx[cur], grad_x0, gv[cur], grad_v0)) != OC_OK) return rc;
     OC_HIP(hipStreamSynchronize(c->stream));
     c->assembled = false;
     return OC_OK;

@@ -30,6 +30,7 @@ struct oc_batch_s {
     int n_planes = 0;
     std::vector<int> nx, ny, voff, nverts;
     oc_params prm{};
+    oc::StateIo io;
     oc_batch_schedule sched{512, 8};
     hipStream_t stream = nullptr;
     hipStream_t capture_stream = nullptr;
@@ -423,6 +424,7 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
         std::string e = oc_last_error();
         return fail_free(rc, e);
     }
+    (void)b->io.prepare((size_t)b->Ntot, 3);  // (a transfer reserves and reports again)
     *out = b;
     rc = oc_batch_set_state(b, x0, v0);
     if (rc != OC_OK) {
@@ -485,18 +487,8 @@ int oc_batch_threads_per_cloth(oc_batch b, int32_t* threads) {
 int oc_batch_set_state(oc_batch b, const float* x, const float* v) {
     if (!b) return set_error(OC_ERR_INVALID_ARGUMENT, "batch is NULL");
     const size_t N = b->Ntot;
-    std::vector<float> t(3 * N);
-    // ordered on the batch's stream; t is reused, so each copy completes first
-    auto up = [&](float* dst, const float* src) -> int {
-        for (size_t i = 0; i < N; i++)
-            for (int k = 0; k < 3; k++) t[k * N + i] = src[3 * i + k];
-        OC_HIP(hipMemcpyAsync(dst, t.data(), t.size() * 4, hipMemcpyHostToDevice, b->stream));
-        OC_HIP(hipStreamSynchronize(b->stream));
-        return OC_OK;
-    };
-    int rc;
-    if (x && (rc = up(b->dc.x, x)) != OC_OK) return rc;
-    if (v && (rc = up(b->dc.v, v)) != OC_OK) return rc;
+    OC_HIP(b->io.write({{x ? b->dc.x : nullptr, N, const_cast<float*>(x)}, {v ? b->dc.v : nullptr, N, const_cast<float*>(v)}},
+                       b->stream));
     if (x) {
         OC_HIP(hipMemsetAsync(b->dc.dv, 0, sizeof(float) * 3 * N, b->stream));
         OC_HIP(hipStreamSynchronize(b->stream));
@@ -507,17 +499,8 @@ int oc_batch_set_state(oc_batch b, const float* x, const float* v) {
 int oc_batch_get_state(oc_batch b, float* x, float* v) {
     if (!b) return set_error(OC_ERR_INVALID_ARGUMENT, "batch is NULL");
     const size_t N = b->Ntot;
-    std::vector<float> t(3 * N);
     OC_HIP(hipStreamSynchronize(b->stream));
-    auto down = [&](float* dst, const float* src) -> int {
-        OC_HIP(hipMemcpy(t.data(), src, t.size() * 4, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < N; i++)
-            for (int k = 0; k < 3; k++) dst[3 * i + k] = t[k * N + i];
-        return OC_OK;
-    };
-    int rc;
-    if (x && (rc = down(x, b->dc.x)) != OC_OK) return rc;
-    if (v && (rc = down(v, b->dc.v)) != OC_OK) return rc;
+    OC_HIP(b->io.read({{b->dc.x, N, x}, {b->dc.v, N, v}}, b->stream));
     return OC_OK;
 }
 
@@ -696,27 +679,6 @@ int batch_restore(oc_batch_s* b, const float* src) {
     return OC_OK;
 }
 
-int batch_upload_aos(oc_batch_s* b, float* dst, const float* aos) {
-    const size_t N = b->Ntot;
-    std::vector<float> t(3 * N, 0.0f);
-    if (aos)
-        for (size_t i = 0; i < N; i++)
-            for (int k = 0; k < 3; k++) t[k * N + i] = aos[3 * i + k];
-    OC_HIP(hipMemcpyAsync(dst, t.data(), t.size() * 4, hipMemcpyHostToDevice, b->stream));
-    OC_HIP(hipStreamSynchronize(b->stream));
-    return OC_OK;
-}
-
-int batch_download_aos(oc_batch_s* b, const float* src, float* aos) {
-    const size_t N = b->Ntot;
-    std::vector<float> t(3 * N);
-    OC_HIP(hipMemcpyAsync(t.data(), src, t.size() * 4, hipMemcpyDeviceToHost, b->stream));
-    OC_HIP(hipStreamSynchronize(b->stream));
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) aos[3 * i + k] = t[k * N + i];
-    return OC_OK;
-}
-
 }  // namespace
 
 extern "C" {
@@ -771,8 +733,8 @@ int oc_batch_rollout_backward(oc_batch b, const float* grad_x, const float* grad
     BatchRollout rv = batch_rollout_views(b, nseg, every);
     int rc;
     if ((rc = ensure_graph(b)) != OC_OK) return rc;
-    if ((rc = batch_upload_aos(b, rv.gx[0], grad_x)) != OC_OK) return rc;
-    if ((rc = batch_upload_aos(b, rv.gv[0], grad_v)) != OC_OK) return rc;
+    const size_t N = (size_t)b->Ntot;
+    OC_HIP(b->io.write({{rv.gx[0], N, const_cast<float*>(grad_x)}, {rv.gv[0], N, const_cast<float*>(grad_v)}}, b->stream));
     OC_HIP(hipMemsetAsync(rv.gks, 0, sizeof(float) * std::max(b->Stot, 1), b->stream));
     oc::StepScalars s = batch_scalars(b);
     s.warm = 0;  // the adjoint assembly must not read or keep a warm start
@@ -812,8 +774,7 @@ int oc_batch_rollout_backward(oc_batch b, const float* grad_x, const float* grad
         OC_HIP(hipMemcpyAsync(grad_ks, rv.gks, sizeof(float) * b->Stot, hipMemcpyDeviceToHost, b->stream));
         OC_HIP(hipStreamSynchronize(b->stream));
     }
-    if (grad_x0 && (rc = batch_download_aos(b, rv.gx[cur], grad_x0)) != OC_OK) return rc;
-    if (grad_v0 && (rc = batch_download_aos(b, rv.gv[cur], grad_v0)) != OC_OK) return rc;
+    OC_HIP(b->io.read({{rv.gx[cur], N, grad_x0}, {rv.gv[cur], N, grad_v0}}, b->stream));
     OC_HIP(hipStreamSynchronize(b->stream));
     return OC_OK;
 }

@@ -99,6 +99,7 @@ int levels(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<i
 struct oc_pbd_s {
     int N = 0;
     oc_pbd_params prm{};
+    oc::StateIo io;
     hipStream_t stream = nullptr;
     void* arena = nullptr;
     oc::DevPbd dev{};
@@ -127,26 +128,6 @@ oc::PbdScalars pscalars(const oc_pbd_s* p) {
     s.bend_2w = (2.0f * s.w) / wsum;
     s.bend_4w = (4.0f * s.w) / wsum;
     return s;
-}
-
-int upload_aos(oc_pbd_s* p, float* dst, const float* aos) {
-    const size_t N = p->N;
-    std::vector<float> t(3 * N);
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) t[k * N + i] = aos ? aos[3 * i + k] : 0.0f;
-    OC_HIP(hipMemcpyAsync(dst, t.data(), t.size() * 4, hipMemcpyHostToDevice, p->stream));
-    OC_HIP(hipStreamSynchronize(p->stream));
-    return OC_OK;
-}
-
-int download_aos(oc_pbd_s* p, const float* src, float* aos) {
-    const size_t N = p->N;
-    std::vector<float> t(3 * N);
-    OC_HIP(hipMemcpyAsync(t.data(), src, t.size() * 4, hipMemcpyDeviceToHost, p->stream));
-    OC_HIP(hipStreamSynchronize(p->stream));
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) aos[3 * i + k] = t[k * N + i];
-    return OC_OK;
 }
 
 int check_pbd_params(const oc_pbd_params* p) {
@@ -373,6 +354,7 @@ int oc_pbd_create(int32_t n_vertices, const float* x0, const uint8_t* pinned,
         delete p;
         return set_error(OC_ERR_DEVICE, "upload failed");
     }
+    (void)p->io.prepare((size_t)N, 3);  // (a transfer reserves and reports again)
     *out = p;
     rc = oc_pbd_set_state(p, x0, nullptr);
     if (rc != OC_OK) {
@@ -402,17 +384,16 @@ int oc_pbd_set_stream(oc_pbd p, void* stream) {
 // the first call from oc_pbd_create.
 int oc_pbd_set_state(oc_pbd p, const float* x, const float* v) {
     if (!p) return set_error(OC_ERR_INVALID_ARGUMENT, "pbd is NULL");
-    int rc;
-    if (x && (rc = upload_aos(p, p->dev.x, x)) != OC_OK) return rc;
-    if (v && (rc = upload_aos(p, p->dev.v, v)) != OC_OK) return rc;
+    const size_t N = (size_t)p->N;
+    OC_HIP(p->io.write({{x ? p->dev.x : nullptr, N, const_cast<float*>(x)},
+                        {v ? p->dev.v : nullptr, N, const_cast<float*>(v)}}, p->stream));
     return OC_OK;
 }
 
 int oc_pbd_get_state(oc_pbd p, float* x, float* v) {
     if (!p) return set_error(OC_ERR_INVALID_ARGUMENT, "pbd is NULL");
-    int rc;
-    if (x && (rc = download_aos(p, p->dev.x, x)) != OC_OK) return rc;
-    if (v && (rc = download_aos(p, p->dev.v, v)) != OC_OK) return rc;
+    const size_t N = (size_t)p->N;
+    OC_HIP(p->io.read({{p->dev.x, N, x}, {p->dev.v, N, v}}, p->stream));
     return OC_OK;
 }
 

@@ -25,6 +25,7 @@ using oc::set_error;
 struct oc_verlet_s {
     oc::GridTopology topo;
     oc_verlet_params prm{};
+    oc::StateIo io;
     hipStream_t stream = nullptr;
     void* arena = nullptr;
     float* pos[3] = {nullptr, nullptr, nullptr};  // rotated: cur, last, next
@@ -74,26 +75,6 @@ oc::VerletScalars vscalars(const oc_verlet_s* v) {
     s.dt = v->prm.dt;
     s.flags = v->prm.flags;
     return s;
-}
-
-int upload_aos(oc_verlet_s* v, float* dst, const float* aos) {
-    const size_t N = v->topo.N;
-    std::vector<float> t(3 * N);
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) t[k * N + i] = aos[3 * i + k];
-    OC_HIP(hipMemcpyAsync(dst, t.data(), t.size() * 4, hipMemcpyHostToDevice, v->stream));
-    OC_HIP(hipStreamSynchronize(v->stream));
-    return OC_OK;
-}
-
-int download_aos(oc_verlet_s* v, const float* src, float* aos) {
-    const size_t N = v->topo.N;
-    std::vector<float> t(3 * N);
-    OC_HIP(hipMemcpyAsync(t.data(), src, t.size() * 4, hipMemcpyDeviceToHost, v->stream));
-    OC_HIP(hipStreamSynchronize(v->stream));
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 3; k++) aos[3 * i + k] = t[k * N + i];
-    return OC_OK;
 }
 
 }  // namespace
@@ -193,6 +174,7 @@ int oc_verlet_create(int32_t nx, int32_t ny, const float* x0, const float* x_las
         delete v;
         return set_error(OC_ERR_DEVICE, "upload failed");
     }
+    (void)v->io.prepare((size_t)v->topo.N, 3);  // (a transfer reserves and reports again)
     *out = v;
     rc = oc_verlet_set_state(v, x0, x_last0 ? x_last0 : x0);
     if (rc != OC_OK) {
@@ -220,24 +202,23 @@ int oc_verlet_set_stream(oc_verlet v, void* stream) {
 
 int oc_verlet_set_state(oc_verlet v, const float* x, const float* x_last) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
-    int rc;
-    if (x && (rc = upload_aos(v, v->pos[v->cur], x)) != OC_OK) return rc;
-    if (x_last && (rc = upload_aos(v, v->pos[v->last], x_last)) != OC_OK) return rc;
+    const size_t N = (size_t)v->topo.N;
+    OC_HIP(v->io.write({{x ? v->pos[v->cur] : nullptr, N, const_cast<float*>(x)},
+                        {x_last ? v->pos[v->last] : nullptr, N, const_cast<float*>(x_last)}}, v->stream));
     return OC_OK;
 }
 
 int oc_verlet_get_state(oc_verlet v, float* x, float* x_last) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
-    int rc;
-    if (x && (rc = download_aos(v, v->pos[v->cur], x)) != OC_OK) return rc;
-    if (x_last && (rc = download_aos(v, v->pos[v->last], x_last)) != OC_OK) return rc;
+    const size_t N = (size_t)v->topo.N;
+    OC_HIP(v->io.read({{v->pos[v->cur], N, x}, {v->pos[v->last], N, x_last}}, v->stream));
     return OC_OK;
 }
 
 int oc_verlet_compute_forces(oc_verlet v, float* f_out) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     OC_HIP(oc::launch_verlet_forces(view(v), vscalars(v), v->stream));
-    if (f_out) return download_aos(v, v->f, f_out);
+    if (f_out) OC_HIP(v->io.read({{v->f, (size_t)v->topo.N, f_out}}, v->stream));
     return OC_OK;
 }
 

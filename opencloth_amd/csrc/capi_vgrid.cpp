@@ -26,6 +26,7 @@ using oc::set_error;
 struct oc_vgrid_s {
     int nx = 0, ny = 0, N = 0;
     oc_vgrid_params prm{};
+    oc::StateIo io;
     hipStream_t stream = nullptr;
     void* arena = nullptr;
     float* x[2] = {nullptr, nullptr};   // position sets, ping-ponged
@@ -67,29 +68,6 @@ oc::VgridScalars scalars(const oc_vgrid_s* g) {
         s.kd[c] = p.kd[c];
     }
     return s;
-}
-
-// Host AoS float4 -> xyz planes at dst, w into w (when given).
-int upload4(oc_vgrid_s* g, float* dst, float* w, const float* aos) {
-    const size_t N = g->N;
-    std::vector<float> t(4 * N);
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 4; k++) t[k * N + i] = aos[4 * i + k];
-    OC_HIP(hipMemcpyAsync(dst, t.data(), 3 * N * sizeof(float), hipMemcpyHostToDevice, g->stream));
-    OC_HIP(hipMemcpyAsync(w, t.data() + 3 * N, N * sizeof(float), hipMemcpyHostToDevice, g->stream));
-    OC_HIP(hipStreamSynchronize(g->stream));
-    return OC_OK;
-}
-
-int download4(oc_vgrid_s* g, const float* src, const float* w, float* aos) {
-    const size_t N = g->N;
-    std::vector<float> t(4 * N);
-    OC_HIP(hipMemcpyAsync(t.data(), src, 3 * N * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-    OC_HIP(hipMemcpyAsync(t.data() + 3 * N, w, N * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-    OC_HIP(hipStreamSynchronize(g->stream));
-    for (size_t i = 0; i < N; i++)
-        for (int k = 0; k < 4; k++) aos[4 * i + k] = t[k * N + i];
-    return OC_OK;
 }
 
 }  // namespace
@@ -140,6 +118,7 @@ int oc_vgrid_create(int32_t width, int32_t height, const float* x0, const float*
         pins[0] = 1;
         pins[width - 1] = 1;
     }
+    (void)g->io.prepare((size_t)g->N, 4);  // (a transfer reserves and reports again)
     *out = g;
     if (hipMemset(g->arena, 0, total) != hipSuccess ||
         hipMemcpy(g->pin, pins.data(), N, hipMemcpyHostToDevice) != hipSuccess) {
@@ -181,17 +160,16 @@ int oc_vgrid_set_params(oc_vgrid g, const oc_vgrid_params* p) {
 
 int oc_vgrid_set_state(oc_vgrid g, const float* x, const float* x_last) {
     if (!g) return set_error(OC_ERR_INVALID_ARGUMENT, "grid is NULL");
-    int rc;
-    if (x && (rc = upload4(g, g->x[g->cur], g->wx, x)) != OC_OK) return rc;
-    if (x_last && (rc = upload4(g, g->xl[g->cur], g->wxl, x_last)) != OC_OK) return rc;
+    const size_t N = (size_t)g->N;
+    OC_HIP(g->io.write({{x ? g->x[g->cur] : nullptr, N, const_cast<float*>(x), g->wx},
+                        {x_last ? g->xl[g->cur] : nullptr, N, const_cast<float*>(x_last), g->wxl}}, g->stream));
     return OC_OK;
 }
 
 int oc_vgrid_get_state(oc_vgrid g, float* x, float* x_last) {
     if (!g) return set_error(OC_ERR_INVALID_ARGUMENT, "grid is NULL");
-    int rc;
-    if (x && (rc = download4(g, g->x[g->cur], g->wx, x)) != OC_OK) return rc;
-    if (x_last && (rc = download4(g, g->xl[g->cur], g->wxl, x_last)) != OC_OK) return rc;
+    const size_t N = (size_t)g->N;
+    OC_HIP(g->io.read({{g->x[g->cur], N, x, g->wx}, {g->xl[g->cur], N, x_last, g->wxl}}, g->stream));
     return OC_OK;
 }
 

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -490,6 +492,43 @@ hipError_t launch_pbd_tiled(const DevPbd& c, const PbdScalars& s, int iterations
 #endif
 constexpr int kTileX = OC_TILE_X;
 constexpr int kTileY = OC_TILE_Y;
+
+// ---- state transfers (state_io.hip) ----------------------------------------
+// n vertices in planes (xyz, stride n; w the fourth components, NULL for
+// arrays of xyz) and the caller's array of them.  Without planes it is left
+// out; without a host array there is nothing to read, or zeros to write.
+struct IoArray {
+    float* planes;
+    size_t n;
+    float* host;
+    float* w = nullptr;
+    int comps() const { return w ? 4 : 3; }
+    size_t bytes(size_t m) const { return sizeof(float) * comps() * m; }
+};
+// A handle's pinned slots (at most 8 MiB, by need) for its transfers.  Both
+// calls are ordered after the stream's work and complete before they return;
+// of several threads one transfers at a time.
+class StateIo {
+  public:
+    StateIo() = default;
+    StateIo(const StateIo&) = delete;
+    StateIo& operator=(const StateIo&) = delete;
+    ~StateIo();
+    // The slots for states of two arrays of n vertices, ahead of the first
+    // transfer (8 MiB of pinned memory take about half a millisecond).
+    hipError_t prepare(size_t n, int comps) { return reserve(2 * sizeof(float) * comps * n + 32); }
+    hipError_t read(std::initializer_list<IoArray> a, hipStream_t st) { return move(true, a.begin(), (int)a.size(), st); }
+    hipError_t write(std::initializer_list<IoArray> a, hipStream_t st) { return move(false, a.begin(), (int)a.size(), st); }
+
+  private:
+    hipError_t move(bool read, const IoArray* a, int n, hipStream_t st);  // at most two, alike in w
+    hipError_t reserve(size_t total);
+    hipError_t chunks(bool read, const IoArray* a, int n, size_t k0, size_t step, hipStream_t st);
+    std::mutex lock_;
+    char* pinned_ = nullptr;
+    size_t bytes_ = 0;
+    hipEvent_t ev_[8] = {};
+};
 
 // ---- batched cloths --------------------------------------------------------
 // All cloths' vertices are concatenated (SoA planes of stride Ntot); slot
