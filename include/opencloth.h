@@ -381,13 +381,16 @@ int oc_pbd_synchronize(oc_pbd pbd);
 int oc_cloth_set_spring_stiffness(oc_cloth cloth, const float* ks);
 int oc_cloth_get_spring_stiffness(oc_cloth cloth, float* ks);
 /* Run nsteps implicit steps from the current state with dv reset to zero,
- * keeping a device checkpoint (x, v, dv) every checkpoint_every steps for
- * oc_cloth_rollout_backward.  The state ends at step nsteps. */
+ * keeping device checkpoints (x, v, dv) for oc_cloth_rollout_backward: every
+ * checkpoint_every steps, or of every step when these (36 bytes per vertex
+ * and step) fit an eighth of the free device memory and 8 GiB.  The state
+ * ends at step nsteps. */
 int oc_cloth_rollout_forward(oc_cloth cloth, int32_t nsteps, int32_t checkpoint_every);
 /* Hand-written adjoint of the last rollout_forward: given dL/dx and dL/dv at
  * its final state (host AoS; grad_v may be NULL for zero), return dL/dks
  * (n_springs floats), dL/dx0 and dL/dv0 (host AoS; any output may be NULL).
- * Each segment between checkpoints is recomputed forward, then every step's
+ * Each segment between checkpoints is recomputed forward (not where every
+ * state was kept, unless parameters were set since), then every step's
  * adjoint solves the same symmetric system (filtered CG) and gathers the
  * derivatives of the spring forces and Jacobians per vertex.  The state is
  * restored to the rollout's final state; synchronises. */

@@ -520,51 +520,8 @@ __device__ float assemble_once(const DevBatch& c, const StepScalars& s, const Ba
     return t;
 }
 
-// Adjoint gather for vertex i (same as the single-cloth k_adj_gather):
-// c.x, c.v the pre-step state, c.dv the adjoint solve mu, a.dvsol the step's
-// solution.
-__device__ inline void adjoint_gather_vertex(const DevBatch& c, const StepScalars& s,
-                                             const BatchAdjBufs& a, int i, int nx) {
-    const int N = c.Ntot;
-    const V3 xi = ld3(c.x, N, i), vi = ld3(c.v, N, i), mi = ld3(c.dv, N, i),
-             pi = ld3(a.dvsol, N, i);
-    const V3 wi = add3(vi, pi);
-    V3 gx = ld3(a.gx_out, N, i), gv = ld3(a.gvt, N, i);
-    if (s.damp != 0.0f && !c.pin[i])  // the damping force c v_i: dJ/dv_i += h c mu_i
-        gv = {gv.x + s.h * (s.damp * mi.x), gv.y + s.h * (s.damp * mi.y), gv.z + s.h * (s.damp * mi.z)};
-    for (int k = 0; k < c.wa; k++) {
-        const int sp = c.ainc_s[(size_t)k * N + i];
-        if (sp < 0) break;
-        const uint16_t m = c.ainc_m[(size_t)k * N + i];
-        const int j = i + slot_dj(m) * nx + slot_di(m);
-        const V3 xj = ld3(c.x, N, j), vj = ld3(c.v, N, j), mj = ld3(c.dv, N, j),
-                 pj = ld3(a.dvsol, N, j);
-        const V3 wj = add3(vj, pj);
-        const bool second = (m >> 8) & 1u;
-        const size_t plane = (size_t)c.wa * N, o = (size_t)k * N + i;
-        const float L0 = c.slot_c[o], ks = c.slot_c[plane + o], kd = c.slot_c[2 * plane + o];
-        float ge[3], gvv[3], gk;
-        if (second)
-            spring_adjoint(xj, xi, vj, vi, mj, mi, wj, wi, pj, pi, L0, ks, kd, s.h,
-                           s.hh, ge, gvv, gk);
-        else
-            spring_adjoint(xi, xj, vi, vj, mi, mj, wi, wj, pi, pj, L0, ks, kd, s.h,
-                           s.hh, ge, gvv, gk);
-        if (second) {
-            gx = {gx.x - ge[0], gx.y - ge[1], gx.z - ge[2]};
-            gv = {gv.x - gvv[0], gv.y - gvv[1], gv.z - gvv[2]};
-        } else {
-            gx = {gx.x + ge[0], gx.y + ge[1], gx.z + ge[2]};
-            gv = {gv.x + gvv[0], gv.y + gvv[1], gv.z + gvv[2]};
-            a.gks[sp] = a.gks[sp] + gk;
-        }
-    }
-    st3(a.gx_in, N, i, gx);
-    st3(a.gv_in, N, i, gv);
-}
-
 // ADJ = false: forward step.  ADJ = true: one step's adjoint at the state in
-// c.x/c.v (assembly without warm start, CG for mu in c.dv, gather).
+// c.x/c.v up to the gather (assembly without warm start, CG for mu in c.dv).
 // ONCE: the spring-once assembly (c.asm_once), a separate instantiation so
 // the default kernel carries none of its registers.
 template <int NT, bool ADJ, bool ONCE>
@@ -781,9 +738,7 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
             sst[g] = st;
         }
         __syncthreads();
-        if constexpr (ADJ) {
-            for (int vv = lt; vv < Ni; vv += T) adjoint_gather_vertex(c, s, adj, voff + vv, nx);
-        } else {
+        if constexpr (!ADJ) {
             bool bad = false;
             for (int vv = lt; vv < Ni; vv += T) {
                 const int i = voff + vv;
@@ -806,6 +761,34 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
         }
         __syncthreads();
     }
+}
+
+// The adjoint's gather (as the single cloth's k_adj_gather): c.x, c.v the
+// pre-step state, c.dv the adjoint solve mu, a.dvsol the step's solution.  A
+// launch of its own over all vertices: it needs no cloth's order, and inside
+// the solve's workgroups the largest cloths' gathers ran on while other CUs
+// were idle.  64 cloths of 32x32 to 96x96: the adjoint's launches take 600 us
+// per step (73 of them here), 1.0 ms as one launch.
+constexpr int kGatherThreads = 64;
+__global__ __launch_bounds__(kGatherThreads) void k_batch_gather(DevBatch c, StepScalars s, BatchAdjBufs a) {
+    const int N = c.Ntot, i = blockIdx.x * kGatherThreads + threadIdx.x;
+    if (i >= N) return;
+    const V3 mi = ld3(c.dv, N, i);
+    V3 gx = ld3(a.gx_out, N, i), gv = ld3(a.gvt, N, i);
+    if (s.damp != 0.0f && !c.pin[i])  // the damping force c v_i: dJ/dv_i += h c mu_i
+        gv = {gv.x + s.h * (s.damp * mi.x), gv.y + s.h * (s.damp * mi.y), gv.z + s.h * (s.damp * mi.z)};
+    const AdjGatherIn in = {c.x, c.v, c.dv, a.dvsol, c.ainc_s, c.ainc_m, N, c.wa};
+    const size_t plane = (size_t)c.wa * N;
+    adj_gather_springs(in, i, c.row[i], s.h, s.hh,
+                       [&](int k, int, float& L0, float& ks, float& kd) {
+                           const size_t o = (size_t)k * N + i;
+                           L0 = c.slot_c[o];
+                           ks = c.slot_c[plane + o];
+                           kd = c.slot_c[2 * plane + o];
+                       },
+                       a.gks, gx, gv);
+    st3(a.gx_in, N, i, gx);
+    st3(a.gv_in, N, i, gv);
 }
 
 // Owner-plane constants from the slot-major copies: the first spring of the
@@ -899,6 +882,13 @@ static hipError_t launch_batch(const DevBatch& c, const StepScalars& s, const Ba
 hipError_t launch_batch_step(const DevBatch& c, const StepScalars& s, int block_threads, int grid,
                              hipStream_t st) {
     return launch_batch<false>(c, s, BatchAdjBufs{}, block_threads, grid, st);
+}
+
+hipError_t launch_batch_gather(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a, hipStream_t st) {
+    if (c.Ntot < 1) return hipSuccess;
+    hipLaunchKernelGGL(k_batch_gather, dim3((c.Ntot + kGatherThreads - 1) / kGatherThreads), dim3(kGatherThreads), 0, st,
+                       c, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_batch_adjoint(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a,

@@ -48,10 +48,7 @@ struct oc_cloth_s {
     int32_t* spring_cst = nullptr;  // stencil assembly form: owner-plane index per spring
     bool assembled = false;
     // differentiable rollouts: checkpoints, one segment of states, adjoint vectors
-    void* adj_arena = nullptr;
-    size_t adj_bytes = 0;
-    int roll_steps = 0, roll_every = 0;
-    bool roll_valid = false;
+    oc::RolloutStore roll;
 };
 
 namespace {
@@ -409,7 +406,7 @@ int oc_cloth_destroy(oc_cloth c) {
     if (c->arena) (void)hipFree(c->arena);
     if (c->scratch) (void)hipFree(c->scratch);
     if (c->ctl_host) (void)hipHostFree(c->ctl_host);
-    if (c->adj_arena) (void)hipFree(c->adj_arena);
+    if (c->roll.arena) (void)hipFree(c->roll.arena);
     delete c;
     return OC_OK;
 }
@@ -426,6 +423,7 @@ int oc_cloth_set_params(oc_cloth c, const oc_params* p) {
     if (rc != OC_OK) return rc;
     if ((rc = ensure_scratch(c, p->cg_max_iters)) != OC_OK) return rc;  // old params stay on failure
     c->prm = *p;
+    c->roll.same = false;
     c->dc.persistent = (p->flags & OC_FLAG_CG_PERSISTENT) ? oc::persistent_cg_grid(c->dc) : 0;
     return OC_OK;
 }
@@ -750,7 +748,7 @@ int oc_cloth_set_spring_stiffness(oc_cloth c, const float* ks) {
                           c->stream));
     if (c->dc.stencil_asm) OC_HIP(oc::launch_scatter_cst(c->dc, c->spring_cst, c->topo.S, 1, 1, c->stream));
     OC_HIP(hipStreamSynchronize(c->stream));
-    c->roll_valid = false;
+    c->roll.valid = false;
     return OC_OK;
 }
 
@@ -766,45 +764,34 @@ int oc_cloth_get_spring_stiffness(oc_cloth c, float* ks) {
 
 namespace {
 
-// Views into the rollout arena: checkpoints [(nseg+1) x (x,v,dv)], one
-// segment of pre-step states and solutions [every x (x,v,dv)], 11 adjoint
-// vectors and the per-spring gradient.
+// The backward pass' vectors, behind the rollout's states.
 struct RolloutViews {
-    float* ckpt;
-    float* seg;
     float* vec[11];
     float* gks;
 };
 
-RolloutViews rollout_views(oc_cloth_s* c, int nseg, int every) {
-    const size_t v3 = 3 * (size_t)c->dc.N;
+RolloutViews rollout_views(oc_cloth_s* c) {
+    const size_t kf = oc::kept_floats((size_t)c->dc.N);
     RolloutViews r;
-    float* p = (float*)c->adj_arena;
-    r.ckpt = p;
-    p += (size_t)(nseg + 1) * 3 * v3;
-    r.seg = p;
-    p += (size_t)every * 3 * v3;
+    float* p = c->roll.rest((size_t)c->dc.N);
     for (int k = 0; k < 11; k++) {
         r.vec[k] = p;
-        p += v3;
+        p += kf;
     }
     r.gks = p;
     return r;
 }
 
 int save_state(oc_cloth_s* c, float* dst) {
-    const size_t b = sizeof(float) * 3 * (size_t)c->dc.N;
-    OC_HIP(hipMemcpyAsync(dst, c->dc.x, b, hipMemcpyDeviceToDevice, c->stream));
-    OC_HIP(hipMemcpyAsync((char*)dst + b, c->dc.v, b, hipMemcpyDeviceToDevice, c->stream));
-    OC_HIP(hipMemcpyAsync((char*)dst + 2 * b, c->dc.dv, b, hipMemcpyDeviceToDevice, c->stream));
+    OC_HIP(oc::launch_keep_state(c->dc.x, c->dc.v, c->dc.dv, dst, oc::kept_floats((size_t)c->dc.N), c->stream));
     return OC_OK;
 }
 
 int load_state(oc_cloth_s* c, const float* src) {
-    const size_t b = sizeof(float) * 3 * (size_t)c->dc.N;
+    const size_t b = sizeof(float) * 3 * (size_t)c->dc.N, kf = oc::kept_floats((size_t)c->dc.N);
     OC_HIP(hipMemcpyAsync(c->dc.x, src, b, hipMemcpyDeviceToDevice, c->stream));
-    OC_HIP(hipMemcpyAsync(c->dc.v, (const char*)src + b, b, hipMemcpyDeviceToDevice, c->stream));
-    OC_HIP(hipMemcpyAsync(c->dc.dv, (const char*)src + 2 * b, b, hipMemcpyDeviceToDevice, c->stream));
+    OC_HIP(hipMemcpyAsync(c->dc.v, src + kf, b, hipMemcpyDeviceToDevice, c->stream));
+    OC_HIP(hipMemcpyAsync(c->dc.dv, src + 2 * kf, b, hipMemcpyDeviceToDevice, c->stream));
     return OC_OK;
 }
 
@@ -822,36 +809,20 @@ extern "C" {
 int oc_cloth_rollout_forward(oc_cloth c, int32_t nsteps, int32_t every) {
     if (!c) return fail(OC_ERR_INVALID_ARGUMENT, "cloth is NULL");
     if (nsteps < 1 || every < 1) return fail(OC_ERR_INVALID_ARGUMENT, "nsteps and checkpoint_every must be >= 1");
-    c->roll_valid = false;  // until this rollout has completed
-    every = std::min(every, nsteps);
-    const int nseg = (nsteps + every - 1) / every;
-    const size_t v3 = 3 * (size_t)c->dc.N;
-    const size_t need = sizeof(float) * ((size_t)(nseg + 1) * 3 * v3 + (size_t)every * 3 * v3 +
-                                         11 * v3 + (size_t)std::max(c->topo.S, 1));
-    if (need > c->adj_bytes) {
-        if (c->adj_arena) {
-            OC_HIP(hipStreamSynchronize(c->stream));
-            OC_HIP(hipFree(c->adj_arena));
-            c->adj_arena = nullptr;
-            c->adj_bytes = 0;
-        }
-        if (hipMalloc(&c->adj_arena, need) != hipSuccess)
-            return fail(OC_ERR_OUT_OF_MEMORY, "hipMalloc of rollout checkpoints failed");
-        c->adj_bytes = need;
-    }
-    RolloutViews rv = rollout_views(c, nseg, every);
+    c->roll.valid = false;  // until this rollout has completed
+    const size_t N = (size_t)c->dc.N;
+    const hipError_t re = c->roll.reserve(N, nsteps, every, 11 * oc::kept_floats(N) + std::max(c->topo.S, 1), c->stream);
+    if (re == hipErrorOutOfMemory) return fail(OC_ERR_OUT_OF_MEMORY, "hipMalloc of rollout checkpoints failed");
+    OC_HIP(re);
     const oc::StepScalars s = scalars(c, c->prm.dt);
-    OC_HIP(hipMemsetAsync(c->dc.dv, 0, sizeof(float) * v3, c->stream));
+    OC_HIP(hipMemsetAsync(c->dc.dv, 0, sizeof(float) * 3 * N, c->stream));
     int rc;
     for (int n = 0; n < nsteps; n++) {
-        if (n % every == 0 && (rc = save_state(c, rv.ckpt + (size_t)(n / every) * 3 * v3)) != OC_OK)
-            return rc;
+        if (c->roll.keeps(n) && (rc = save_state(c, c->roll.state(N, n))) != OC_OK) return rc;
         if ((rc = one_step(c, s)) != OC_OK) return rc;
     }
-    if ((rc = save_state(c, rv.ckpt + (size_t)nseg * 3 * v3)) != OC_OK) return rc;
-    c->roll_steps = nsteps;
-    c->roll_every = every;
-    c->roll_valid = true;
+    if ((rc = save_state(c, c->roll.state(N, nsteps))) != OC_OK) return rc;
+    c->roll.valid = c->roll.same = true;
     c->assembled = false;
     return OC_OK;
 }
@@ -860,11 +831,11 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
                               float* grad_x0, float* grad_v0) {
     if (!c) return fail(OC_ERR_INVALID_ARGUMENT, "cloth is NULL");
     if (!grad_x) return fail(OC_ERR_INVALID_ARGUMENT, "grad_x is NULL");
-    if (!c->roll_valid) return fail(OC_ERR_INVALID_ARGUMENT, "no rollout_forward to differentiate");
-    const int nsteps = c->roll_steps, every = c->roll_every;
-    const int nseg = (nsteps + every - 1) / every;
-    const size_t v3 = 3 * (size_t)c->dc.N;
-    RolloutViews rv = rollout_views(c, nseg, every);
+    if (!c->roll.valid) return fail(OC_ERR_INVALID_ARGUMENT, "no rollout_forward to differentiate");
+    const oc::RolloutStore& roll = c->roll;
+    const int nsteps = roll.steps, every = roll.every;
+    const size_t N = (size_t)c->dc.N, kf = oc::kept_floats(N);
+    RolloutViews rv = rollout_views(c);
     float* mu = rv.vec[0];
     float* gx[2] = {rv.vec[7], rv.vec[8]};
     float* gv[2] = {rv.vec[9], rv.vec[10]};
@@ -875,22 +846,25 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
     oc::StepScalars s_cold = s;
     s_cold.warm = 0;
     int cur = 0;
-    for (int seg = nseg - 1; seg >= 0; seg--) {
-        const int n0 = seg * every, n1 = std::min(n0 + every, nsteps);
-        if ((rc = load_state(c, rv.ckpt + (size_t)seg * 3 * v3)) != OC_OK) return rc;
-        for (int n = n0; n < n1; n++) {
-            float* slot = rv.seg + (size_t)(n - n0) * 3 * v3;
-            const size_t b = sizeof(float) * v3;
+    const bool again = roll.recompute();  // a segment's states, from its checkpoint
+    for (int n0 = (nsteps - 1) / every * every; n0 >= 0; n0 -= every) {
+        const int n1 = std::min(n0 + every, nsteps);
+        if (again && (rc = load_state(c, roll.state(N, n0))) != OC_OK) return rc;
+        for (int n = n0; again && n < n1; n++) {
+            float* slot = roll.segment(N, n - n0);
+            const size_t b = sizeof(float) * 3 * N;
             OC_HIP(hipMemcpyAsync(slot, c->dc.x, b, hipMemcpyDeviceToDevice, c->stream));
-            OC_HIP(hipMemcpyAsync(slot + v3, c->dc.v, b, hipMemcpyDeviceToDevice, c->stream));
+            OC_HIP(hipMemcpyAsync(slot + kf, c->dc.v, b, hipMemcpyDeviceToDevice, c->stream));
             if ((rc = one_step(c, s)) != OC_OK) return rc;
-            OC_HIP(hipMemcpyAsync(slot + 2 * v3, c->dc.dv, b, hipMemcpyDeviceToDevice, c->stream));
+            OC_HIP(hipMemcpyAsync(slot + 2 * kf, c->dc.dv, b, hipMemcpyDeviceToDevice, c->stream));
         }
         for (int n = n1 - 1; n >= n0; n--) {
-            float* slot = rv.seg + (size_t)(n - n0) * 3 * v3;
+            // the state before step n, and the step's solution
+            float* slot = again ? roll.segment(N, n - n0) : roll.state(N, n);
+            float* sol = (again ? slot : roll.state(N, n + 1)) + 2 * kf;
             oc::DevCloth ca = c->dc;  // adjoint solve view: own CG vectors
             ca.x = slot;
-            ca.v = slot + v3;
+            ca.v = slot + kf;
             ca.dv = mu;
             ca.r = rv.vec[1];
             ca.d0 = rv.vec[2];
@@ -910,13 +884,13 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
             OC_HIP(oc::launch_cg(ca, s, c->stream));
             oc::DevCloth cg = c->dc;  // pre-step state and the step's solution
             cg.x = slot;
-            cg.v = slot + v3;
-            cg.dv = slot + 2 * v3;
+            cg.v = slot + kf;
+            cg.dv = sol;
             OC_HIP(oc::launch_adj_gather(cg, s, ab, c->stream));
             cur = 1 - cur;
         }
     }
-    if ((rc = load_state(c, rv.ckpt + (size_t)nseg * 3 * v3)) != OC_OK) return rc;
+    if ((rc = load_state(c, roll.state(N, nsteps))) != OC_OK) return rc;
     if (grad_ks) {
         OC_HIP(hipMemcpyAsync(grad_ks, rv.gks, sizeof(float) * c->topo.S, hipMemcpyDeviceToHost,
                               c->stream));

@@ -43,10 +43,7 @@ struct oc_batch_s {
     int grid = 0;
     oc::DevBatch dc{};
     // differentiable rollouts
-    void* adj_arena = nullptr;
-    size_t adj_bytes = 0;
-    int roll_steps = 0, roll_every = 0;
-    bool roll_valid = false;
+    oc::RolloutStore roll;
     // spring-once batched assembly (OPENCLOTH_ASSEMBLY=once) where the
     // schedule's LDS fits; off by default: on the 4096-cloth workload it ran
     // 9.30 ms per step against 8.45 ms for the per-end stencil form
@@ -170,6 +167,7 @@ int apply_schedule(oc_batch_s* b) {
     b->dc.asm_once = once ? 1 : 0;
     b->dc.lds_floats = once ? lds_floats : 0;
     b->grid = grid;
+    b->roll.same = false;  // (the order of the sums follows the schedule)
     b->graph_dirty = true;
     return OC_OK;
 }
@@ -306,9 +304,10 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
     const size_t slotc = align_up(sizeof(float) * 3 * (size_t)std::max(wa, 1) * N);
     const size_t pin = align_up(N);
     const size_t per = align_up(sizeof(int) * n_cloths);
+    const size_t row = align_up(sizeof(int) * N);
     const size_t amask = align_up(sizeof(uint32_t) * (st_asm ? N : 1));
     const size_t cst = align_up(sizeof(float) * 3 * oc::kOwned * (st_asm ? N : 1));
-    const size_t total = 8 * vec + blocks + as + am + pm + pk + 3 * sp + slotc + pin + 6 * per + amask + cst + 256;
+    const size_t total = 8 * vec + blocks + as + am + pm + pk + 3 * sp + slotc + pin + 6 * per + amask + cst + row + 256;
     if (hipMalloc(&b->arena, total) != hipSuccess) {
         delete b;
         return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(total) + " bytes failed");
@@ -350,6 +349,7 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
     d.inst_status = (int*)take(per);
     d.inst_sticky = (int*)take(per);
     d.queue = (int*)take(256);
+    d.row = (const int*)take(row);
     d.asm_mask = (const uint32_t*)take(amask);
     d.stencil_asm = st_asm ? 1 : 0;
     d.cst = (float*)take(cst);
@@ -406,13 +406,15 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
         std::vector<uint8_t> pins(N, 0);
         if (pinned)
             for (size_t i = 0; i < N; i++) pins[i] = pinned[i] ? 1 : 0;
-        std::vector<int> nxv(b->nx), nv(b->nverts);
+        std::vector<int> nxv(b->nx), nv(b->nverts), row(N);
+        for (int c = 0; c < n_cloths; c++) std::fill_n(row.begin() + b->voff[c], b->nverts[c], b->nx[c]);
         if (hipMemcpy((void*)d.L0, L0.data(), S * 4, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.ks, ks.data(), S * 4, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.kd, kd.data(), S * 4, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.pin, pins.data(), N, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.inst_voff, b->voff.data(), sizeof(int) * n_cloths, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.inst_nx, nxv.data(), sizeof(int) * n_cloths, hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy((void*)d.row, row.data(), sizeof(int) * N, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy((void*)d.inst_n, nv.data(), sizeof(int) * n_cloths, hipMemcpyHostToDevice) != hipSuccess)
             return fail_free(OC_ERR_DEVICE, "upload failed");
         if (oc::launch_batch_slot_constants(d, 0, 3, nullptr) != hipSuccess ||
@@ -443,7 +445,7 @@ int oc_batch_destroy(oc_batch b) {
     if (b->capture_stream) (void)hipStreamDestroy(b->capture_stream);
     if (b->sched_buf) (void)hipFree(b->sched_buf);
     if (b->arena) (void)hipFree(b->arena);
-    if (b->adj_arena) (void)hipFree(b->adj_arena);
+    if (b->roll.arena) (void)hipFree(b->roll.arena);
     delete b;
     return OC_OK;
 }
@@ -459,6 +461,7 @@ int oc_batch_set_params(oc_batch b, const oc_params* p) {
     int rc = check_params(p);
     if (rc != OC_OK) return rc;
     b->prm = *p;
+    b->roll.same = false;
     b->graph_dirty = true;
     return OC_OK;
 }
@@ -614,7 +617,7 @@ int oc_batch_set_spring_stiffness(oc_batch b, const float* ks) {
     OC_HIP(oc::launch_batch_slot_constants(b->dc, 1, 1, b->stream));
     OC_HIP(oc::launch_batch_owner_constants(b->dc, b->stream));
     OC_HIP(hipStreamSynchronize(b->stream));
-    b->roll_valid = false;
+    b->roll.valid = false;
     return OC_OK;
 }
 
@@ -629,11 +632,8 @@ int oc_batch_get_spring_stiffness(oc_batch b, float* ks) {
 
 namespace {
 
-// Rollout arena: checkpoints [(nseg+1) x (x,v,dv)], one segment of pre-step
-// states and solutions [every x (x,v,dv)], mu, gvt, gx[2], gv[2], gks.
+// The backward pass' vectors, behind the rollout's states.
 struct BatchRollout {
-    float* ckpt;
-    float* seg;
     float* mu;
     float* gvt;
     float* gx[2];
@@ -641,41 +641,34 @@ struct BatchRollout {
     float* gks;
 };
 
-BatchRollout batch_rollout_views(oc_batch_s* b, int nseg, int every) {
-    const size_t v3 = 3 * (size_t)b->Ntot;
+BatchRollout batch_rollout_views(oc_batch_s* b) {
+    const size_t N = (size_t)b->Ntot, kf = oc::kept_floats(N);
     BatchRollout r;
-    float* p = (float*)b->adj_arena;
-    r.ckpt = p;
-    p += (size_t)(nseg + 1) * 3 * v3;
-    r.seg = p;
-    p += (size_t)every * 3 * v3;
+    float* p = b->roll.rest(N);
     r.mu = p;
-    p += v3;
+    p += kf;
     r.gvt = p;
-    p += v3;
+    p += kf;
     for (int k = 0; k < 2; k++) {
         r.gx[k] = p;
-        p += v3;
+        p += kf;
         r.gv[k] = p;
-        p += v3;
+        p += kf;
     }
     r.gks = p;
     return r;
 }
 
-int batch_copy3(oc_batch_s* b, float* dst, const float* x, const float* v, const float* dv) {
-    const size_t n = sizeof(float) * 3 * (size_t)b->Ntot;
-    OC_HIP(hipMemcpyAsync(dst, x, n, hipMemcpyDeviceToDevice, b->stream));
-    OC_HIP(hipMemcpyAsync((char*)dst + n, v, n, hipMemcpyDeviceToDevice, b->stream));
-    OC_HIP(hipMemcpyAsync((char*)dst + 2 * n, dv, n, hipMemcpyDeviceToDevice, b->stream));
+int batch_keep(oc_batch_s* b, float* dst) {
+    OC_HIP(oc::launch_keep_state(b->dc.x, b->dc.v, b->dc.dv, dst, oc::kept_floats((size_t)b->Ntot), b->stream));
     return OC_OK;
 }
 
 int batch_restore(oc_batch_s* b, const float* src) {
-    const size_t n = sizeof(float) * 3 * (size_t)b->Ntot;
+    const size_t n = sizeof(float) * 3 * (size_t)b->Ntot, kf = oc::kept_floats((size_t)b->Ntot);
     OC_HIP(hipMemcpyAsync(b->dc.x, src, n, hipMemcpyDeviceToDevice, b->stream));
-    OC_HIP(hipMemcpyAsync(b->dc.v, (const char*)src + n, n, hipMemcpyDeviceToDevice, b->stream));
-    OC_HIP(hipMemcpyAsync(b->dc.dv, (const char*)src + 2 * n, n, hipMemcpyDeviceToDevice, b->stream));
+    OC_HIP(hipMemcpyAsync(b->dc.v, src + kf, n, hipMemcpyDeviceToDevice, b->stream));
+    OC_HIP(hipMemcpyAsync(b->dc.dv, src + 2 * kf, n, hipMemcpyDeviceToDevice, b->stream));
     return OC_OK;
 }
 
@@ -687,38 +680,20 @@ int oc_batch_rollout_forward(oc_batch b, int32_t nsteps, int32_t every) {
     if (!b) return set_error(OC_ERR_INVALID_ARGUMENT, "batch is NULL");
     if (nsteps < 1 || every < 1)
         return set_error(OC_ERR_INVALID_ARGUMENT, "nsteps and checkpoint_every must be >= 1");
-    b->roll_valid = false;  // until this rollout has completed
-    every = std::min(every, nsteps);
-    const int nseg = (nsteps + every - 1) / every;
-    const size_t v3 = 3 * (size_t)b->Ntot;
-    const size_t need = sizeof(float) * ((size_t)(nseg + 1) * 3 * v3 + (size_t)every * 3 * v3 +
-                                         6 * v3 + (size_t)std::max(b->Stot, 1));
-    if (need > b->adj_bytes) {
-        if (b->adj_arena) {
-            OC_HIP(hipStreamSynchronize(b->stream));
-            OC_HIP(hipFree(b->adj_arena));
-            b->adj_arena = nullptr;
-            b->adj_bytes = 0;
-        }
-        if (hipMalloc(&b->adj_arena, need) != hipSuccess)
-            return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc of rollout checkpoints failed");
-        b->adj_bytes = need;
-    }
-    BatchRollout rv = batch_rollout_views(b, nseg, every);
+    b->roll.valid = false;  // until this rollout has completed
+    const size_t N = (size_t)b->Ntot;
+    const hipError_t re = b->roll.reserve(N, nsteps, every, 6 * oc::kept_floats(N) + std::max(b->Stot, 1), b->stream);
+    if (re == hipErrorOutOfMemory) return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc of rollout checkpoints failed");
+    OC_HIP(re);
     int rc = ensure_graph(b);
     if (rc != OC_OK) return rc;
-    OC_HIP(hipMemsetAsync(b->dc.dv, 0, sizeof(float) * v3, b->stream));
+    OC_HIP(hipMemsetAsync(b->dc.dv, 0, sizeof(float) * 3 * N, b->stream));
     for (int n = 0; n < nsteps; n++) {
-        if (n % every == 0 &&
-            (rc = batch_copy3(b, rv.ckpt + (size_t)(n / every) * 3 * v3, b->dc.x, b->dc.v, b->dc.dv)) != OC_OK)
-            return rc;
+        if (b->roll.keeps(n) && (rc = batch_keep(b, b->roll.state(N, n))) != OC_OK) return rc;
         OC_HIP(hipGraphLaunch(b->graph, b->stream));
     }
-    if ((rc = batch_copy3(b, rv.ckpt + (size_t)nseg * 3 * v3, b->dc.x, b->dc.v, b->dc.dv)) != OC_OK)
-        return rc;
-    b->roll_steps = nsteps;
-    b->roll_every = every;
-    b->roll_valid = true;
+    if ((rc = batch_keep(b, b->roll.state(N, nsteps))) != OC_OK) return rc;
+    b->roll.valid = b->roll.same = true;
     return OC_OK;
 }
 
@@ -726,50 +701,53 @@ int oc_batch_rollout_backward(oc_batch b, const float* grad_x, const float* grad
                               float* grad_x0, float* grad_v0) {
     if (!b) return set_error(OC_ERR_INVALID_ARGUMENT, "batch is NULL");
     if (!grad_x) return set_error(OC_ERR_INVALID_ARGUMENT, "grad_x is NULL");
-    if (!b->roll_valid) return set_error(OC_ERR_INVALID_ARGUMENT, "no rollout_forward to differentiate");
-    const int nsteps = b->roll_steps, every = b->roll_every;
-    const int nseg = (nsteps + every - 1) / every;
-    const size_t v3 = 3 * (size_t)b->Ntot;
-    BatchRollout rv = batch_rollout_views(b, nseg, every);
+    if (!b->roll.valid) return set_error(OC_ERR_INVALID_ARGUMENT, "no rollout_forward to differentiate");
+    const oc::RolloutStore& roll = b->roll;
+    const int nsteps = roll.steps, every = roll.every;
+    const size_t N = (size_t)b->Ntot, kf = oc::kept_floats(N);
+    BatchRollout rv = batch_rollout_views(b);
     int rc;
     if ((rc = ensure_graph(b)) != OC_OK) return rc;
-    const size_t N = (size_t)b->Ntot;
     OC_HIP(b->io.write({{rv.gx[0], N, const_cast<float*>(grad_x)}, {rv.gv[0], N, const_cast<float*>(grad_v)}}, b->stream));
     OC_HIP(hipMemsetAsync(rv.gks, 0, sizeof(float) * std::max(b->Stot, 1), b->stream));
     oc::StepScalars s = batch_scalars(b);
     s.warm = 0;  // the adjoint assembly must not read or keep a warm start
     int cur = 0;
-    for (int seg = nseg - 1; seg >= 0; seg--) {
-        const int n0 = seg * every, n1 = std::min(n0 + every, nsteps);
-        if ((rc = batch_restore(b, rv.ckpt + (size_t)seg * 3 * v3)) != OC_OK) return rc;
-        for (int n = n0; n < n1; n++) {
-            float* slot = rv.seg + (size_t)(n - n0) * 3 * v3;
-            const size_t bytes = sizeof(float) * v3;
+    const bool again = roll.recompute();  // a segment's states, from its checkpoint
+    for (int n0 = (nsteps - 1) / every * every; n0 >= 0; n0 -= every) {
+        const int n1 = std::min(n0 + every, nsteps);
+        if (again && (rc = batch_restore(b, roll.state(N, n0))) != OC_OK) return rc;
+        for (int n = n0; again && n < n1; n++) {
+            float* slot = roll.segment(N, n - n0);
+            const size_t bytes = sizeof(float) * 3 * N;
             OC_HIP(hipMemcpyAsync(slot, b->dc.x, bytes, hipMemcpyDeviceToDevice, b->stream));
-            OC_HIP(hipMemcpyAsync(slot + v3, b->dc.v, bytes, hipMemcpyDeviceToDevice, b->stream));
+            OC_HIP(hipMemcpyAsync(slot + kf, b->dc.v, bytes, hipMemcpyDeviceToDevice, b->stream));
             OC_HIP(hipGraphLaunch(b->graph, b->stream));
-            OC_HIP(hipMemcpyAsync(slot + 2 * v3, b->dc.dv, bytes, hipMemcpyDeviceToDevice, b->stream));
+            OC_HIP(hipMemcpyAsync(slot + 2 * kf, b->dc.dv, bytes, hipMemcpyDeviceToDevice, b->stream));
         }
         for (int n = n1 - 1; n >= n0; n--) {
-            float* slot = rv.seg + (size_t)(n - n0) * 3 * v3;
+            // the state before step n, and the step's solution
+            float* slot = again ? roll.segment(N, n - n0) : roll.state(N, n);
+            float* sol = (again ? slot : roll.state(N, n + 1)) + 2 * kf;
             oc::DevBatch ca = b->dc;
             ca.x = slot;
-            ca.v = slot + v3;
+            ca.v = slot + kf;
             ca.dv = rv.mu;
             oc::BatchAdjBufs ab;
             ab.gx_out = rv.gx[cur];
             ab.gv_out = rv.gv[cur];
             ab.gvt = rv.gvt;
-            ab.dvsol = slot + 2 * v3;
+            ab.dvsol = sol;
             ab.gx_in = rv.gx[1 - cur];
             ab.gv_in = rv.gv[1 - cur];
             ab.gks = rv.gks;
             OC_HIP(oc::launch_batch_reset(b->dc, b->stream));
             OC_HIP(oc::launch_batch_adjoint(ca, s, ab, b->sched.block_threads, b->grid, b->stream));
+            OC_HIP(oc::launch_batch_gather(ca, s, ab, b->stream));
             cur = 1 - cur;
         }
     }
-    if ((rc = batch_restore(b, rv.ckpt + (size_t)nseg * 3 * v3)) != OC_OK) return rc;
+    if ((rc = batch_restore(b, roll.state(N, nsteps))) != OC_OK) return rc;
     if (grad_ks) {
         OC_HIP(hipMemcpyAsync(grad_ks, rv.gks, sizeof(float) * b->Stot, hipMemcpyDeviceToHost, b->stream));
         OC_HIP(hipStreamSynchronize(b->stream));

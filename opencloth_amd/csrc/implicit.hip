@@ -1723,46 +1723,40 @@ __global__ __launch_bounds__(TX* TY) void k_adj_init(DevCloth c, StepScalars s, 
 }
 
 // gx_in = gx' + dJ/dx, gv_in = gvt + dJ/dv, gks += dJ/dks (added by each
-// spring's p1).  c.x, c.v: pre-step state; c.dv: the step's solution.
-template <int TX, int TY>
-__global__ __launch_bounds__(TX* TY) void k_adj_gather(DevCloth c, StepScalars s, AdjointBufs a) {
-    const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
-    const int tile = tile_of_block(blockIdx.x, c.nt);
-    const int bx = tile % c.ntx, by = tile / c.ntx;
-    const int gi = bx * TX + lx, gj = by * TY + ly;
-    if (gi >= c.nx || gj >= c.ny) return;
-    const int N = c.N, i = gj * c.nx + gi;
-    const V3 xi = ld3(c.x, N, i), vi = ld3(c.v, N, i), mi = ld3(a.mu, N, i), pi = ld3(c.dv, N, i);
-    const V3 wi = add3(vi, pi);
+// spring's p1).  c.x, c.v: pre-step state; c.dv: the step's solution.  One
+// wave per block, so that a cloth of 128x128 already has a wave on every CU:
+// 15 us there, 43 when the slots, neighbours and constants of a spring were
+// loaded one after the other by 512-thread blocks.  Bound by the issue of a
+// wave's twelve springs, about 400 instructions each.
+constexpr int kGatherThreads = 64;
+__global__ __launch_bounds__(kGatherThreads) void k_adj_gather(DevCloth c, StepScalars s, AdjointBufs a) {
+    const int N = c.N, i = blockIdx.x * kGatherThreads + threadIdx.x;
+    if (i >= N) return;
     V3 gx = ld3(a.gx_out, N, i), gv = ld3(a.gvt, N, i);
+    const V3 mi = ld3(a.mu, N, i);
     if (s.damp != 0.0f && !c.pin[i])  // the damping force c v_i: dJ/dv_i += h c mu_i
         gv = {gv.x + s.h * (s.damp * mi.x), gv.y + s.h * (s.damp * mi.y), gv.z + s.h * (s.damp * mi.z)};
-    for (int k = 0; k < c.wa; k++) {
-        const int sp = c.ainc_s[k * N + i];
-        if (sp < 0) break;
-        const uint16_t m = c.ainc_m[k * N + i];
-        const int j = i + slot_dj(m) * c.nx + slot_di(m);
-        const V3 xj = ld3(c.x, N, j), vj = ld3(c.v, N, j), mj = ld3(a.mu, N, j), pj = ld3(c.dv, N, j);
-        const V3 wj = add3(vj, pj);
-        const bool second = (m >> 8) & 1u;
-        float ge[3], gvv[3], gk;
-        if (second)
-            spring_adjoint(xj, xi, vj, vi, mj, mi, wj, wi, pj, pi, c.L0[sp], c.ks[sp], c.kd[sp], s.h,
-                           s.hh, ge, gvv, gk);
-        else
-            spring_adjoint(xi, xj, vi, vj, mi, mj, wi, wj, pi, pj, c.L0[sp], c.ks[sp], c.kd[sp], s.h,
-                           s.hh, ge, gvv, gk);
-        if (second) {
-            gx = {gx.x - ge[0], gx.y - ge[1], gx.z - ge[2]};
-            gv = {gv.x - gvv[0], gv.y - gvv[1], gv.z - gvv[2]};
-        } else {
-            gx = {gx.x + ge[0], gx.y + ge[1], gx.z + ge[2]};
-            gv = {gv.x + gvv[0], gv.y + gvv[1], gv.z + gvv[2]};
-            a.gks[sp] = a.gks[sp] + gk;
-        }
-    }
+    const AdjGatherIn in = {c.x, c.v, a.mu, c.dv, c.ainc_s, c.ainc_m, N, c.wa};
+    adj_gather_springs(in, i, c.nx, s.h, s.hh,
+                       [&](int, int sp, float& L0, float& ks, float& kd) {
+                           L0 = c.L0[sp];
+                           ks = c.ks[sp];
+                           kd = c.kd[sp];
+                       },
+                       a.gks, gx, gv);
     st3(a.gx_in, N, i, gx);
     st3(a.gv_in, N, i, gv);
+}
+
+// Three vectors of n quads of floats into dst, one after the other.
+__global__ __launch_bounds__(256) void k_keep_state(const float4* x, const float4* v, const float4* dv, float4* dst,
+                                                    unsigned n) {
+    const unsigned t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    const float4 a = x[t], b = v[t], c = dv[t];
+    dst[t] = a;
+    dst[n + t] = b;
+    dst[2 * (size_t)n + t] = c;
 }
 
 thread_local LaunchProfile* t_prof = nullptr;
@@ -1795,8 +1789,18 @@ hipError_t launch_adj_init(const DevCloth& c, const StepScalars& s, const Adjoin
 
 hipError_t launch_adj_gather(const DevCloth& c, const StepScalars& s, const AdjointBufs& a,
                              hipStream_t st) {
-    hipLaunchKernelGGL((k_adj_gather<kTileX, kTileY>), dim3(c.nt), dim3(kTileX * kTileY), 0, st, c,
+    hipLaunchKernelGGL(k_adj_gather, dim3((c.N + kGatherThreads - 1) / kGatherThreads), dim3(kGatherThreads), 0, st, c,
                        s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_keep_state(const float* x, const float* v, const float* dv, float* dst, size_t floats,
+                             hipStream_t st) {
+    if (floats % 4 != 0 || floats > (size_t)UINT32_MAX) return hipErrorInvalidValue;
+    const unsigned n = (unsigned)(floats / 4);
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_keep_state, dim3((n + 255) / 256), dim3(256), 0, st, (const float4*)x, (const float4*)v,
+                       (const float4*)dv, (float4*)dst, n);
     return hipGetLastError();
 }
 

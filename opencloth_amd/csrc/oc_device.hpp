@@ -250,5 +250,79 @@ __device__ inline void spring_adjoint(V3 xa, V3 xb, V3 va, V3 vb, V3 ua, V3 ub, 
     gk = h * (ue * il) * (-(l - L0)) + hh * ((L0 * il - 1.0f) * uw - L0 * ue * we * il3);
 }
 
+// What the adjoint gather reads: pre-step x, v, the adjoint solve mu and the
+// step's solution p (planes of stride N), the assembly slots (slot-major).
+struct AdjGatherIn {
+    const float* x;
+    const float* v;
+    const float* mu;
+    const float* p;
+    const int32_t* ainc_s;
+    const uint16_t* ainc_m;
+    int N, wa;
+};
+
+// Adjoint gather of vertex i: the spring terms of dJ/dx into gx, of dJ/dv
+// into gv and, at a spring's first end, dJ/dks into gks.  Every spring is
+// evaluated from this vertex's side, which is bitwise the negated terms of
+// the other side, so it is always added.  constants(k, sp, L0, ks, kd) reads
+// a spring's.  What bounds it is the chain slot -> neighbour and constants ->
+// terms, so slots are read two springs ahead, neighbours and constants one,
+// by unconditional loads (of vertex i itself past the last slot).
+template <class Constants>
+__device__ __forceinline__ void adj_gather_springs(const AdjGatherIn& c, int i, int nx, float h, float hh,
+                                                   const Constants& constants, float* gks, V3& gx, V3& gv) {
+    if (c.wa < 1) return;
+    const int N = c.N;
+    struct Slot {
+        int sp;
+        uint16_t m;
+    };
+    struct Spring {
+        int sp;
+        bool second;
+        V3 x, v, mu, p;
+        float L0, ks, kd, g;
+    };
+    auto slot = [&](int k) {
+        const size_t o = (size_t)min(k, c.wa - 1) * N + i;
+        Slot r = {c.ainc_s[o], c.ainc_m[o]};
+        if (k >= c.wa) r.sp = -1;
+        return r;
+    };
+    auto fetch = [&](int k, Slot q) {
+        const bool have = q.sp >= 0;
+        Spring r;
+        r.sp = q.sp;
+        r.second = (q.m >> 8) & 1u;
+        const int j = have ? i + slot_dj(q.m) * nx + slot_di(q.m) : i, sp = have ? q.sp : 0;
+        r.x = ld3(c.x, N, j);
+        r.v = ld3(c.v, N, j);
+        r.mu = ld3(c.mu, N, j);
+        r.p = ld3(c.p, N, j);
+        constants(min(k, c.wa - 1), sp, r.L0, r.ks, r.kd);
+        r.g = gks[sp];
+        return r;
+    };
+    const V3 xi = ld3(c.x, N, i), vi = ld3(c.v, N, i), mi = ld3(c.mu, N, i), pi = ld3(c.p, N, i);
+    const V3 wi = add3(vi, pi);
+    Slot ahead = slot(1);
+    Spring nxt = fetch(0, slot(0));
+#pragma unroll 1
+    for (int k = 0; k < c.wa; k++) {
+        const Spring in = nxt;
+        if (in.sp < 0) break;
+        const Slot q = ahead;
+        ahead = slot(k + 2);
+        nxt = fetch(k + 1, q);
+        float ge[3], gvv[3], gk;
+        spring_adjoint(xi, in.x, vi, in.v, mi, in.mu, wi, add3(in.v, in.p), pi, in.p, in.L0, in.ks, in.kd, h, hh, ge,
+                       gvv, gk);
+        gx = {gx.x + ge[0], gx.y + ge[1], gx.z + ge[2]};
+        gv = {gv.x + gvv[0], gv.y + gvv[1], gv.z + gvv[2]};
+        if (!in.second) gks[in.sp] = in.g + gk;
+    }
+}
+
 }  // namespace dev
 }  // namespace oc

@@ -327,6 +327,39 @@ hipError_t launch_adj_init(const DevCloth& c, const StepScalars& s, const Adjoin
                            hipStream_t st);
 hipError_t launch_adj_gather(const DevCloth& c, const StepScalars& s, const AdjointBufs& a,
                              hipStream_t st);
+// x, v and dv (16-byte aligned, `floats` of each, a multiple of 4) to dst.
+hipError_t launch_keep_state(const float* x, const float* v, const float* dv, float* dst, size_t floats,
+                             hipStream_t st);
+
+// The states a rollout keeps for its backward pass (rollout_store.cpp): all of
+// them when they fit a share of the device's free memory, else the caller's
+// checkpoints.  A state is x, v and dv before a step (dv: the previous step's
+// solution), each padded to kept_floats(n) floats.  The arena holds the kept
+// states, a segment of `every` states to recompute between checkpoints, and
+// what else the backward pass needs.
+constexpr size_t kept_floats(size_t n) { return (3 * n + 63) / 64 * 64; }
+struct RolloutStore {
+    void* arena = nullptr;  // freed by the handle
+    size_t bytes = 0;
+    int steps = 0, every = 0;
+    bool valid = false;  // there is a rollout to differentiate
+    bool all = false;    // every state is kept
+    bool same = false;   // the step's parameters are still the rollout's
+    // Room for a rollout of n vertices with `tail` more floats; sets steps,
+    // every and all.
+    hipError_t reserve(size_t n, int nsteps, int checkpoint_every, size_t tail, hipStream_t st);
+    int states() const { return all ? steps + 1 : (steps + every - 1) / every + 1; }
+    bool keeps(int step) const { return all || step % every == 0 || step == steps; }
+    bool recompute() const { return !(all && same); }
+    float* state(size_t n, int step) const {  // of a kept step
+        return slot(n, all ? step : step == steps ? states() - 1 : step / every);
+    }
+    float* segment(size_t n, int k) const { return slot(n, states() + k); }
+    float* rest(size_t n) const { return slot(n, states() + every); }
+
+  private:
+    float* slot(size_t n, int k) const { return (float*)arena + 3 * kept_floats(n) * (size_t)k; }
+};
 
 // Post-step passes on an implicit cloth (post.hip).
 hipError_t launch_ellipsoid(float* x, float* w, int N, const oc_ellipsoid& e, int mode,
@@ -559,6 +592,7 @@ struct DevBatch {
     // the constants again per assembly slot, coalesced: plane q (0 L0, 1 ks,
     // 2 kd) of slot k of vertex i at slot_c[(q * wa + k) * Ntot + i]
     float* slot_c;
+    const int* row;  // per vertex, its cloth's row length
     const int* inst_voff;
     const int* inst_nx;
     const int* inst_n;
@@ -625,6 +659,8 @@ struct BatchAdjBufs {
 
 hipError_t launch_batch_adjoint(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a,
                                 int block_threads, int grid, hipStream_t st);
+// dJ/dx, dJ/dv and dJ/dks of the step whose adjoint solve is in c.dv.
+hipError_t launch_batch_gather(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a, hipStream_t st);
 hipError_t launch_batch_reset(const DevBatch& c, hipStream_t st);
 // Fill slot_c planes q0 .. q0+nq-1 from L0/ks/kd through the slot tables.
 hipError_t launch_batch_slot_constants(const DevBatch& c, int q0, int nq, hipStream_t st);

@@ -1,0 +1,60 @@
+// Device memory of differentiable rollouts.
+#include <algorithm>
+
+#include "oc_internal.hpp"
+
+namespace oc {
+
+// Keeping every state saves the backward pass the second run of every step
+// (a third of a 128x128 rollout's time); it takes 36 bytes per vertex and
+// step.  kShare of the free memory, and at most kMost, bounds what a handle
+// takes beyond the checkpoints that its caller asked for.
+constexpr size_t kShare = 8, kMost = size_t(8) << 30;
+
+hipError_t RolloutStore::reserve(size_t n, int nsteps, int checkpoint_every, size_t tail, hipStream_t st) {
+    steps = nsteps;
+    every = std::min(checkpoint_every, nsteps);
+    auto need = [&](bool with_all) {
+        all = with_all;
+        return sizeof(float) * (3 * kept_floats(n) * ((size_t)states() + every) + tail);
+    };
+    const size_t least = need(false);
+    size_t want = need(true);
+    if (want <= bytes) return hipSuccess;
+    bool fits = true;
+    if (least <= bytes) {  // only to grow: not while the stream's work is captured
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        fits = hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+    }
+    if (fits) {
+        size_t avail = 0, total = 0;
+        fits = hipMemGetInfo(&avail, &total) == hipSuccess && want <= std::min(avail / kShare, kMost);
+    }
+    if (!fits) want = need(false);
+    if (want <= bytes) return hipSuccess;
+    void* fresh = nullptr;
+    if (all && hipMalloc(&fresh, want) != hipSuccess) {
+        fresh = nullptr;
+        want = need(false);
+        if (want <= bytes) return hipSuccess;
+    }
+    if (arena) {
+        const hipError_t r = hipStreamSynchronize(st);
+        if (r != hipSuccess) {
+            if (fresh) (void)hipFree(fresh);
+            return r;
+        }
+        (void)hipFree(arena);
+        arena = nullptr;
+        bytes = 0;
+    }
+    if (!fresh) {
+        const hipError_t r = hipMalloc(&fresh, want);
+        if (r != hipSuccess) return r;
+    }
+    arena = fresh;
+    bytes = want;
+    return hipSuccess;
+}
+
+}  // namespace oc
