@@ -24,8 +24,8 @@ state resident in HBM.  Prints one JSON line:
                from the committed rocprofv3 summary
   config       the kernel split per step, and the same workload with the
                single-reduction CG
-  batch        4096 uneven cloths, 200 steps, one graph-replayed launch per
-               step, against one-cloth-per-launch forms; the roofline of the
+  batch        4096 uneven cloths, 200 steps, one graph replay (assembly and
+               solve launches) per step, against one-cloth-per-launch forms; the roofline of the
                launch after the timed steps
   batch_adjoint, adjoint
                batched (512 cloths, 60 steps) and single-cloth (128x128, 120
@@ -297,7 +297,8 @@ def bench_batch(steps: int, warmup: int, n_cloths: int = 4096, plain_steps: int 
     ms = e0.elapsed_ms(e1)
     # the roofline launch: one more step timed alone; its algorithmic bytes
     # come from its own CG iteration counts (the committed counters are of
-    # this launch: the batch leg's last k_batch_step dispatch)
+    # this step: the batch leg's last k_batch_assemble and k_batch_step
+    # dispatches)
     r0, r1 = Event(), Event()
     r0.record()
     b.step(1)

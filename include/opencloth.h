@@ -417,9 +417,9 @@ int oc_cloth_get_pairs(oc_cloth cloth, int32_t* a, int32_t* b);
 int oc_cloth_get_system(oc_cloth cloth, float* blocks, float* rhs);
 
 /* ---- batched cloths ---------------------------------------------------- */
-/* Many independent cloths of uneven sizes stepped together: one persistent
- * kernel launch per step runs assembly, filtered CG (per-cloth stopping
- * test, converged cloths masked out) and the update for every cloth.  No
+/* Many independent cloths of uneven sizes stepped together: per step one
+ * launch assembles every cloth and one persistent launch runs filtered CG
+ * (per-cloth stopping test, converged cloths masked out) and the update.  No
  * counterpart in the reference, whose demos each step one global cloth; each
  * cloth follows the same step as oc_cloth_step. */
 typedef struct oc_batch_s* oc_batch;
@@ -471,9 +471,9 @@ int oc_batch_sticky_status(oc_batch batch, int32_t* status);
 int oc_batch_set_spring_stiffness(oc_batch batch, const float* ks);
 int oc_batch_get_spring_stiffness(oc_batch batch, float* ks);
 /* Batched differentiable rollout: as oc_cloth_rollout_forward/backward for
- * every cloth at once; each step's adjoint is one persistent launch that
- * re-assembles, solves the adjoint system per cloth (masked CG) and gathers
- * the derivatives.  Arrays are all cloths' vertices/springs concatenated. */
+ * every cloth at once; each step's adjoint is three launches that re-assemble,
+ * solve the adjoint system per cloth (masked CG) and gather the
+ * derivatives.  Arrays are all cloths' vertices/springs concatenated. */
 int oc_batch_rollout_forward(oc_batch batch, int32_t nsteps, int32_t checkpoint_every);
 int oc_batch_rollout_backward(oc_batch batch, const float* grad_x, const float* grad_v,
                               float* grad_ks, float* grad_x0, float* grad_v0);

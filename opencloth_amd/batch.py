@@ -1,6 +1,6 @@
 """Batched cloths over the C ABI (oc_batch_*): many independent cloths of
-uneven sizes stepped by one persistent kernel launch per step, replayed from a
-captured HIP graph."""
+uneven sizes stepped by an assembly and a persistent solve launch per step,
+replayed from a captured HIP graph."""
 from __future__ import annotations
 
 import ctypes as C

@@ -1,10 +1,11 @@
 // Persistent batched implicit step (gfx950, wave64).
 //
-// One launch steps every cloth of a batch.  Workgroups pull work items (packs
-// of similar-sized cloths, largest first) from a queue; the threads of a
-// workgroup are split evenly over the pack's cloths and each cloth's
-// assembly, filtered CG and update run inside its workgroup, so no step needs
-// a grid-wide barrier.  Cloths that meet their stopping test are masked out
+// Two launches step every cloth of a batch: the assembly over all vertices,
+// and a persistent one in which workgroups pull work items (packs of
+// similar-sized cloths, largest first) from a queue; the threads of a
+// workgroup are split evenly over the pack's cloths and each cloth's filtered
+// CG and update run inside its workgroup, so no step needs a grid-wide
+// barrier.  Cloths that meet their stopping test are masked out
 // while the rest of the pack iterates.  The loop exits when the queue is
 // drained, which every workgroup reaches.
 //
@@ -15,7 +16,12 @@
 // Reductions: thread t of a cloth's T threads sums vertices t, t+T, ... in
 // order, then the 64-lane wave tree, then the cloth's waves in order.  A
 // thread's first kResidentPerThread vertices keep their CG vectors (d, r, q
-// and the solution) in LDS through the solve; the rest stream from memory.
+// and the solution) in LDS through the solve, the next kInRegisters in
+// registers; the rest stream from memory.  An iteration over 3.1 M vertices
+// takes 190 us: 144 bytes of blocks per vertex and the vectors that stream,
+// about 3.5 TB/s.
+#include <algorithm>
+
 #include "oc_device.hpp"
 
 namespace oc {
@@ -48,18 +54,15 @@ __device__ inline float jacobi_inv(float dg) {
 
 // CG start of vertex i from its assembled sums: b = h (f + h K v),
 // r = S (b - A dv), the Jacobi entries and d = z = P^-1 r (z = r without the
-// preconditioner); returns r.z.  keep (a vertex whose CG state stays in
-// LDS): r, z and the solution's start go there, and r is not written to
-// memory (d is: the neighbours' SpMV reads it).
-__device__ inline float cg_start(const DevBatch& c, const StepScalars& s, int i, bool pinned, V3 acc, V3 kv,
-                                 V3 adv, V3 dg, V3 dvi, V3* keep) {
+// preconditioner).
+__device__ inline void cg_start(const DevBatch& c, const StepScalars& s, int i, bool pinned, V3 acc, V3 kv,
+                                 V3 adv, V3 dg) {
     const int N = c.Ntot;
     const float h = s.h;
     V3 b;
     b.x = pinned ? 0.0f : h * (acc.x + h * kv.x);
     b.y = pinned ? 0.0f : h * (acc.y + h * kv.y);
     b.z = pinned ? 0.0f : h * (acc.z + h * kv.z);
-    st3(c.b, N, i, b);
     const V3 r = pinned ? V3{0.0f, 0.0f, 0.0f} : sub3(b, adv);
     V3 z = r;
     if (s.flags & OC_FLAG_JACOBI) {
@@ -68,14 +71,7 @@ __device__ inline float cg_start(const DevBatch& c, const StepScalars& s, int i,
         z = {pv.x * r.x, pv.y * r.y, pv.z * r.z};
     }
     st3(c.d, N, i, z);
-    if (keep) {
-        keep[0] = r;
-        keep[1] = z;
-        keep[2] = dvi;
-    } else {
-        st3(c.r, N, i, r);
-    }
-    return dot3(r, z);
+    st3(c.r, N, i, r);
 }
 
 // Slot k of vertex i: spring id and meta, the other end's x, v (dv for a
@@ -110,9 +106,8 @@ __device__ inline BSpringIn fetch_bspring(const DevBatch& c, const StepScalars& 
 
 // Assembly of vertex i (global index) of a cloth with row length nx:
 // pair blocks it owns, rhs b, CG start r = S(b - A dv), d = z = P^-1 r (z = r
-// without the Jacobi preconditioner); returns r.z.
-__device__ inline float assemble_vertex(const DevBatch& c, const StepScalars& s, int i, int nx,
-                                       V3* keep = nullptr) {
+// without the Jacobi preconditioner).
+__device__ inline void assemble_vertex(const DevBatch& c, const StepScalars& s, int i, int nx) {
     const int N = c.Ntot;
     const float h = s.h, hh = s.hh;
     const bool pinned = c.pin[i] != 0;
@@ -156,7 +151,7 @@ __device__ inline float assemble_vertex(const DevBatch& c, const StepScalars& s,
             for (int q = 0; q < 6; q++) C[q] = 0.0f;
         }
     }
-    return cg_start(c, s, i, pinned, acc, kv, adv, dg, dvi, keep);
+    cg_start(c, s, i, pinned, acc, kv, adv, dg);
 }
 
 // Stencil form of assemble_vertex, for batches whose cloths all have the
@@ -193,8 +188,7 @@ __device__ inline StencilIn fetch_stencil(const DevBatch& c, const StepScalars& 
     return r;
 }
 
-__device__ inline float assemble_vertex_stencil(const DevBatch& c, const StepScalars& s, int i, int nx,
-                                               V3* keep = nullptr) {
+__device__ inline void assemble_vertex_stencil(const DevBatch& c, const StepScalars& s, int i, int nx) {
     const int N = c.Ntot;
     const float h = s.h, hh = s.hh;
     const bool pinned = c.pin[i] != 0;
@@ -245,7 +239,7 @@ __device__ inline float assemble_vertex_stencil(const DevBatch& c, const StepSca
         adv = add3(adv, symmv(C, sub3(in.dv, dvi)));
         dg = {dg.x - C[0], dg.y - C[1], dg.z - C[2]};
     }
-    return cg_start(c, s, i, pinned, acc, kv, adv, dg, dvi, keep);
+    cg_start(c, s, i, pinned, acc, kv, adv, dg);
 }
 
 // z = P^-1 r of vertex i (r itself without the Jacobi preconditioner).
@@ -334,7 +328,7 @@ __device__ inline float spmv_vertex(const DevBatch& c, const StepScalars& s, int
 // Adjoint start for vertex i: gvt = gv' + h gx', r = S gvt, d = P^-1 r (the
 // solution buffer, c.dv, was zeroed by the cold assembly); returns r.(P^-1 r).
 __device__ inline float adjoint_start_vertex(const DevBatch& c, const StepScalars& s,
-                                             const BatchAdjBufs& a, int i, V3* keep = nullptr) {
+                                             const BatchAdjBufs& a, int i) {
     const int N = c.Ntot;
     const V3 gx = ld3(a.gx_out, N, i), gv = ld3(a.gv_out, N, i);
     const V3 g = {gv.x + s.h * gx.x, gv.y + s.h * gx.y, gv.z + s.h * gx.z};
@@ -342,13 +336,7 @@ __device__ inline float adjoint_start_vertex(const DevBatch& c, const StepScalar
     const V3 r = c.pin[i] ? V3{0.0f, 0.0f, 0.0f} : g;
     const V3 z = precond(c, s, i, r);  // the preconditioner of the cold assembly
     st3(c.d, N, i, z);
-    if (keep) {  // as in cg_start; the solve starts from mu = 0
-        keep[0] = r;
-        keep[1] = z;
-        keep[2] = V3{0.0f, 0.0f, 0.0f};
-    } else {
-        st3(c.r, N, i, r);
-    }
+    st3(c.r, N, i, r);
     return dot3(r, z);
 }
 
@@ -497,7 +485,6 @@ __device__ float assemble_once(const DevBatch& c, const StepScalars& s, const Ba
             b.x = pinned ? 0.0f : h * (acc.x + h * kv.x);
             b.y = pinned ? 0.0f : h * (acc.y + h * kv.y);
             b.z = pinned ? 0.0f : h * (acc.z + h * kv.z);
-            st3(c.b, N, i, b);
             V3 r = pinned ? V3{0.0f, 0.0f, 0.0f} : sub3(b, adv);
             st3(c.r, N, i, r);
             float rr;
@@ -527,7 +514,7 @@ __device__ float assemble_once(const DevBatch& c, const StepScalars& s, const Ba
 template <int NT, bool ADJ, bool ONCE>
 __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s, BatchAdjBufs adj) {
     constexpr int NW = NT / 64;
-    constexpr int RV = ONCE ? 0 : kResidentPerThread;
+    constexpr int RV = ONCE ? 0 : kResidentPerThread, RG = ONCE ? 0 : kInRegisters, RM = RV + RG;
     __shared__ float ws[NW];
     __shared__ float sd[NW], sd_old[NW], sd0[NW], ssig[NW];
     __shared__ int sdone[NW], sit[NW], sst[NW];
@@ -569,6 +556,10 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
             rs[(3 * pl + 2) * RP + o] = v.z;
         };
 
+        struct {
+            V3 d, r, x, q;
+        } kept[RG + 1];  // the next RG vertices' (the last entry is not used)
+
         // ---- assembly and CG start
         float t = 0.0f;
         if constexpr (ONCE) {
@@ -582,23 +573,31 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
             t = assemble_once<NT, ADJ>(c, s, adj, dyn_lds, T, g, lt, act, voff, nx, Ni, Nmax,
                                        ring_floats(nxm));
         } else {
-            // the thread's first RV vertices keep their CG state in LDS
-            int u = 0;
-            for (int vv = lt; vv < Ni; vv += T, u++) {
-                V3 keep[3];
-                V3* const kp = u < RV ? keep : nullptr;
-                const float rr = c.stencil_asm ? assemble_vertex_stencil(c, s, voff + vv, nx, ADJ ? nullptr : kp)
-                                               : assemble_vertex(c, s, voff + vv, nx, ADJ ? nullptr : kp);
-                if constexpr (ADJ)
-                    t += adjoint_start_vertex(c, s, adj, voff + vv, kp);
-                else
-                    t += rr;
-                if (kp) {
-                    rst(0, u, keep[1]);
-                    rst(1, u, keep[0]);
-                    rst(2, u, keep[2]);
+            // the CG start as the assembly launch left it; the thread's first
+            // RV vertices' state moves to LDS
+#pragma unroll 1
+            for (int u = 0; u < RV; u++) {
+                const int vv = lt + u * T;
+                if (vv < Ni) {
+                    const int i = voff + vv;
+                    const V3 r = ld3(c.r, N, i), z = ld3(c.d, N, i), x = ld3(c.dv, N, i);
+                    rst(0, u, z);
+                    rst(1, u, r);
+                    rst(2, u, x);
+                    t += dot3(r, z);
                 }
             }
+#pragma unroll
+            for (int u = 0; u < RG; u++) {
+                const int vv = lt + (RV + u) * T;
+                if (vv < Ni) {
+                    const int i = voff + vv;
+                    kept[u] = {ld3(c.d, N, i), ld3(c.r, N, i), ld3(c.dv, N, i), V3{0.0f, 0.0f, 0.0f}};
+                    t += dot3(kept[u].r, kept[u].d);
+                }
+            }
+            for (int vv = lt + RM * T; vv < Ni; vv += T)
+                t += dot3(ld3(c.r, N, voff + vv), ld3(c.d, N, voff + vv));
         }
         float tot = seg_sum<NW>(t, T, ws);
         if (act && lt == 0) {
@@ -639,7 +638,17 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
                         st3(c.d, N, i, dn);
                     }
                 }
-                for (int vv = lt + RV * T; vv < Ni; vv += T) {
+#pragma unroll
+                for (int u = 0; u < RG; u++) {
+                    const int vv = lt + (RV + u) * T;
+                    if (vv < Ni) {
+                        const int i = (int)here(voff + vv);
+                        const V3 z = precond(c, s, i, kept[u].r), dp = kept[u].d;
+                        kept[u].d = {z.x + beta * dp.x, z.y + beta * dp.y, z.z + beta * dp.z};
+                        st3(c.d, N, i, kept[u].d);
+                    }
+                }
+                for (int vv = lt + RM * T; vv < Ni; vv += T) {
                     const int i = voff + vv;
                     V3 z = precond(c, s, i, ld3(c.r, N, i)), dp = ld3(c.d, N, i);
                     st3(c.d, N, i, V3{z.x + beta * dp.x, z.y + beta * dp.y, z.z + beta * dp.z});
@@ -657,7 +666,12 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
                         rst(3, u, q);
                     }
                 }
-                for (int vv = lt + RV * T; vv < Ni; vv += T) t += spmv_vertex(c, s, voff + vv, nx);
+#pragma unroll
+                for (int u = 0; u < RG; u++) {
+                    const int vv = lt + (RV + u) * T;
+                    if (vv < Ni) t += spmv_core(c, s, (int)here(voff + vv), nx, kept[u].q);
+                }
+                for (int vv = lt + RM * T; vv < Ni; vv += T) t += spmv_vertex(c, s, voff + vv, nx);
             }
             tot = seg_sum<NW>(t, T, ws);
             if (act && lt == 0) ssig[g] = tot;
@@ -693,7 +707,18 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
                         t += dot3(r, precond(c, s, i, r));
                     }
                 }
-                for (int vv = lt + RV * T; vv < Ni; vv += T) {
+#pragma unroll
+                for (int u = 0; u < RG; u++) {
+                    const int vv = lt + (RV + u) * T;
+                    if (vv < Ni) {
+                        const V3 d = kept[u].d, q = kept[u].q;
+                        V3 &x = kept[u].x, &r = kept[u].r;
+                        x = {x.x + alpha * d.x, x.y + alpha * d.y, x.z + alpha * d.z};
+                        r = {r.x - alpha * q.x, r.y - alpha * q.y, r.z - alpha * q.z};
+                        t += dot3(r, precond(c, s, (int)here(voff + vv), r));
+                    }
+                }
+                for (int vv = lt + RM * T; vv < Ni; vv += T) {
                     const int i = voff + vv;
                     V3 d = ld3(c.d, N, i), q = ld3(c.q, N, i), x = ld3(c.dv, N, i),
                        r = ld3(c.r, N, i);
@@ -721,6 +746,11 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
                 for (int u = 0; u < RV; u++) {
                     const int vv = lt + u * T;
                     if (vv < Ni) st3(c.dv, N, voff + vv, rld(2, u));
+                }
+#pragma unroll
+                for (int u = 0; u < RG; u++) {
+                    const int vv = lt + (RV + u) * T;
+                    if (vv < Ni) st3(c.dv, N, voff + vv, kept[u].x);
                 }
             }
         }
@@ -761,6 +791,27 @@ __global__ __launch_bounds__(NT, 4) void k_batch_step(DevBatch c, StepScalars s,
         }
         __syncthreads();
     }
+}
+
+// Assembly and CG start of all cloths' vertices.  A launch of its own: no
+// vertex waits for another's sums, so every CU has work however uneven the
+// cloths are, and the solve's kernel keeps its registers (with the assembly
+// inside it spilled).  512 cloths of 16x16 to 128x128 (3.1 M vertices): the
+// step took 1441 us in one launch, 1284 in both (this one 330: 890 MB to and
+// from memory, twelve springs per vertex to issue; 64- and 128-thread blocks
+// take 363 and 338); 64 cloths of 32x32 to 96x96, a quarter of the CUs in the
+// solve: 607 and 400 us (this one 42).  It also rewinds the solve's queue.
+constexpr int kAssembleThreads = 256;
+template <bool ADJ>
+__global__ __launch_bounds__(kAssembleThreads) void k_batch_assemble(DevBatch c, StepScalars s, BatchAdjBufs adj) {
+    const int i = blockIdx.x * kAssembleThreads + threadIdx.x;
+    if (i == 0) *c.queue = 0;
+    if (i >= c.Ntot) return;
+    if (c.stencil_asm)
+        assemble_vertex_stencil(c, s, i, c.row[i]);
+    else
+        assemble_vertex(c, s, i, c.row[i]);
+    if constexpr (ADJ) adjoint_start_vertex(c, s, adj, i);
 }
 
 // The adjoint's gather (as the single cloth's k_adj_gather): c.x, c.v the
@@ -843,17 +894,17 @@ hipError_t launch_batch_owner_constants(const DevBatch& c, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_batch_reset(const DevBatch& c, hipStream_t st) {
-    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, st, c.queue);
-    return hipGetLastError();
-}
-
 template <bool ADJ>
 static hipError_t launch_batch(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a,
                                int block_threads, int grid, hipStream_t st) {
     if (c.asm_once && (c.lds_floats < 12 * block_threads || c.lds_floats > kBatchLdsFloats))
         return hipErrorInvalidValue;
     const size_t lds = sizeof(float) * (size_t)(c.asm_once ? c.lds_floats : batch_resident_floats(block_threads));
+    if (c.asm_once)
+        hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, st, c.queue);
+    else
+        hipLaunchKernelGGL(k_batch_assemble<ADJ>, dim3(std::max(1, (c.Ntot + kAssembleThreads - 1) / kAssembleThreads)),
+                           dim3(kAssembleThreads), 0, st, c, s, a);
     switch (block_threads * 2 + (c.asm_once ? 1 : 0)) {
         case 512:
             hipLaunchKernelGGL((k_batch_step<256, ADJ, false>), dim3(grid), dim3(256), lds, st, c, s, a);

@@ -173,7 +173,6 @@ int apply_schedule(oc_batch_s* b) {
 }
 
 int launch_step(oc_batch_s* b, hipStream_t st) {
-    OC_HIP(oc::launch_batch_reset(b->dc, st));
     OC_HIP(oc::launch_batch_step(b->dc, batch_scalars(b), b->sched.block_threads, b->grid, st));
     return OC_OK;
 }
@@ -307,7 +306,7 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
     const size_t row = align_up(sizeof(int) * N);
     const size_t amask = align_up(sizeof(uint32_t) * (st_asm ? N : 1));
     const size_t cst = align_up(sizeof(float) * 3 * oc::kOwned * (st_asm ? N : 1));
-    const size_t total = 8 * vec + blocks + as + am + pm + pk + 3 * sp + slotc + pin + 6 * per + amask + cst + row + 256;
+    const size_t total = 7 * vec + blocks + as + am + pm + pk + 3 * sp + slotc + pin + 6 * per + amask + cst + row + 256;
     if (hipMalloc(&b->arena, total) != hipSuccess) {
         delete b;
         return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(total) + " bytes failed");
@@ -328,7 +327,6 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
     d.r = (float*)take(vec);
     d.d = (float*)take(vec);
     d.q = (float*)take(vec);
-    d.b = (float*)take(vec);
     d.pinv = (float*)take(vec);
     d.blocks = (float*)take(blocks);
     d.ainc_s = (const int32_t*)take(as);
@@ -741,7 +739,6 @@ int oc_batch_rollout_backward(oc_batch b, const float* grad_x, const float* grad
             ab.gx_in = rv.gx[1 - cur];
             ab.gv_in = rv.gv[1 - cur];
             ab.gks = rv.gks;
-            OC_HIP(oc::launch_batch_reset(b->dc, b->stream));
             OC_HIP(oc::launch_batch_adjoint(ca, s, ab, b->sched.block_threads, b->grid, b->stream));
             OC_HIP(oc::launch_batch_gather(ca, s, ab, b->stream));
             cur = 1 - cur;

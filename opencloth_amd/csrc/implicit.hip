@@ -1141,12 +1141,6 @@ constexpr unsigned kRollClosed = 1u << 15;       // count in bits 0-14, team siz
 constexpr unsigned long long kRollCallTicks = 50000;  // 0.5 ms of the 100 MHz counter
 constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
 
-// v, opaque to the compiler: what is computed from it is not moved ahead of
-// the iteration loop, where the exchange's few dozen addresses would spill.
-__device__ inline unsigned here(unsigned v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
 // Word i of the exchange, from a uniform base and a 32-bit offset.
 __device__ inline uint64_t xch_load(const uint64_t* p, unsigned i) {
     return __hip_atomic_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(p) + here(i * 8u)),

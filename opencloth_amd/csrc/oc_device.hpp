@@ -119,6 +119,13 @@ __device__ inline V3 spring_force(V3 x1, V3 x2, V3 v1, V3 v2, float L0, float Ks
     return {s * (dp.x * inv), s * (dp.y * inv), s * (dp.z * inv)};
 }
 
+// v, opaque to the compiler: what is computed from it is not moved ahead of
+// an iteration loop, where a few dozen addresses would spill.
+__device__ inline unsigned here(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Wave tree: lane l += lane l+off for off = 32..1; lane 0 ends with the sum
 // (the other lanes' values are not the tree's).  Offsets 32 and 16 by gfx950's
 // lane-swap instructions, the rest by row shifts inside 16 lanes: register

@@ -576,7 +576,6 @@ struct DevBatch {
     float* r;
     float* d;
     float* q;
-    float* b;
     float* pinv;    // Jacobi preconditioner 1/diag(A)
     const uint8_t* pin;
     float* blocks;  // n_planes*6*Ntot
@@ -644,6 +643,7 @@ constexpr int kBatchLdsFloats = 160 * 1024 / 4;
 // Batched CG: vertices per thread whose d, r, q and solution stay in LDS for
 // a whole solve (12 floats each: 36 KiB per 256 threads, 144 KiB for 1024).
 constexpr int kResidentPerThread = 3;
+constexpr int kInRegisters = 2;  // the next ones', in registers (3% of a step)
 constexpr int batch_resident_floats(int block_threads) { return 12 * kResidentPerThread * block_threads; }
 
 // Buffers of one batched adjoint step (SoA, stride Ntot).
@@ -661,7 +661,6 @@ hipError_t launch_batch_adjoint(const DevBatch& c, const StepScalars& s, const B
                                 int block_threads, int grid, hipStream_t st);
 // dJ/dx, dJ/dv and dJ/dks of the step whose adjoint solve is in c.dv.
 hipError_t launch_batch_gather(const DevBatch& c, const StepScalars& s, const BatchAdjBufs& a, hipStream_t st);
-hipError_t launch_batch_reset(const DevBatch& c, hipStream_t st);
 // Fill slot_c planes q0 .. q0+nq-1 from L0/ks/kd through the slot tables.
 hipError_t launch_batch_slot_constants(const DevBatch& c, int q0, int nq, hipStream_t st);
 hipError_t launch_batch_step(const DevBatch& c, const StepScalars& s, int block_threads,
