@@ -1141,17 +1141,6 @@ constexpr unsigned kRollClosed = 1u << 15;       // count in bits 0-14, team siz
 constexpr unsigned long long kRollCallTicks = 50000;  // 0.5 ms of the 100 MHz counter
 constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
 
-// Word i of the exchange, from a uniform base and a 32-bit offset.
-__device__ inline uint64_t xch_load(const uint64_t* p, unsigned i) {
-    return __hip_atomic_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(p) + here(i * 8u)),
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void xch_store(uint64_t* p, unsigned i, unsigned tag, float v) {
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(p) + here(i * 8u)),
-                       ((uint64_t)tag << 32) | (uint64_t)__float_as_uint(v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Sign in (one thread per block); returns this block's rank, or -1 when the
 // roll is closed.
 __device__ inline int roll_call_sign(unsigned* roll) {

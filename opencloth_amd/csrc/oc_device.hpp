@@ -126,6 +126,17 @@ __device__ inline unsigned here(unsigned v) {
     return v;
 }
 
+// Word i of an exchange between blocks, from a uniform base and a 32-bit offset.
+__device__ inline uint64_t xch_load(const uint64_t* p, unsigned i) {
+    return __hip_atomic_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(p) + here(i * 8u)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void xch_store(uint64_t* p, unsigned i, unsigned tag, float v) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(p) + here(i * 8u)),
+                       ((uint64_t)tag << 32) | (uint64_t)__float_as_uint(v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Wave tree: lane l += lane l+off for off = 32..1; lane 0 ends with the sum
 // (the other lanes' values are not the tree's).  Offsets 32 and 16 by gfx950's
 // lane-swap instructions, the rest by row shifts inside 16 lanes: register

@@ -384,6 +384,10 @@ struct DevVerlet {
     const uint32_t* asm_mask;
     const float* cst;
     int stencil_asm;
+    // resident steps: two sets of 4 words per vertex, and a host word set
+    // when a wait for one ended without it
+    uint64_t* xch;
+    int* err;
 };
 struct VerletScalars {
     float mass, gx, gy, gz, damping, dt;
@@ -391,6 +395,14 @@ struct VerletScalars {
 };
 hipError_t launch_verlet_forces(const DevVerlet& c, const VerletScalars& s, hipStream_t st);
 hipError_t launch_verlet_step(const DevVerlet& c, const VerletScalars& s, hipStream_t st);
+// Side of the square regions of a resident launch on the current device, 0
+// when the cloth (mask: its asm_mask) does not fit it.
+int verlet_resident_region(int nx, int ny, const uint32_t* mask);
+// nsteps >= 2 steps of c.x and c.xl with the collider (e may be NULL) in one
+// cooperative launch; the results go to x and xl, which may be c.x and c.xl.
+// The tags base + 2 .. base + 2 nsteps (base even) must not be in c.xch.
+hipError_t launch_verlet_resident(const DevVerlet& c, const VerletScalars& s, float* x, float* xl, int region, int nsteps,
+                                  unsigned base, const oc_ellipsoid* e, hipStream_t st);
 
 // Grid Verlet (grid_verlet.hip): the reference's GPU Verlet kernel on a
 // width x height grid with a fixed 12-neighbour stencil.  Two position sets

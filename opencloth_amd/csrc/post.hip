@@ -12,6 +12,8 @@
 //                 thread sees a half-updated neighbour
 //
 // Expressions follow the reference's GLM order, built with -ffp-contract=off.
+#include <algorithm>
+
 #include "oc_device.hpp"
 
 namespace oc {
@@ -217,6 +219,272 @@ __global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s)
     st3(c.xn, N, i, xn);
 }
 
+// ---------------------------------------------------------------------------
+// resident Verlet: many steps in one launch, the cloth in registers and LDS
+// ---------------------------------------------------------------------------
+// A launch per step reads 36 floats of every vertex and its springs again and
+// waits for the launch before it.  Here every block keeps a region of T x T
+// vertices for all steps of a call, a vertex per thread: positions and spring
+// constants in registers, the region's positions and velocities with their
+// halo in LDS.  In a step a thread evaluates the six springs its vertex owns
+// (threads of the first waves also one of the strips around the region, whose
+// owners are outside), hands the forces to the partners through LDS, and adds
+// all of its vertex's in stencil order.  The outer two rows and columns go to
+// the neighbouring regions as 8-byte words (value, tag) that are stored and
+// polled with relaxed device-scope accesses, each its own flag.  A region
+// publishes step n + 2 only after it has read its neighbours' step n + 1, and
+// these publish that only after they have read its step n, so two sets of
+// words are enough.  The tag's low bit tells that the collider moved the
+// vertex (its previous position is then the position itself; else the reader
+// knows it).  Blocks wait for each other, so the launch is cooperative; a
+// wait is bounded, and one that ends without its word sets *err and every
+// block leaves.
+//
+// Measured per step of 200, with the collider, a launch each for step and
+// collider before: 512x512 14.2 -> 6.5 us, 256x256 12 -> 4.6, 21x21 8.4 ->
+// 3.9.  About 1 us of it is the exchange; the rest is the chain through a step
+// (six springs with a square root and two divisions each, the sum over
+// twelve, three barriers), at 512x512 with four waves per SIMD to issue.
+constexpr int kVerletPolls = 1 << 21;  // seconds
+
+template <int T>
+struct VerletRegion {
+    static constexpr int NT = T * T, H = kHalo, W = T + 2 * H, NW = W * W, NS = strip_total<T, T>();
+    static constexpr int NH = NW - NT;  // halo vertices
+    static constexpr int HR = (3 * NH + NT - 1) / NT;
+    static constexpr int NJ = NT - NS;  // second springs a region can take (see below)
+    static constexpr size_t lds = sizeof(float) * (6 * NW + 18 * NT + 3 * NT);
+};
+
+template <int T>
+__global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletScalars s, float* xo, float* xlo, int nsteps,
+                                                          unsigned base, oc_ellipsoid e, int has_e) {
+    using R = VerletRegion<T>;
+    constexpr int NT = R::NT, H = R::H, W = R::W, NW = R::NW, NS = R::NS;
+    static_assert(R::NJ > 0 && 4 * R::NJ <= 18 * NT, "one extra spring per thread, room for their list");
+    extern __shared__ float lds[];
+    __shared__ int lost, jobs;
+    float* const wx = lds;           // 3 planes of the window: positions
+    float* const wv = lds + 3 * NW;  // velocities
+    float* const fo = lds + 6 * NW;  // 18 planes of NT: force of own spring o, component c at plane 3 o + c
+    float* const fs = fo + 18 * NT;  // 3 planes of NT: the threads' extra springs' forces
+    const int tid = threadIdx.x, N = c.N, nx = c.nx, ny = c.ny;
+    const int ntx = (nx + T - 1) / T, nt = ntx * ((ny + T - 1) / T);
+    const int tile = tile_of_block(blockIdx.x, nt);
+    const int bx = tile % ntx, by = tile / ntx;
+    const int lx = tid % T, ly = tid / T;
+    const int gi = bx * T + lx, gj = by * T + ly, i = gj * nx + gi;
+    const bool own = gi < nx && gj < ny;
+    if (tid == 0) lost = jobs = 0;
+    for (int w = tid; w < NW; w += NT) {
+        const int gx = bx * T - H + w % W, gy = by * T - H + w / W;
+        V3 x = {0.0f, 0.0f, 0.0f}, v = x;
+        if (gx >= 0 && gx < nx && gy >= 0 && gy < ny) {
+            x = ld3(c.x, N, gy * nx + gx);
+            const V3 xl = ld3(c.xl, N, gy * nx + gx);
+            v = {(x.x - xl.x) / s.dt, (x.y - xl.y) / s.dt, (x.z - xl.z) / s.dt};
+        }
+        wx[w] = x.x;
+        wx[NW + w] = x.y;
+        wx[2 * NW + w] = x.z;
+        wv[w] = v.x;
+        wv[NW + w] = v.y;
+        wv[2 * NW + w] = v.z;
+    }
+    const int at = (ly + H) * W + lx + H;
+    V3 xi = {0.0f, 0.0f, 0.0f}, xl = xi;
+    uint32_t mi = 0u;
+    bool pinned = true;
+    float L0[kOwned], ks[kOwned], kd[kOwned];
+#pragma unroll
+    for (int o = 0; o < kOwned; o++) L0[o] = ks[o] = kd[o] = 0.0f;
+    if (own) {
+        xi = ld3(c.x, N, i);
+        xl = ld3(c.xl, N, i);
+        mi = c.asm_mask[i];
+        pinned = c.pin[i] != 0;
+#pragma unroll
+        for (int o = 0; o < kOwned; o++) {
+            const float* p = c.cst + (size_t)(3 * o) * N + i;
+            L0[o] = p[0];
+            ks[o] = p[N];
+            kd[o] = p[2 * (size_t)N];
+        }
+    }
+    // this thread's extra spring: the window places of its ends, -1 for none.
+    // The first threads' are the strips'; the next ones' the second springs
+    // of the region's pairs (the stencil's duplicated bends), which each end
+    // evaluates for itself: a vertex lists its own, at most two (second), in
+    // stencil order
+    int sa = -1, sb = 0;
+    float sL0 = 0.0f, sks = 0.0f, skd = 0.0f;
+    if (tid < NS) {
+        int o, k, px, py;
+        strip_of_column<T, T>(tid, o, k);
+        strip_owner<T, T>(o, k, px, py);
+        const int gx = bx * T + px, gy = by * T + py;
+        if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && ((c.asm_mask[gy * nx + gx] >> owned_k(o)) & 1u)) {
+            const float* p = c.cst + (size_t)(3 * o) * N + gy * nx + gx;
+            sL0 = p[0];
+            sks = p[N];
+            skd = p[2 * (size_t)N];
+            sa = (py + H) * W + px + H;
+            sb = sa + own_dy(o) * W + own_dx(o);
+        }
+    }
+    __syncthreads();
+    unsigned second = 0;
+    {
+        int found = 0;
+#pragma unroll 1
+        for (unsigned m = mi >> 16; m; m &= m - 1u) {
+            const int k = __ffs(m) - 1, o = owned_index(k);
+            const int slot = atomicAdd(&jobs, 1);
+            if (slot >= R::NJ || found >= 2) break;  // (verlet_seconds_fit has ruled this out)
+            const float* p = c.cst + (size_t)(3 * (kOwned + o)) * N +
+                             (stencil_owner(k) ? i : i + stencil_dj(k) * nx + stencil_di(k));
+            float* const job = fo + 4 * slot;
+            job[0] = __int_as_float(at | (at + stencil_dj(k) * W + stencil_di(k)) << 16);
+            job[1] = p[0];
+            job[2] = p[N];
+            job[3] = p[2 * (size_t)N];
+            second |= (unsigned)(NS + slot) << (16 * found++);
+        }
+    }
+    __syncthreads();
+    if (tid >= NS && tid - NS < jobs) {
+        const float* job = fo + 4 * (tid - NS);
+        sa = __float_as_int(job[0]) & 0xFFFF;
+        sb = __float_as_int(job[0]) >> 16;
+        sL0 = job[1];
+        sks = job[2];
+        skd = job[3];
+    }
+    // where the force of the partner's spring in direction o is: in fo, or
+    // (one's complement) in fs
+    int part[kOwned];
+#pragma unroll
+    for (int o = 0; o < kOwned; o++) {
+        const int px = lx - own_dx(o), py = ly - own_dy(o);
+        part[o] = px >= 0 && px < T && py >= 0 && py < T ? 3 * o * NT + py * T + px
+                                                         : ~(strip_base<T, T>(o) + strip_index<T, T>(o, px, py));
+    }
+    // the halo words this thread reads: word of the exchange (-1: outside the
+    // cloth) and place in the window's planes
+    int hsrc[R::HR], hdst[R::HR];
+#pragma unroll
+    for (int q = 0; q < R::HR; q++) {
+        const int k = tid + q * NT, h = k / 3, comp = k % 3;
+        int px = 0, py = 0;
+        if (h < 2 * W) {
+            px = h % W;
+            py = h / W;
+        } else if (h < 4 * W) {
+            px = h % W;
+            py = T + h / W;
+        } else {
+            const int r = h - 4 * W;
+            px = (r & 1) + (r >= 2 * T ? T + H : 0);
+            py = H + (r % (2 * T)) / 2;
+        }
+        const int gx = bx * T - H + px, gy = by * T - H + py;
+        hsrc[q] = h < R::NH && gx >= 0 && gx < nx && gy >= 0 && gy < ny ? 4 * (gy * nx + gx) + comp : -1;
+        hdst[q] = comp * NW + py * W + px;
+    }
+    const bool rim = own && (lx < H || lx >= T - H || ly < H || ly >= T - H);
+    const float c2 = (s.dt * s.dt) / s.mass;
+    auto win = [&](const float* p, int a) { return V3{p[a], p[NW + a], p[2 * NW + a]}; };
+
+    for (int n = 0; n < nsteps; n++) {
+        __syncthreads();  // the window is complete
+        if (lost) return;
+        const V3 vi = win(wv, at);
+        V3 f[kOwned];
+#pragma unroll
+        for (int o = 0; o < kOwned; o++) {
+            f[o] = V3{0.0f, 0.0f, 0.0f};
+            if ((mi >> owned_k(o)) & 1u) {
+                const int b = at + own_dy(o) * W + own_dx(o);
+                f[o] = spring_force(xi, win(wx, b), vi, win(wv, b), L0[o], ks[o], kd[o]);
+            }
+            fo[(3 * o) * NT + tid] = f[o].x;
+            fo[(3 * o + 1) * NT + tid] = f[o].y;
+            fo[(3 * o + 2) * NT + tid] = f[o].z;
+        }
+        if (sa >= 0) {
+            const V3 g = spring_force(win(wx, sa), win(wx, sb), win(wv, sa), win(wv, sb), sL0, sks, skd);
+            fs[tid] = g.x;
+            fs[NT + tid] = g.y;
+            fs[2 * NT + tid] = g.z;
+        }
+        __syncthreads();
+        V3 F = {0.0f, 0.0f, 0.0f};
+        if (!pinned) F = {F.x + s.gx * s.mass, F.y + s.gy * s.mass, F.z + s.gz * s.mass};
+        F = {F.x + s.damping * vi.x, F.y + s.damping * vi.y, F.z + s.damping * vi.z};
+        if (!pinned) {
+            unsigned q = second;
+#pragma unroll
+            for (int k = 0; k < kStencil; k++) {
+                if (!((mi >> k) & 1u)) continue;
+                const int o = owned_index(k);
+                if (stencil_owner(k)) {
+                    F = add3(F, f[o]);
+                } else {  // the force on the spring's owner
+                    const float* p = part[o] >= 0 ? fo + part[o] : fs + ~part[o];
+                    F = sub3(F, V3{p[0], p[NT], p[2 * NT]});
+                }
+                if ((mi >> (16 + k)) & 1u) {
+                    const float* p = fs + (q & 0xFFFFu);
+                    F = add3(F, V3{p[0], p[NT], p[2 * NT]});
+                    q >>= 16;
+                }
+            }
+        }
+        V3 xn = {xi.x + (xi.x - xl.x) + c2 * F.x, xi.y + (xi.y - xl.y) + c2 * F.y, xi.z + (xi.z - xl.z) + c2 * F.z};
+        if ((s.flags & OC_FLAG_GROUND_CLAMP) && xn.y < 0.0f) xn.y = 0.0f;
+        xl = xi;
+        bool moved = false;
+        if (has_e) xn = ellipsoid_push(e, xn, moved);
+        if (moved) xl = xn;
+        xi = xn;
+        if (n + 1 == nsteps) break;
+        uint64_t* const words = c.xch + (size_t)(n & 1) * 4 * N;
+        const unsigned tag = base + 2u * (unsigned)(n + 1);
+        if (rim) {
+            xch_store(words, 4u * i, tag + moved, xi.x);
+            xch_store(words, 4u * i + 1u, tag + moved, xi.y);
+            xch_store(words, 4u * i + 2u, tag + moved, xi.z);
+        }
+        __syncthreads();  // the window has been read
+        wx[at] = xi.x;
+        wx[NW + at] = xi.y;
+        wx[2 * NW + at] = xi.z;
+        wv[at] = (xi.x - xl.x) / s.dt;
+        wv[NW + at] = (xi.y - xl.y) / s.dt;
+        wv[2 * NW + at] = (xi.z - xl.z) / s.dt;
+#pragma unroll
+        for (int q = 0; q < R::HR; q++) {
+            if (hsrc[q] < 0) continue;
+            uint64_t w = xch_load(words, (unsigned)hsrc[q]);
+            for (int polls = 0; (((unsigned)(w >> 32)) & ~1u) != tag; polls++) {
+                if (polls == kVerletPolls) {
+                    lost = 1;
+                    __hip_atomic_store(c.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    break;
+                }
+                w = xch_load(words, (unsigned)hsrc[q]);
+            }
+            const float x = __uint_as_float((unsigned)w), before = ((w >> 32) & 1u) ? x : wx[hdst[q]];
+            wx[hdst[q]] = x;
+            wv[hdst[q]] = (x - before) / s.dt;
+        }
+    }
+    if (own) {
+        st3(xo, N, i, xi);
+        st3(xlo, N, i, xl);
+    }
+}
+
 // The Verlet step has no reduction, so its tile shape is free: 32x8 measured
 // faster than the implicit kernels' 64x8 at 512x512 (15.5 against 17.4 us).
 constexpr int kVerletTileX = 32, kVerletTileY = 8;
@@ -249,6 +517,63 @@ hipError_t launch_provot(const DevCloth& c, float slack, hipStream_t st) {
     else
         hipLaunchKernelGGL(k_provot<kMaxAssemblyWidth>, dim3((c.N + 255) / 256), dim3(256), 0, st, c, slack);
     return hipGetLastError();
+}
+
+// CUs, if a region's block fits one and cooperative launches are there.
+template <int T>
+static int verlet_blocks_fit() {
+    int dev = 0, coop = 0, cus = 0, per_cu = 0, lds = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+        VerletRegion<T>::lds + 64 > (size_t)lds ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_verlet_resident<T>, T * T, VerletRegion<T>::lds) !=
+            hipSuccess)
+        return 0;
+    return per_cu > 0 ? cus : 0;
+}
+
+static int verlet_regions(int nx, int ny, int T) { return ((nx + T - 1) / T) * ((ny + T - 1) / T); }
+
+// A region's second springs have a thread each, a vertex at most two.
+template <int T>
+static bool verlet_seconds_fit(int nx, int ny, const uint32_t* mask) {
+    for (int by = 0; by < ny; by += T)
+        for (int bx = 0; bx < nx; bx += T) {
+            int n = 0;
+            for (int y = by; y < std::min(by + T, ny); y++)
+                for (int x = bx; x < std::min(bx + T, nx); x++) {
+                    const int k = __builtin_popcount(mask[(size_t)y * nx + x] >> 16);
+                    if (k > 2) return false;
+                    n += k;
+                }
+            if (n > VerletRegion<T>::NJ) return false;
+        }
+    return true;
+}
+
+// The smaller regions while each has a CU of its own (a wave per SIMD: 256x256
+// 4.6 us per step, in 32x32 regions 5.2; 128x128 4.1 and 5.2), then the larger
+// ones (512x512 6.5 us, in 1024 small regions, four per CU, 7.0).
+int verlet_resident_region(int nx, int ny, const uint32_t* mask) {
+    if (verlet_regions(nx, ny, 16) <= verlet_blocks_fit<16>() && verlet_seconds_fit<16>(nx, ny, mask)) return 16;
+    if (verlet_regions(nx, ny, 32) <= verlet_blocks_fit<32>() && verlet_seconds_fit<32>(nx, ny, mask)) return 32;
+    return 0;
+}
+
+hipError_t launch_verlet_resident(const DevVerlet& c, const VerletScalars& s, float* x, float* xl, int T, int nsteps,
+                                  unsigned base, const oc_ellipsoid* e, hipStream_t st) {
+    if ((T != 16 && T != 32) || nsteps < 2 || (base & 1u) || !c.stencil_asm) return hipErrorInvalidValue;
+    DevVerlet ca = c;
+    VerletScalars sa = s;
+    oc_ellipsoid el = e ? *e : oc_ellipsoid{};
+    int has_e = e != nullptr;
+    void* args[] = {&ca, &sa, &x, &xl, &nsteps, &base, &el, &has_e};
+    const void* k = T == 16 ? reinterpret_cast<const void*>(k_verlet_resident<16>)
+                            : reinterpret_cast<const void*>(k_verlet_resident<32>);
+    const size_t lds = T == 16 ? VerletRegion<16>::lds : VerletRegion<32>::lds;
+    return hipLaunchCooperativeKernel(k, dim3(verlet_regions(c.nx, c.ny, T)), dim3(T * T), args, (unsigned)lds, st);
 }
 
 hipError_t launch_verlet_forces(const DevVerlet& c, const VerletScalars& s, hipStream_t st) {

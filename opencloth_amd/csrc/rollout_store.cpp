@@ -25,6 +25,7 @@ hipError_t RolloutStore::reserve(size_t n, int nsteps, int checkpoint_every, siz
     if (least <= bytes) {  // only to grow: not while the stream's work is captured
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         fits = hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        if (!fits) (void)hipGetLastError();
     }
     if (fits) {
         size_t avail = 0, total = 0;
