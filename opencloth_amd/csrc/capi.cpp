@@ -686,8 +686,7 @@ int oc_cloth_step_physics(oc_cloth c, int32_t nsteps, const oc_ellipsoid* e, flo
     for (int k = 0; k < nsteps; k++) {
         OC_HIP(oc::launch_assemble(c->dc, s, c->stream));
         OC_HIP(oc::launch_cg(c->dc, s, c->stream, false));
-        OC_HIP(oc::launch_update(c->dc, s, c->stream, true));
-        if (e) OC_HIP(oc::launch_ellipsoid(c->dc.x, c->dc.v, c->dc.N, *e, 0, c->stream));
+        OC_HIP(oc::launch_update(c->dc, s, c->stream, true, e));
         if (slack > 0.0f) OC_HIP(oc::launch_provot(c->dc, slack, c->stream));
     }
     c->assembled = false;

@@ -1642,8 +1642,10 @@ __global__ void k_cg_finish(DevCloth c, StepScalars s) {
 
 // v += dv, x += h v, optional ground clamp (IE:693-699).  FIN: block 0 also
 // records the solve's iteration count and status (the step's last launch).
-template <bool FIN>
-__global__ __launch_bounds__(256) void k_update(DevCloth c, StepScalars s) {
+// BALL: then the collider, which puts a vertex on its surface and stops it
+// (k_ellipsoid's work without a launch of its own).
+template <bool FIN, bool BALL>
+__global__ __launch_bounds__(256) void k_update(DevCloth c, StepScalars s, oc_ellipsoid e) {
     if (FIN && blockIdx.x == 0) {
         __shared__ float bc;
         cg_finish_block(c, s, &bc);
@@ -1655,8 +1657,11 @@ __global__ __launch_bounds__(256) void k_update(DevCloth c, StepScalars s) {
     v = {v.x + dv.x, v.y + dv.y, v.z + dv.z};
     x = {x.x + s.h * v.x, x.y + s.h * v.y, x.z + s.h * v.z};
     if ((s.flags & OC_FLAG_GROUND_CLAMP) && x.y < 0.0f) x.y = 0.0f;
-    st3o(c.v, N, i, v);
-    st3o(c.x, N, i, x);
+    bool inside = false;
+    V3 p = x;
+    if constexpr (BALL) p = ellipsoid_push(e, x, inside);
+    st3o(c.v, N, i, inside ? V3{0.0f, 0.0f, 0.0f} : v);
+    st3o(c.x, N, i, p);
     if (!(isfinite(x.x) && isfinite(x.y) && isfinite(x.z) && isfinite(v.x) && isfinite(v.y) &&
           isfinite(v.z))) {
         atomicOr(c.ctl + 2, OC_SOLVE_NONFINITE);
@@ -1929,10 +1934,14 @@ hipError_t launch_cg(const DevCloth& c, const StepScalars& s, hipStream_t st, bo
     return finish ? launch_cg_finish(c, s, st) : hipSuccess;
 }
 
-hipError_t launch_update(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish) {
+hipError_t launch_update(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish, const oc_ellipsoid* e) {
     const dim3 grid((c.N + 255) / 256), block(256);
-    return finish ? launch_k(4, k_update<true>, grid, block, st, c, s)
-                  : launch_k(4, k_update<false>, grid, block, st, c, s);
+    const oc_ellipsoid el = e ? *e : oc_ellipsoid{};
+    if (e)
+        return finish ? launch_k(4, k_update<true, true>, grid, block, st, c, s, el)
+                      : launch_k(4, k_update<false, true>, grid, block, st, c, s, el);
+    return finish ? launch_k(4, k_update<true, false>, grid, block, st, c, s, el)
+                  : launch_k(4, k_update<false, false>, grid, block, st, c, s, el);
 }
 
 }  // namespace oc

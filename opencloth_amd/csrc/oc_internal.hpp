@@ -311,8 +311,9 @@ hipError_t launch_cg_resident(const DevCloth& c, const StepScalars& s, hipStream
 hipError_t launch_cg_spmv(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_axpy(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_finish(const DevCloth& c, const StepScalars& s, hipStream_t st);
+// e: the collider right after the update (NULL: none).
 hipError_t launch_update(const DevCloth& c, const StepScalars& s, hipStream_t st,
-                         bool finish = false);
+                         bool finish = false, const oc_ellipsoid* e = nullptr);
 // Buffers of one adjoint step (SoA vectors of the cloth's size).
 struct AdjointBufs {
     const float* gx_out;  // dL/dx after the step

@@ -48,59 +48,65 @@ __device__ inline bool provot_delta(V3 x1, V3 x2, float rest, float slack, V3& d
     return true;
 }
 
-// Every slot's loads (slot table, then the other end's position and pin and
-// the spring's rest length) are issued before the first correction is
-// computed: the pass is one short chain per vertex rather than one load
-// round trip per spring.  The corrections are then added in slot order.
-template <int WA>
-__global__ __launch_bounds__(256) void k_provot(DevCloth c, float slack) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+// A vertex's corrections in slot order.  The slot table is read three springs
+// ahead, the other end's position and pin and the rest length two, in a loop
+// of 1 KB: with every load of every slot issued first the code was 20 KB,
+// straight through, and a launch spends about 0.4 us per KB on fetching code
+// that it runs once.  21x21: PROVOT_FIGURES
+constexpr int kProvotThreads = 64;
+__global__ __launch_bounds__(kProvotThreads) void k_provot(DevCloth c, float slack) {
+    const int i = blockIdx.x * kProvotThreads + threadIdx.x;
     if (i >= c.N) return;
     const int N = c.N;
-    int sps[WA];
-    uint16_t ms[WA];
-#pragma unroll
-    for (int k = 0; k < WA; k++) {
-        sps[k] = k < c.wa ? c.ainc_s[k * N + i] : -1;
-        ms[k] = k < c.wa ? c.ainc_m[k * N + i] : kEmptySlot;
-    }
+    struct Slot {
+        int sp;
+        uint16_t m;
+    };
+    struct Spring {
+        int sp;
+        uint16_t m;
+        V3 x;
+        float rest;
+        bool pin;
+    };
+    auto slot = [&](int k) {
+        const size_t o = (size_t)min(k, c.wa - 1) * N + i;
+        Slot r = {c.ainc_s[o], c.ainc_m[o]};
+        if (k >= c.wa) r.sp = -1;
+        return r;
+    };
+    auto fetch = [&](Slot q) {  // of vertex i itself past the last slot
+        const int j = q.sp >= 0 ? i + slot_dj(q.m) * c.nx + slot_di(q.m) : i;
+        return Spring{q.sp, q.m, ld3(c.x, N, j), c.L0[max(q.sp, 0)], c.pin[j] != 0};
+    };
+    if (c.wa < 1) return;
+    const Slot s0 = slot(0), s1 = slot(1);
+    Slot ahead = slot(2);
+    Spring nxt = fetch(s0), nxt2 = fetch(s1);
     const V3 xi = ld3(c.x, N, i);
     V3 v = ld3(c.v, N, i);
     const bool pin_i = c.pin[i] != 0;
-    V3 xs[WA];
-    float rest[WA];
-    bool pins[WA];
-#pragma unroll
-    for (int k = 0; k < WA; k++) {
-        xs[k] = V3{0.0f, 0.0f, 0.0f};
-        rest[k] = 0.0f;
-        pins[k] = false;
-        if (sps[k] >= 0) {
-            const int j = i + slot_dj(ms[k]) * c.nx + slot_di(ms[k]);
-            xs[k] = ld3(c.x, N, j);
-            rest[k] = c.L0[sps[k]];
-            pins[k] = c.pin[j] != 0;
-        }
-    }
     bool touched = false;
-#pragma unroll
-    for (int k = 0; k < WA; k++) {
-        if (sps[k] < 0) continue;  // (the slots are packed: the rest are empty too)
-        const bool second = (ms[k] >> 8) & 1u;
-        V3 dP;
-        if (!(second ? provot_delta(xs[k], xi, rest[k], slack, dP)
-                     : provot_delta(xi, xs[k], rest[k], slack, dP)))
-            continue;
+#pragma unroll 1
+    for (int k = 0; k < c.wa; k++) {
+        const Spring in = nxt;
+        if (in.sp < 0) break;  // (the slots are packed)
+        const Slot q = ahead;
+        ahead = slot(k + 3);
+        nxt = nxt2;
+        nxt2 = fetch(q);
+        const bool second = (in.m >> 8) & 1u;
+        V3 dP;  // from the first end's side
+        const V3 a = second ? in.x : xi, b = second ? xi : in.x;
+        if (!provot_delta(a, b, in.rest, slack, dP)) continue;
         if (!second) {  // i is p1: V[p1] -= dP unless p1 is pinned
             if (!pin_i) {
                 v = sub3(v, dP);
                 touched = true;
             }
-        } else {  // i is p2: V[p2] += dP when p1 is pinned or p2 is free
-            if (pins[k] || !pin_i) {
-                v = add3(v, dP);
-                touched = true;
-            }
+        } else if (in.pin || !pin_i) {  // i is p2: V[p2] += dP when p1 is pinned or p2 is free
+            v = add3(v, dP);
+            touched = true;
         }
     }
     if (touched) st3(c.v, N, i, v);
@@ -512,10 +518,7 @@ hipError_t launch_ellipsoid(float* x, float* w, int N, const oc_ellipsoid& e, in
 }
 
 hipError_t launch_provot(const DevCloth& c, float slack, hipStream_t st) {
-    if (c.wa <= 16)
-        hipLaunchKernelGGL(k_provot<16>, dim3((c.N + 255) / 256), dim3(256), 0, st, c, slack);
-    else
-        hipLaunchKernelGGL(k_provot<kMaxAssemblyWidth>, dim3((c.N + 255) / 256), dim3(256), 0, st, c, slack);
+    hipLaunchKernelGGL(k_provot, dim3((c.N + kProvotThreads - 1) / kProvotThreads), dim3(kProvotThreads), 0, st, c, slack);
     return hipGetLastError();
 }
 
