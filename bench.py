@@ -507,7 +507,7 @@ def bench_batch_adjoint(n_cloths: int = 512, steps: int = 60, every: int = 10, p
         "speedup_vs_plain_persistent": ms_plain_p / ms,
         "schedule": {"block_threads": sched[0], "vertices_per_thread": sched[1]},
         "grad_error_vs_fp64": errs,
-        # the adjoint launch (k_batch_step<..., true>) from the committed
+        # the adjoint step (its three launches) from the committed
         # kernel trace and PMC summary of bench.py's batch_adjoint leg
         "adjoint_kernel": adjoint_kernel_profile(),
     }

@@ -819,7 +819,7 @@ __global__ __launch_bounds__(kAssembleThreads) void k_batch_assemble(DevBatch c,
 // launch of its own over all vertices: it needs no cloth's order, and inside
 // the solve's workgroups the largest cloths' gathers ran on while other CUs
 // were idle.  64 cloths of 32x32 to 96x96: the adjoint's launches take 600 us
-// per step (73 of them here), 1.0 ms as one launch.
+// per step (70 of them here), 1.0 ms as one launch.
 constexpr int kGatherThreads = 64;
 __global__ __launch_bounds__(kGatherThreads) void k_batch_gather(DevBatch c, StepScalars s, BatchAdjBufs a) {
     const int N = c.Ntot, i = blockIdx.x * kGatherThreads + threadIdx.x;

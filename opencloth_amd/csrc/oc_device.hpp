@@ -319,7 +319,7 @@ __device__ __forceinline__ void adj_gather_springs(const AdjGatherIn& c, int i, 
         r.mu = ld3(c.mu, N, j);
         r.p = ld3(c.p, N, j);
         constants(min(k, c.wa - 1), sp, r.L0, r.ks, r.kd);
-        r.g = gks[sp];
+        r.g = gks[r.second ? 0 : sp];  // (the first end adds; the ids of a column are far apart)
         return r;
     };
     const V3 xi = ld3(c.x, N, i), vi = ld3(c.v, N, i), mi = ld3(c.mu, N, i), pi = ld3(c.p, N, i);
