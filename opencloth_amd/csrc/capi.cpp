@@ -170,6 +170,7 @@ int cloth_step(oc_cloth_s* c, int nsteps, float* partials) {
     // is not fused: its assembly zeroes dv, which neighbouring blocks of a
     // fused assembly would still be reading for the update.
     const bool fuse = s.warm && s.max_it >= 1;
+    d.asm_rows = assembles_rows(d, s);
     bool pending = false;  // a solve whose update has not been launched yet
     hipError_t e = hipSuccess;
     for (int k = 0; k < nsteps; k++) {
@@ -305,8 +306,9 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
                                                                                  oc::kTileY))
                                 : 0;
     const size_t sync = align_up(sizeof(unsigned) * 4);
+    const size_t rows = align_up(sizeof(float) * oc::kTileY * (size_t)d.nt);
     const size_t total = 17 * vec + blocks + ainc_s + ainc_m + pair_m + pair_k + 3 * sp + pin + amask + cst + scst +
-                         xch + sync;
+                         xch + sync + rows;
     if (hipMalloc(&c->arena, total) != hipSuccess) {
         delete c;
         return fail(OC_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(total) + " bytes failed");
@@ -352,6 +354,7 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     d.xstride = d.res_vt ? oc::resident_stride(d.ntx, d.nty) : 0;
     d.xch = d.res_vt ? (uint64_t*)take(xch) : nullptr;
     d.sync = (unsigned*)take(sync);
+    d.row_part = (float*)take(rows);  // zeros where a tile has no row
 
     auto cleanup = [&](int code) {
         (void)hipFree(c->arena);
@@ -683,11 +686,13 @@ int oc_cloth_step_physics(oc_cloth c, int32_t nsteps, const oc_ellipsoid* e, flo
     if (!c) return fail(OC_ERR_INVALID_ARGUMENT, "cloth is NULL");
     if (nsteps < 0) return fail(OC_ERR_INVALID_ARGUMENT, "nsteps < 0");
     const oc::StepScalars s = scalars(c, c->prm.dt);
+    oc::DevCloth d = c->dc;
+    d.asm_rows = oc::assembles_rows(d, s);
     for (int k = 0; k < nsteps; k++) {
-        OC_HIP(oc::launch_assemble(c->dc, s, c->stream));
-        OC_HIP(oc::launch_cg(c->dc, s, c->stream, false));
-        OC_HIP(oc::launch_update(c->dc, s, c->stream, true, e));
-        if (slack > 0.0f) OC_HIP(oc::launch_provot(c->dc, slack, c->stream));
+        OC_HIP(oc::launch_assemble(d, s, c->stream));
+        OC_HIP(oc::launch_cg(d, s, c->stream, false));
+        OC_HIP(oc::launch_update(d, s, c->stream, true, e));
+        if (slack > 0.0f) OC_HIP(oc::launch_provot(d, slack, c->stream));
     }
     c->assembled = false;
     return OC_OK;
@@ -795,9 +800,11 @@ int load_state(oc_cloth_s* c, const float* src) {
 }
 
 int one_step(oc_cloth_s* c, const oc::StepScalars& s) {
-    OC_HIP(oc::launch_assemble(c->dc, s, c->stream));
-    OC_HIP(oc::launch_cg(c->dc, s, c->stream, false));
-    OC_HIP(oc::launch_update(c->dc, s, c->stream, true));
+    oc::DevCloth d = c->dc;
+    d.asm_rows = oc::assembles_rows(d, s);
+    OC_HIP(oc::launch_assemble(d, s, c->stream));
+    OC_HIP(oc::launch_cg(d, s, c->stream, false));
+    OC_HIP(oc::launch_update(d, s, c->stream, true));
     return OC_OK;
 }
 
@@ -878,7 +885,9 @@ int oc_cloth_rollout_backward(oc_cloth c, const float* grad_x, const float* grad
             ab.gx_in = gx[1 - cur];
             ab.gv_in = gv[1 - cur];
             ab.gks = rv.gks;
-            OC_HIP(oc::launch_assemble(ca, s_cold, c->stream));
+            oc::DevCloth rows = ca;  // (the adjoint's start brings the tiles' sums)
+            rows.asm_rows = oc::assembles_rows(ca, s);
+            OC_HIP(oc::launch_assemble(rows, s_cold, c->stream));
             OC_HIP(oc::launch_adj_init(ca, s, ab, c->stream));
             OC_HIP(oc::launch_cg(ca, s, c->stream));
             oc::DevCloth cg = c->dc;  // pre-step state and the step's solution

@@ -598,6 +598,324 @@ __global__ __launch_bounds__(TX* TY, 4) void k_assemble_st(DevCloth c, StepScala
     if (threadIdx.x == 0) c.del_part[tile] = p;
 }
 
+// The assembly of a cloth of few tiles: blocks of TX x TY vertices, rows of
+// the reduction's tiles; each wave's sum of r.z goes to c.row_part (tile, row
+// of the tile).  A few tiles leave most CUs idle, and what takes the time is
+// a wave's own chain (about 9.5 cycles per instruction with one or two waves
+// on a SIMD: 2000 per direction to evaluate, 2500 to accumulate).  So a block
+// is half a tile, the six directions go in three pairs whose evaluations have
+// no branch and overlap, what an accumulation reads is read before it starts,
+// and second springs are evaluated ahead: 21x21 20.5 -> 17.0 us, 90x71
+// 21.9 -> 16.9, 128x128 21.6 -> 16.9 (half tiles alone, direction by
+// direction, 24, 22.5 and 21.4).
+template <int TX, int TY>
+struct AssemblePairShared {
+    static constexpr int WX = TX + 2 * H, WY = TY + 2 * H, NT = TX * TY, NS = strip_total<TX, TY>();
+    float wx[3][WY][WX];
+    float wv[3][WY][WX];
+    float wdv[3][WY][WX];
+    uint32_t wm[WY][WX];
+    float res[2][12 * NT];  // per direction of the pair 12 planes: f, K w, block term
+    float second[2][12 * NT];
+    float strip[12 * NS];
+    float bc;
+};
+
+template <int TX, int TY, bool UPD>
+__global__ __launch_bounds__(TX* TY, 2) void k_assemble_pairs(DevCloth c, StepScalars s) {
+    constexpr int NT = TX * TY;
+    using SH = AssemblePairShared<TX, TY>;
+    constexpr int WX = SH::WX, WY = SH::WY, NS = SH::NS;
+    constexpr int NWIN = (WX * WY + NT - 1) / NT;
+    constexpr int NSR = (NS + NT - 1) / NT;  // rounds of the strips
+    __shared__ SH sh;
+    const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
+    const int tile = tile_of_block(blockIdx.x, gridDim.x);
+    const int bx = tile % c.ntx, by = tile / c.ntx;
+    const int gi = bx * TX + lx, gj = by * TY + ly;
+    const bool own = gi < c.nx && gj < c.ny;
+    const int N = c.N, nx = c.nx, i = gj * nx + gi;
+    if (blockIdx.x == 0) {
+        if (UPD) cg_finish_block(c, s, &sh.bc);
+        if (threadIdx.x == 0) start_solve(c);
+    }
+    auto own_cst = [&](int m, int o, int q, int g) {
+        return ldo(c.cst, (uint32_t)(((m * kOwned + o) * 3 + q) * N + g));
+    };
+    const uint32_t mi = own ? ldo(c.asm_mask, (uint32_t)i) : 0u;
+    float L0[2], ks[2], kd[2];  // of the pair of directions to come
+    auto prefetch = [&](int p) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int g = own ? i : 0;
+            L0[q] = own_cst(0, 2 * p + q, 0, g);
+            ks[q] = own_cst(0, 2 * p + q, 1, g);
+            kd[q] = own_cst(0, 2 * p + q, 2, g);
+        }
+    };
+    prefetch(0);
+    // this thread's strip springs (owner outside the block, partner inside)
+    int so[NSR], swx[NSR], swy[NSR];
+    bool sin[NSR];
+    float sL0[NSR], sks[NSR], skd[NSR];
+#pragma unroll
+    for (int n = 0; n < NSR; n++) {
+        so[n] = swx[n] = swy[n] = 0;
+        sin[n] = false;
+        sL0[n] = sks[n] = skd[n] = 0.0f;
+        const int col = threadIdx.x + n * NT;
+        if (col < NS) {
+            int ss;
+            strip_of_column<TX, TY>(col, so[n], ss);
+            strip_owner<TX, TY>(so[n], ss, swx[n], swy[n]);
+            const int gx = bx * TX + swx[n], gy = by * TY + swy[n];
+            if (gx >= 0 && gx < nx && gy >= 0 && gy < c.ny) {
+                const int g = gy * nx + gx;
+                sin[n] = true;
+                sL0[n] = own_cst(0, so[n], 0, g);
+                sks[n] = own_cst(0, so[n], 1, g);
+                skd[n] = own_cst(0, so[n], 2, g);
+            }
+        }
+    }
+    // the window: x, v, dv and the stencil masks of the tile and its halo
+    const int x0 = bx * TX - H, y0 = by * TY - H;
+#pragma unroll
+    for (int n = 0; n < NWIN; n++) {
+        const int idx = threadIdx.x + n * NT;
+        if (idx < WX * WY) {
+            const int wx = idx % WX, wy = idx / WX;
+            const int gx = x0 + wx, gy = y0 + wy;
+            V3 xw = {0.0f, 0.0f, 0.0f}, vw = xw, dw = xw;
+            uint32_t mw = 0;
+            if (gx >= 0 && gx < nx && gy >= 0 && gy < c.ny) {
+                const int g = gy * nx + gx;
+                mw = ldo(c.asm_mask, (uint32_t)g);
+                xw = ld3o(c.x, N, g);
+                vw = ld3o(c.v, N, g);
+                if (UPD) {
+                    const V3 dp = ld3o(c.dv, N, g);
+                    vw = {vw.x + dp.x, vw.y + dp.y, vw.z + dp.z};
+                    xw = {xw.x + s.h * vw.x, xw.y + s.h * vw.y, xw.z + s.h * vw.z};
+                    if ((s.flags & OC_FLAG_GROUND_CLAMP) && xw.y < 0.0f) xw.y = 0.0f;
+                    dw = dp;
+                } else if (s.warm) {
+                    dw = ld3o(c.dv, N, g);
+                }
+            }
+            sh.wx[0][wy][wx] = xw.x;
+            sh.wx[1][wy][wx] = xw.y;
+            sh.wx[2][wy][wx] = xw.z;
+            sh.wv[0][wy][wx] = vw.x;
+            sh.wv[1][wy][wx] = vw.y;
+            sh.wv[2][wy][wx] = vw.z;
+            sh.wdv[0][wy][wx] = dw.x;
+            sh.wdv[1][wy][wx] = dw.y;
+            sh.wdv[2][wy][wx] = dw.z;
+            sh.wm[wy][wx] = mw;
+        }
+    }
+    // the first two second springs of this vertex's pairs, in stencil order
+    float eL0[2] = {0.0f, 0.0f}, eks[2] = {0.0f, 0.0f}, ekd[2] = {0.0f, 0.0f};
+    int ek[2] = {-1, -1};
+    {
+        uint32_t m = mi >> 16;
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+            if (m) {
+                const int k = __ffs(m) - 1, o = owned_index(k);
+                const int g = stencil_owner(k) ? i : i + stencil_dj(k) * nx + stencil_di(k);
+                ek[q] = k;
+                eL0[q] = own_cst(1, o, 0, g);
+                eks[q] = own_cst(1, o, 1, g);
+                ekd[q] = own_cst(1, o, 2, g);
+                m &= m - 1u;
+            }
+    }
+    __syncthreads();
+
+    const float h = s.h, hh = s.hh;
+    const int cx = lx + H, cy = ly + H;
+    const V3 xi = {sh.wx[0][cy][cx], sh.wx[1][cy][cx], sh.wx[2][cy][cx]};
+    const V3 vi = {sh.wv[0][cy][cx], sh.wv[1][cy][cx], sh.wv[2][cy][cx]};
+    const V3 dvi = {sh.wdv[0][cy][cx], sh.wdv[1][cy][cx], sh.wdv[2][cy][cx]};
+    bool pinned = true;
+    V3 acc = {0.0f, 0.0f, 0.0f}, kv = {0.0f, 0.0f, 0.0f};
+    V3 adv = {0.0f, 0.0f, 0.0f}, dg = {0.0f, 0.0f, 0.0f};
+    if (own) {
+        pinned = ldo(c.pin, (uint32_t)i) != 0;
+        if (!s.warm) st3o(c.dv, N, i, dvi);
+        if (UPD) {
+            st3o(c.xo, N, i, xi);
+            st3o(c.vo, N, i, vi);
+            if (!(isfinite(xi.x) && isfinite(xi.y) && isfinite(xi.z) && isfinite(vi.x) &&
+                  isfinite(vi.y) && isfinite(vi.z)))
+                atomicOr(c.ctl + 3, OC_SOLVE_NONFINITE);
+        }
+        if (!pinned) acc = {0.0f + s.mass * s.gx, 0.0f + s.mass * s.gy, 0.0f + s.mass * s.gz};
+        if (!pinned && s.damp != 0.0f)
+            acc = {acc.x + s.damp * vi.x, acc.y + s.damp * vi.y, acc.z + s.damp * vi.z};
+        adv = {s.md * dvi.x, s.md * dvi.y, s.md * dvi.z};
+        dg = {s.md, s.md, s.md};
+    }
+    auto window3 = [&](float (&w)[3][WY][WX], int px, int py) {
+        return V3{w[0][py][px], w[1][py][px], w[2][py][px]};
+    };
+    auto put = [&](float* p, int stride, const SpringOut& e) {
+        p[0] = e.f.x;
+        p[stride] = e.f.y;
+        p[2 * stride] = e.f.z;
+        p[3 * stride] = e.kw.x;
+        p[4 * stride] = e.kw.y;
+        p[5 * stride] = e.kw.z;
+#pragma unroll
+        for (int q = 0; q < 6; q++) p[(6 + q) * stride] = e.c[q];
+    };
+    auto get = [&](const float* p, int stride) {
+        SpringOut e;
+        e.f = {p[0], p[stride], p[2 * stride]};
+        e.kw = {p[3 * stride], p[4 * stride], p[5 * stride]};
+#pragma unroll
+        for (int q = 0; q < 6; q++) e.c[q] = p[(6 + q) * stride];
+        return e;
+    };
+    // ---- the strips' springs, and this vertex's second springs
+#pragma unroll 1
+    for (int n = 0; n < NSR + 2; n++) {
+        int ax = cx, ay = cy, px = cx, py = cy, stride = NT;
+        float l0 = 0.0f, k0 = 0.0f, d0 = 0.0f;
+        float* dst = nullptr;
+#pragma unroll
+        for (int q = 0; q < NSR; q++)
+            if (n == q && sin[q] && ((sh.wm[swy[q] + H][swx[q] + H] >> owned_k(so[q])) & 1u)) {
+                ax = swx[q] + H;
+                ay = swy[q] + H;
+                px = ax + own_dx(so[q]);
+                py = ay + own_dy(so[q]);
+                l0 = sL0[q];
+                k0 = sks[q];
+                d0 = skd[q];
+                dst = sh.strip + threadIdx.x + q * NT;
+                stride = NS;
+            }
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+            if (n == NSR + q && ek[q] >= 0) {
+                px = cx + stencil_di(ek[q]);
+                py = cy + stencil_dj(ek[q]);
+                l0 = eL0[q];
+                k0 = eks[q];
+                d0 = ekd[q];
+                dst = sh.second[q] + threadIdx.x;
+            }
+        if (dst)
+            put(dst, stride,
+                eval_spring(window3(sh.wx, ax, ay), window3(sh.wx, px, py), window3(sh.wv, ax, ay), window3(sh.wv, px, py),
+                            l0, k0, d0, h, hh));
+    }
+    // One pair of this vertex: position k, its spring's terms from this side,
+    // the neighbour's dv.
+    auto add_pair = [&](int k, const SpringOut& r, V3 dvj, bool owner) {
+        if (!((mi >> k) & 1u)) return;
+        float C[6];
+        auto add = [&](const SpringOut& e) {
+#pragma unroll
+            for (int q = 0; q < 6; q++) C[q] += e.c[q];
+            acc = {acc.x + e.f.x, acc.y + e.f.y, acc.z + e.f.z};
+            kv = {kv.x + e.kw.x, kv.y + e.kw.y, kv.z + e.kw.z};
+        };
+#pragma unroll
+        for (int q = 0; q < 6; q++) C[q] = 0.0f;
+        add(r);
+        if ((mi >> (16 + k)) & 1u) {
+            if (k == ek[0] || k == ek[1]) {
+                add(get(sh.second[k == ek[0] ? 0 : 1] + threadIdx.x, NT));
+            } else {  // a third one (no topology of the reference's)
+                const int o = owned_index(k), di = stencil_di(k), dj = stencil_dj(k), g = owner ? i : i + dj * nx + di;
+                add(eval_spring(xi, window3(sh.wx, cx + di, cy + dj), vi, window3(sh.wv, cx + di, cy + dj),
+                                own_cst(1, o, 0, g), own_cst(1, o, 1, g), own_cst(1, o, 2, g), h, hh));
+            }
+        }
+        if (owner) {
+            const int plane = c.stencil_plane[k];
+#pragma unroll
+            for (int q = 0; q < 6; q++) sto(c.blocks + (size_t)q * N, (uint32_t)(plane * 6 * N + i), C[q]);
+        }
+        const V3 a = symmv(C, V3{dvj.x - dvi.x, dvj.y - dvi.y, dvj.z - dvi.z});
+        adv = {adv.x + a.x, adv.y + a.y, adv.z + a.z};
+        dg = {dg.x - C[0], dg.y - C[1], dg.z - C[2]};
+    };
+#pragma unroll 1
+    for (int p = 0; p < kOwned / 2; p++) {
+        const int oa = 2 * p, ob = 2 * p + 1;
+        const int ax = own_dx(oa), ay = own_dy(oa), bx2 = own_dx(ob), by2 = own_dy(ob);
+        // ---- evaluate this vertex's pairs in both directions (past the
+        // cloth's edge: of the window's zeros, not used)
+        const SpringOut ea = eval_spring(xi, window3(sh.wx, cx + ax, cy + ay), vi, window3(sh.wv, cx + ax, cy + ay), L0[0],
+                                         ks[0], kd[0], h, hh);
+        const SpringOut eb = eval_spring(xi, window3(sh.wx, cx + bx2, cy + by2), vi, window3(sh.wv, cx + bx2, cy + by2),
+                                         L0[1], ks[1], kd[1], h, hh);
+        put(sh.res[0] + threadIdx.x, NT, ea);
+        put(sh.res[1] + threadIdx.x, NT, eb);
+        if (p + 1 < kOwned / 2) prefetch(p + 1);
+        __syncthreads();
+        // ---- accumulate, in this vertex's stencil order
+        auto partner = [&](int q, int o, int dx, int dy) {
+            const int wx = lx - dx, wy = ly - dy;
+            const bool in = wx >= 0 && wx < TX && wy >= 0;
+            const bool have = (mi >> owned_partner_k(o)) & 1u;
+            const float* src = sh.res[q] + (in ? wy * TX + wx : 0);
+            int stride = NT;
+            if (!in && have) {
+                src = sh.strip + strip_base<TX, TY>(o) + strip_index<TX, TY>(o, wx, wy);
+                stride = NS;
+            }
+            SpringOut e = get(src, stride);
+            e.f = {0.0f - e.f.x, 0.0f - e.f.y, 0.0f - e.f.z};
+            e.kw = {0.0f - e.kw.x, 0.0f - e.kw.y, 0.0f - e.kw.z};
+            return e;
+        };
+        const SpringOut pa = partner(0, oa, ax, ay), pb = partner(1, ob, bx2, by2);
+        const V3 va = window3(sh.wdv, cx - ax, cy - ay), vb = window3(sh.wdv, cx - bx2, cy - by2);
+        const V3 ua = window3(sh.wdv, cx + ax, cy + ay), ub = window3(sh.wdv, cx + bx2, cy + by2);
+        add_pair(owned_partner_k(oa), pa, va, false);
+        if (p == 1) {  // 4, 5, 6, 7: the diagonals
+            add_pair(owned_partner_k(ob), pb, vb, false);
+            add_pair(owned_k(ob), eb, ub, true);
+            add_pair(owned_k(oa), ea, ua, true);
+        } else {
+            add_pair(owned_k(oa), ea, ua, true);
+            add_pair(owned_partner_k(ob), pb, vb, false);
+            add_pair(owned_k(ob), eb, ub, true);
+        }
+        __syncthreads();
+    }
+
+    float t = 0.0f;
+    if (own) {
+        V3 b;
+        b.x = pinned ? 0.0f : h * (acc.x + h * kv.x);
+        b.y = pinned ? 0.0f : h * (acc.y + h * kv.y);
+        b.z = pinned ? 0.0f : h * (acc.z + h * kv.z);
+        st3o(c.b, N, i, b);
+        V3 r = pinned ? V3{0.0f, 0.0f, 0.0f} : V3{b.x - adv.x, b.y - adv.y, b.z - adv.z};
+        st3o(c.r, N, i, r);
+        if (s.flags & OC_FLAG_JACOBI) {
+            const V3 pv = {jacobi_inv(dg.x), jacobi_inv(dg.y), jacobi_inv(dg.z)};
+            st3o(c.pinv, N, i, pv);
+            const V3 z = {pv.x * r.x, pv.y * r.y, pv.z * r.z};
+            st3o(c.s, N, i, z);
+            st3o(c.d0, N, i, z);
+            t = dot3(r, z);
+        } else {
+            st3o(c.d0, N, i, r);
+            t = dot3(r, r);
+        }
+    }
+    const float w = wave_sum(t);
+    if (lx == 0) c.row_part[(gj / kTileY * c.ntx + bx) * kTileY + gj % kTileY] = w;
+}
+
 // ---------------------------------------------------------------------------
 // CG iteration k, part 1: direction update on the tile + halo, q = S A d
 // ---------------------------------------------------------------------------
@@ -1254,6 +1572,29 @@ struct ResidentShared {
 };
 constexpr int kGo = 0, kStop = 1, kBreakdown = 2, kTimeout = 4;
 
+// Up to here two assembly blocks per tile have a CU each.
+constexpr int kRowTiles = 128;
+static_assert(kRowTiles <= 64 * kPartialRegs, "the rows are combined into a solve's first loads");
+// A tile's partial of r.z from its rows' sums, as tile_sum adds them, and
+// partial_load of them (nt <= kRowTiles).
+__device__ inline float row_partial(const DevCloth& c, int tile) {
+    const float* q = c.row_part + tile * kTileY;
+    float w[kTileY];
+#pragma unroll
+    for (int k = 0; k < kTileY; k++) w[k] = q[k];
+    float p = w[0];
+#pragma unroll
+    for (int k = 1; k < kTileY; k++) p = p + w[k];
+    return p;
+}
+__device__ inline void row_partial_load(const DevCloth& c, float* v) {
+#pragma unroll
+    for (int j = 0; j < kPartialRegs; j++) {
+        const int k = threadIdx.x + 64 * j;
+        v[j] = 64 * j < kRowTiles && k < c.nt ? row_partial(c, k) : 0.0f;
+    }
+}
+
 template <int TX, int HY>
 __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars s, int nb, int finish) {
     constexpr int TY = kTileY, VT = HY / TY;            // tiles per region
@@ -1294,7 +1635,12 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
     // ---- this thread's vertex: mask, vectors, owned blocks
     const uint32_t mask = own ? ldo(c.pair_mask, (uint32_t)i) : 0u;
     float pv[kPartialRegs];
-    if (tid < 64) partial_load(c.del_part, c.nt, pv);
+    if (tid < 64) {
+        if (VT == 1 && c.asm_rows)
+            row_partial_load(c, pv);
+        else
+            partial_load(c.del_part, c.nt, pv);
+    }
     V3 r = {0.0f, 0.0f, 0.0f}, pn = r, d = r;
     bool pinned = true;
     if (own) {
@@ -1454,6 +1800,10 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
     if (rank < 0) return;
     if (team < nb) {
         __syncthreads();  // (the shared words above have been read)
+        if (VT == 1 && c.asm_rows) {  // every block for itself, all the same
+            for (int k = tid; k < c.nt; k += NT) c.del_part[k] = row_partial(c, k);
+            __syncthreads();
+        }
         if (tid >= TX * TY) return;
         if (!cg_team<TX, TY, kStencil, true>(c, s, c.sync + 2, rank, team, lds.t.sp, lds.t.ws, lds.t.bc)) return;
         __syncthreads();
@@ -1804,6 +2154,11 @@ hipError_t launch_assemble(const DevCloth& c, const StepScalars& s, hipStream_t 
     // solve without iterations leaves where this assembly writes its own).
     if (fused_update && (!s.warm || s.max_it < 1)) return hipErrorInvalidValue;
     const dim3 grid(c.nt), block(kTileX * kTileY);
+    if (c.asm_rows) {
+        const dim3 half(c.ntx * ((c.ny + kTileY / 2 - 1) / (kTileY / 2))), hb(kTileX * kTileY / 2);
+        return fused_update ? launch_k(0, k_assemble_pairs<kTileX, kTileY / 2, true>, half, hb, st, c, s)
+                            : launch_k(0, k_assemble_pairs<kTileX, kTileY / 2, false>, half, hb, st, c, s);
+    }
     if (c.stencil_asm)
         return fused_update ? launch_k(0, k_assemble_st<kTileX, kTileY, true>, grid, block, st, c, s)
                             : launch_k(0, k_assemble_st<kTileX, kTileY, false>, grid, block, st, c, s);
@@ -1873,6 +2228,14 @@ int persistent_cg_grid(const DevCloth& c) {
     return std::min(grid, c.nt);
 }
 
+static bool solves_resident(const DevCloth& c, const StepScalars& s) {
+    return c.res_vt && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION);
+}
+
+bool assembles_rows(const DevCloth& c, const StepScalars& s) {
+    return c.stencil_asm && c.res_vt == 1 && c.nt <= kRowTiles && solves_resident(c, s);
+}
+
 int resident_cg_tiles(const DevCloth& c) {
     int dev = 0, cus = 0;
     if (!c.stencil || c.nt > kResidentTiles || hipGetDevice(&dev) != hipSuccess ||
@@ -1895,7 +2258,7 @@ hipError_t launch_cg_resident(const DevCloth& c, const StepScalars& s, hipStream
 
 hipError_t launch_cg(const DevCloth& c, const StepScalars& s, hipStream_t st, bool finish) {
     hipError_t e;
-    if (c.res_vt && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION))
+    if (solves_resident(c, s))
         return launch_cg_resident(c, s, st, finish, resident_blocks(c.ntx, c.nty, c.res_vt));
     if (c.persistent && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION)) {
         if (c.persistent > c.nt) return hipErrorInvalidValue;  // a block without a tile

@@ -231,6 +231,11 @@ struct DevCloth {
     int xslots, xstride;
     uint64_t* xch;
     unsigned* sync;
+    // sums of r.z per row of a tile, kTileY each; asm_rows: the assembly
+    // leaves these, not del_part, and a resident solve takes them (set only
+    // for launches that follow each other)
+    float* row_part;
+    int asm_rows;
 };
 
 // Resident solve (k_cg_resident): one block per region of kTileX x (kTileY
@@ -311,6 +316,8 @@ hipError_t launch_cg_resident(const DevCloth& c, const StepScalars& s, hipStream
 hipError_t launch_cg_spmv(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_axpy(const DevCloth& c, const StepScalars& s, int k, hipStream_t st);
 hipError_t launch_cg_finish(const DevCloth& c, const StepScalars& s, hipStream_t st);
+// Whether an assembly directly followed by a solve of c should leave row sums.
+bool assembles_rows(const DevCloth& c, const StepScalars& s);
 // e: the collider right after the update (NULL: none).
 hipError_t launch_update(const DevCloth& c, const StepScalars& s, hipStream_t st,
                          bool finish = false, const oc_ellipsoid* e = nullptr);
