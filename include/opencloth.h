@@ -276,7 +276,11 @@ int oc_verlet_get_state(oc_verlet verlet, float* x, float* x_last);
 int oc_verlet_compute_forces(oc_verlet verlet, float* f_out);
 /* nsteps of ComputeForces + IntegrateVerlet (VL:428-444) fused per vertex,
  * then the ellipsoid pass (x_last = x on contact, VL:509-533) when given.
- * Replaces StepPhysics of the Verlet demo (VL:557-562). */
+ * Replaces StepPhysics of the Verlet demo (VL:557-562).  From four steps on,
+ * a cloth in the reference's form of up to 512x512 runs them in one
+ * cooperative launch (not while its stream is captured); should a wait
+ * between the launch's blocks ever time out, the next oc_verlet_get_state
+ * returns OC_ERR_DEVICE. */
 int oc_verlet_step(oc_verlet verlet, int32_t nsteps, const oc_ellipsoid* ellipsoid);
 
 /* ---- grid Verlet: the GPU demos' kernel ---------------------------------- */

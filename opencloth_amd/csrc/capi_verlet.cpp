@@ -94,9 +94,11 @@ bool resident(const oc_verlet_s* v, int nsteps) {
     (void)hipGetLastError();
     return false;
 }
-int resident_error(const oc_verlet_s* v) {
-    if (v->err && *(volatile int*)v->err) return set_error(OC_ERR_DEVICE, "a wait between blocks of resident steps timed out");
-    return OC_OK;
+// Reported once, after the stream's work is done.
+int resident_error(oc_verlet_s* v) {
+    if (!v->err || !*(volatile int*)v->err) return OC_OK;
+    *v->err = 0;
+    return set_error(OC_ERR_DEVICE, "a wait between blocks of resident steps timed out");
 }
 
 }  // namespace
