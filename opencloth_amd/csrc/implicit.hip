@@ -31,6 +31,7 @@
 #include <algorithm>
 
 #include "oc_device.hpp"
+#include "cg_control.hpp"
 
 namespace oc {
 
@@ -80,52 +81,9 @@ __global__ __launch_bounds__(TX* TY) void k_forces(DevCloth c, StepScalars s) {
     st3(c.f, N, i, acc);
 }
 
-// Iteration count and status of the solve, by all threads of one block
-// (uniform control flow: partial_sum synchronises the block).  Bits are
-// OR-ed in, so update blocks may flag non-finite values concurrently.
-__device__ inline void cg_finish_block(const DevCloth& c, const StepScalars& s, float* bc) {
-    const int done = c.ctl[0];
-    int it;
-    float delta;
-    if (done) {
-        it = c.ctl[1];
-        delta = c.scal[it];
-    } else {
-        it = s.max_it;
-        delta = partial_sum(c.del_part + (size_t)it * c.nt, c.nt, bc);
-    }
-    // r0.r0: written by the first spmv phase, or equal to delta without iterations
-    const float delta0 = s.max_it > 0 ? c.scal[0] : delta;
-    if (threadIdx.x == 0) {
-        const float thresh = s.tol_mode == 1 ? s.tol2 * delta0 : s.tol2;
-        const int st = c.ctl[2];
-        int extra = 0;
-        if (s.tol_mode != 2 && delta > thresh && !(st & OC_SOLVE_BREAKDOWN))
-            extra |= OC_SOLVE_NOT_CONVERGED;
-        if (!isfinite(delta)) extra |= OC_SOLVE_NONFINITE;
-        c.ctl[1] = it;
-        atomicOr(c.ctl + 2, extra);
-        atomicOr(c.ctl + 3, st | extra);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // assembly + CG start
 // ---------------------------------------------------------------------------
-// Control words of the solve that follows an assembly (one thread): not done,
-// no status; for the resident solve a new roll call, barrier counter and
-// epoch base (past every tag the last resident solve used).
-__device__ inline void start_solve(const DevCloth& c) {
-    c.ctl[0] = 0;
-    c.ctl[1] = 0;
-    c.ctl[2] = 0;
-    if (c.res_vt) {
-        c.sync[0] = c.sync[3];
-        c.sync[1] = 0;
-        c.sync[2] = 0;
-    }
-}
-
 // Constants of one incident spring (gathered by spring id).
 struct SpringC {
     float L0, ks, kd;
@@ -171,13 +129,7 @@ __global__ __launch_bounds__(TX* TY) void k_assemble(DevCloth c, StepScalars s) 
     const int gi = bx * TX + lx, gj = by * TY + ly;
     const bool own = gi < c.nx && gj < c.ny;
     const int N = c.N, i = gj * c.nx + gi;
-    if (blockIdx.x == 0) {
-        // the previous solve's iteration count and status bits go into the
-        // sticky word before the control block is cleared (with UPD that
-        // solve had no update launch to record them)
-        if (UPD) cg_finish_block(c, s, &sh.bc);
-        if (threadIdx.x == 0) start_solve(c);
-    }
+    if (blockIdx.x == 0) begin_solve<UPD>(c, s, &sh.bc);
     // own slot tables and the first springs' constants, then the window
     int sps[WA];
     uint16_t ms[WA];
@@ -362,10 +314,7 @@ __global__ __launch_bounds__(TX* TY, 4) void k_assemble_st(DevCloth c, StepScala
     const int gi = bx * TX + lx, gj = by * TY + ly;
     const bool own = gi < c.nx && gj < c.ny;
     const int N = c.N, nx = c.nx, i = gj * nx + gi;
-    if (blockIdx.x == 0) {
-        if (UPD) cg_finish_block(c, s, &sh.bc);
-        if (threadIdx.x == 0) start_solve(c);
-    }
+    if (blockIdx.x == 0) begin_solve<UPD>(c, s, &sh.bc);
     auto own_cst = [&](int m, int o, int q, int g) {
         return ldo(c.cst, (uint32_t)(((m * kOwned + o) * 3 + q) * N + g));
     };
@@ -635,10 +584,7 @@ __global__ __launch_bounds__(TX* TY, 2) void k_assemble_pairs(DevCloth c, StepSc
     const int gi = bx * TX + lx, gj = by * TY + ly;
     const bool own = gi < c.nx && gj < c.ny;
     const int N = c.N, nx = c.nx, i = gj * nx + gi;
-    if (blockIdx.x == 0) {
-        if (UPD) cg_finish_block(c, s, &sh.bc);
-        if (threadIdx.x == 0) start_solve(c);
-    }
+    if (blockIdx.x == 0) begin_solve<UPD>(c, s, &sh.bc);
     auto own_cst = [&](int m, int o, int q, int g) {
         return ldo(c.cst, (uint32_t)(((m * kOwned + o) * 3 + q) * N + g));
     };
