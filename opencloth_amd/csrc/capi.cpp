@@ -19,7 +19,10 @@ namespace {
 
 thread_local std::string g_err;
 
+// A HIP failure that is reported here is not left for the check after the
+// next launch.
 int fail(int code, const std::string& msg) {
+    if (code == OC_ERR_OUT_OF_MEMORY || code == OC_ERR_DEVICE || code == OC_ERR_NO_DEVICE) (void)hipGetLastError();
     g_err = msg;
     return code;
 }

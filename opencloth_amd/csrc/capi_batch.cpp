@@ -424,7 +424,7 @@ int oc_batch_create(int32_t n_cloths, const int32_t* nx, const int32_t* ny, cons
         std::string e = oc_last_error();
         return fail_free(rc, e);
     }
-    (void)b->io.prepare((size_t)b->Ntot, 3);  // (a transfer reserves and reports again)
+    b->io.prepare((size_t)b->Ntot, 3);
     *out = b;
     rc = oc_batch_set_state(b, x0, v0);
     if (rc != OC_OK) {

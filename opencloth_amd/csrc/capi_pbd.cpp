@@ -211,8 +211,8 @@ int oc_pbd_create(int32_t n_vertices, const float* x0, const uint8_t* pinned,
         // reference's lists, where a solver iteration takes 10 us against 77
         // us for a launch per colour)
         int dev = 0, lds = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        if (!oc::hip_ok(hipGetDevice(&dev)) ||
+            !oc::hip_ok(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)))
             lds = 0;
         const int local = std::min(oc::kPbdLocal, (lds - 4096) / 16);
         const oc::PbdFamily df{n_distance, 2, p->n_dcol, dp.data(), dcol.data()};
@@ -354,7 +354,7 @@ int oc_pbd_create(int32_t n_vertices, const float* x0, const uint8_t* pinned,
         delete p;
         return set_error(OC_ERR_DEVICE, "upload failed");
     }
-    (void)p->io.prepare((size_t)N, 3);  // (a transfer reserves and reports again)
+    p->io.prepare((size_t)N, 3);
     *out = p;
     rc = oc_pbd_set_state(p, x0, nullptr);
     if (rc != OC_OK) {

@@ -90,9 +90,7 @@ constexpr int kResidentSteps = 4;
 bool resident(const oc_verlet_s* v, int nsteps) {
     if (!v->region || nsteps < kResidentSteps || nsteps >= (1 << 24)) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(v->stream, &cap) == hipSuccess) return cap == hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return false;
+    return oc::hip_ok(hipStreamIsCapturing(v->stream, &cap)) && cap == hipStreamCaptureStatusNone;
 }
 // Reported once, after the stream's work is done.
 int resident_error(oc_verlet_s* v) {
@@ -169,7 +167,7 @@ int oc_verlet_create(int32_t nx, int32_t ny, const float* x0, const float* x_las
         v->cst = (float*)p;
         p += cst;
     }
-    if (region && hipHostMalloc((void**)&v->err, sizeof(int)) == hipSuccess) {
+    if (region && oc::hip_ok(hipHostMalloc((void**)&v->err, sizeof(int)))) {
         *v->err = 0;
         v->region = region;
         v->xch = (uint64_t*)p;
@@ -207,7 +205,7 @@ int oc_verlet_create(int32_t nx, int32_t ny, const float* x0, const float* x_las
         delete v;
         return set_error(OC_ERR_DEVICE, "upload failed");
     }
-    (void)v->io.prepare((size_t)v->topo.N, 3);  // (a transfer reserves and reports again)
+    v->io.prepare((size_t)v->topo.N, 3);
     *out = v;
     rc = oc_verlet_set_state(v, x0, x_last0 ? x_last0 : x0);
     if (rc != OC_OK) {

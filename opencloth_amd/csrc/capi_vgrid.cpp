@@ -118,7 +118,7 @@ int oc_vgrid_create(int32_t width, int32_t height, const float* x0, const float*
         pins[0] = 1;
         pins[width - 1] = 1;
     }
-    (void)g->io.prepare((size_t)g->N, 4);  // (a transfer reserves and reports again)
+    g->io.prepare((size_t)g->N, 4);
     *out = g;
     if (hipMemset(g->arena, 0, total) != hipSuccess ||
         hipMemcpy(g->pin, pins.data(), N, hipMemcpyHostToDevice) != hipSuccess) {

@@ -2154,13 +2154,10 @@ hipError_t launch_cg_finish(const DevCloth& c, const StepScalars& s, hipStream_t
 int persistent_cg_grid(const DevCloth& c) {
     if (c.wp > 12) return 0;
     int dev = 0, coop = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop)
-        return 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_cg_persistent<kTileX, kTileY, 12>,
-                                                     kTileX * kTileY, 0) != hipSuccess)
+    if (!hip_ok(hipGetDevice(&dev)) || !hip_ok(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev)) ||
+        !coop || !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) ||
+        !hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_cg_persistent<kTileX, kTileY, 12>, kTileX * kTileY,
+                                                             0)))
         return 0;
     // Every block must own at least one tile: a block without one would not
     // see the stop decision and would wait at a barrier the others have
@@ -2184,8 +2181,8 @@ bool assembles_rows(const DevCloth& c, const StepScalars& s) {
 
 int resident_cg_tiles(const DevCloth& c) {
     int dev = 0, cus = 0;
-    if (!c.stencil || c.nt > kResidentTiles || hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    if (!c.stencil || c.nt > kResidentTiles || !hip_ok(hipGetDevice(&dev)) ||
+        !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)))
         return 0;
     if (c.nt <= cus) return 1;
     return c.ntx * ((c.nty + 1) / 2) <= cus ? 2 : 0;

@@ -13,6 +13,14 @@
 
 namespace oc {
 
+// Whether a call succeeded, for one that may fail: its error is taken off the
+// thread, where the check after the next launch would find it (a call that
+// succeeds does not clear it).
+inline bool hip_ok(hipError_t r) {
+    if (r != hipSuccess) (void)hipGetLastError();
+    return r == hipSuccess;
+}
+
 // A spring may join vertices at most kHalo rows and kHalo columns apart
 // (the reference's bend springs span 2, IE:519-530).  The SpMV stages a
 // kHalo-wide halo around each tile in LDS.
@@ -569,7 +577,8 @@ class StateIo {
     ~StateIo();
     // The slots for states of two arrays of n vertices, ahead of the first
     // transfer (8 MiB of pinned memory take about half a millisecond).
-    hipError_t prepare(size_t n, int comps) { return reserve(2 * sizeof(float) * comps * n + 32); }
+    // Where that fails, a transfer reserves and reports again.
+    void prepare(size_t n, int comps) { (void)hip_ok(reserve(2 * sizeof(float) * comps * n + 32)); }
     hipError_t read(std::initializer_list<IoArray> a, hipStream_t st) { return move(true, a.begin(), (int)a.size(), st); }
     hipError_t write(std::initializer_list<IoArray> a, hipStream_t st) { return move(false, a.begin(), (int)a.size(), st); }
 

@@ -523,13 +523,11 @@ hipError_t launch_provot(const DevCloth& c, float slack, hipStream_t st) {
 template <int T>
 static int verlet_blocks_fit() {
     int dev = 0, coop = 0, cus = 0, per_cu = 0, lds = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+    if (!hip_ok(hipGetDevice(&dev)) || !hip_ok(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev)) ||
+        !coop || !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) ||
+        !hip_ok(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) ||
         VerletRegion<T>::lds + 64 > (size_t)lds ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_verlet_resident<T>, T * T, VerletRegion<T>::lds) !=
-            hipSuccess)
+        !hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_verlet_resident<T>, T * T, VerletRegion<T>::lds)))
         return 0;
     return per_cu > 0 ? cus : 0;
 }

@@ -24,17 +24,16 @@ hipError_t RolloutStore::reserve(size_t n, int nsteps, int checkpoint_every, siz
     bool fits = true;
     if (least <= bytes) {  // only to grow: not while the stream's work is captured
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        fits = hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-        if (!fits) (void)hipGetLastError();
+        fits = hip_ok(hipStreamIsCapturing(st, &cap)) && cap == hipStreamCaptureStatusNone;
     }
     if (fits) {
         size_t avail = 0, total = 0;
-        fits = hipMemGetInfo(&avail, &total) == hipSuccess && want <= std::min(avail / kShare, kMost);
+        fits = hip_ok(hipMemGetInfo(&avail, &total)) && want <= std::min(avail / kShare, kMost);
     }
     if (!fits) want = need(false);
     if (want <= bytes) return hipSuccess;
     void* fresh = nullptr;
-    if (all && hipMalloc(&fresh, want) != hipSuccess) {
+    if (all && !hip_ok(hipMalloc(&fresh, want))) {
         fresh = nullptr;
         want = need(false);
         if (want <= bytes) return hipSuccess;
