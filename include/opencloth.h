@@ -387,8 +387,9 @@ int oc_cloth_get_spring_stiffness(oc_cloth cloth, float* ks);
 /* Run nsteps implicit steps from the current state with dv reset to zero,
  * keeping device checkpoints (x, v, dv) for oc_cloth_rollout_backward: every
  * checkpoint_every steps, or of every step when these (36 bytes per vertex
- * and step) fit an eighth of the free device memory and 8 GiB.  The state
- * ends at step nsteps. */
+ * and step) take at most 8 times the memory of the checkpoints, an eighth of
+ * the free device memory and 8 GiB.  The memory stays with the cloth.  The
+ * state ends at step nsteps. */
 int oc_cloth_rollout_forward(oc_cloth cloth, int32_t nsteps, int32_t checkpoint_every);
 /* Hand-written adjoint of the last rollout_forward: given dL/dx and dL/dv at
  * its final state (host AoS; grad_v may be NULL for zero), return dL/dks

@@ -7,9 +7,11 @@ namespace oc {
 
 // Keeping every state saves the backward pass the second run of every step
 // (a third of a 128x128 rollout's time); it takes 36 bytes per vertex and
-// step.  kShare of the free memory, and at most kMost, bounds what a handle
-// takes beyond the checkpoints that its caller asked for.
-constexpr size_t kShare = 8, kMost = size_t(8) << 30;
+// step.  The caller's checkpoint_every says how much memory a rollout may
+// take, so every state is kept only where that is at most kTimes of it (with
+// checkpoints every sqrt(n) steps: rollouts of up to some 250 steps), and
+// beyond that at most one kShare-th of the free memory and kMost.
+constexpr size_t kTimes = 8, kShare = 8, kMost = size_t(8) << 30;
 
 hipError_t RolloutStore::reserve(size_t n, int nsteps, int checkpoint_every, size_t tail, hipStream_t st) {
     steps = nsteps;
@@ -21,8 +23,8 @@ hipError_t RolloutStore::reserve(size_t n, int nsteps, int checkpoint_every, siz
     const size_t least = need(false);
     size_t want = need(true);
     if (want <= bytes) return hipSuccess;
-    bool fits = true;
-    if (least <= bytes) {  // only to grow: not while the stream's work is captured
+    bool fits = want / kTimes <= least;
+    if (fits && least <= bytes) {  // only to grow: not while the stream's work is captured
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         fits = hip_ok(hipStreamIsCapturing(st, &cap)) && cap == hipStreamCaptureStatusNone;
     }

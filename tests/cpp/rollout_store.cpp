@@ -112,6 +112,17 @@ int main() {
         check("captured", g[0], g[1], ok);
         g_capturing = false;
     }
+    // the caller's checkpoint_every bounds the memory, however much is free
+    const int lengths[][2] = {{24, 8}, {120, 10}, {400, 20}, {1000, 32}, {5000, 70}, {5000, 1}, {5000, 5000}};
+    for (const auto& g : lengths) {
+        oc::RolloutStore r, few;
+        g_free = 0;
+        bool ok = few.reserve(n, g[0], g[1], tail, nullptr) == hipSuccess;
+        g_free = ~size_t(0) / 2;
+        ok = ok && r.reserve(n, g[0], g[1], tail, nullptr) == hipSuccess && laid_out(r, n, tail) &&
+             r.bytes <= 8 * few.bytes && (r.all || (size_t)(g[0] + 1) * 9 * oc::kept_floats(n) > 7 * few.bytes / 4);
+        check("bounded by the checkpoints", g[0], g[1], ok);
+    }
     // no room at all: the error goes to the caller
     oc::RolloutStore none;
     g_most = 0;

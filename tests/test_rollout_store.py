@@ -16,4 +16,4 @@ def test_layouts_and_failures(tmp_path):
                     os.path.join(csrc, "rollout_store.cpp"), "-o", exe], check=True, capture_output=True, timeout=120)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
-    assert len(r.stdout.strip().splitlines()) == 9 * 7 + 1
+    assert len(r.stdout.strip().splitlines()) == 9 * 7 + 7 + 1
