@@ -224,7 +224,9 @@ hipError_t StateIo::move(bool read, const IoArray* in, int n, hipStream_t st) {
         return r;
     }
     if (na > 0) {
-        const int nt = threads_of(total);
+        // (hipStreamPerThread is another stream in every thread: its work is
+        // the caller's own thread's)
+        const int nt = st == hipStreamPerThread ? 1 : threads_of(total);
         if ((r = reserve(total)) != hipSuccess) return r;
         int dev = 0;
         if ((r = hipGetDevice(&dev)) != hipSuccess) return r;
