@@ -1890,7 +1890,11 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
         go = sh.late ? kTimeout : last ? sh.go & kTimeout : sh.go;
     }
 
-    if (blockIdx.x == 0 && tid == 0) c.sync[3] = base + 2u * (unsigned)s.max_it;  // the next solve's base
+    // the next solve's base: past the tags that were used, which every block
+    // has written over the older ones in the words (a solve that stops at once
+    // uses none; were the base to move on all the same, it could come round to
+    // tags that the words still hold)
+    if (blockIdx.x == 0 && tid == 0) c.sync[3] = base + 2u * (unsigned)it + (go == kGo || go == kStop ? 0u : 2u);
     if (go == kTimeout) {  // an exchange timed out: report it, leave dv as it was
         if (tid == 0) {
             __hip_atomic_fetch_or(c.ctl + 4, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
