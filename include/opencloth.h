@@ -62,7 +62,9 @@ typedef enum {
                                    phases); ignored where cooperative launch is absent.
                                    Cloths whose pairs follow the reference's stencil and
                                    that fit the device (about 512 tiles of 64x8 on MI355X)
-                                   are solved in one launch with or without it */
+                                   are solved in one launch with or without it, whose
+                                   blocks wait up to 1 ms for each other and otherwise go
+                                   on, some 7 times slower, with those that get a CU */
 #define OC_FLAG_JACOBI 4        /* Jacobi-preconditioned CG: Baraff and Witkin's modified PCG
                                    with P = diag(A), the intent of BW:308-330 and BW:784-785;
                                    the stopping tests then measure r.(P^-1 r) */

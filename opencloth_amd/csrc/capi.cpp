@@ -308,7 +308,7 @@ int oc_cloth_create(int32_t nx, int32_t ny, const float* x0, const float* v0,
     const size_t xch = d.res_vt ? align_up(sizeof(uint64_t) * oc::resident_words(d.ntx, d.nty, d.res_vt, oc::kTileX,
                                                                                  oc::kTileY))
                                 : 0;
-    const size_t sync = align_up(sizeof(unsigned) * 4);
+    const size_t sync = align_up(sizeof(unsigned) * oc::kSyncWords);
     const size_t rows = align_up(sizeof(float) * oc::kTileY * (size_t)d.nt);
     const size_t total = 17 * vec + blocks + ainc_s + ainc_m + pair_m + pair_k + 3 * sp + pin + amask + cst + scst +
                          xch + sync + rows;

@@ -39,7 +39,7 @@ __device__ inline void cg_finish_block(const DevCloth& c, const StepScalars& s, 
 }
 
 // Control words of the solve that follows an assembly (one thread): not done,
-// no status; for the resident solve a new roll call, barrier counter and
+// no status; for the resident solve a new roll call, new tickets and the
 // epoch base (past every tag the last resident solve used).
 __device__ inline void start_solve(const DevCloth& c) {
     c.ctl[0] = 0;
@@ -48,7 +48,7 @@ __device__ inline void start_solve(const DevCloth& c) {
     if (c.res_vt) {
         c.sync[0] = c.sync[3];
         c.sync[1] = 0;
-        c.sync[2] = 0;
+        c.sync[kSyncTickets] = c.sync[kSyncTickets + kTicketDone] = 0;
     }
 }
 

@@ -1390,10 +1390,10 @@ __global__ __launch_bounds__(TX* TY) void k_cg_axpy(DevCloth c, StepScalars s, i
 // are launched one per CU at most, but another stream's or process's work may
 // hold some CUs: thread 0 of each block signs in, and the blocks take the
 // resident path once all have.  If they have not within kRollCallTicks, the
-// roll is closed; the blocks signed in by then run the solve with the
-// per-iteration code below (memory-based phases, a barrier between them) and
-// later ones leave.  So the launch needs no cooperative launch (20 us each,
-// measured) and cannot wait for a block that never starts.
+// roll is closed, and every block, those that start later too, runs tiles of
+// the per-iteration phases below, by tickets, until the solve is done.  So the
+// launch needs no cooperative launch (20 us each, measured) and cannot wait
+// for a block that never starts.
 //
 // Measured per iteration (30 to 40 iterations, two launches per iteration
 // before): 512x512 16.3 -> 7.1 us, 256x256 about 9 -> 4.3, 128x128 9.7 -> 3.9,
@@ -1401,36 +1401,38 @@ __global__ __launch_bounds__(TX* TY) void k_cg_axpy(DevCloth c, StepScalars s, i
 // 2.4 us among 256 (store to the coherence point, then polled loads of 512
 // words); the rest at 512x512, 2.9 us, is the arithmetic: 16 waves per CU
 // issue about 200 instructions each per iteration.
-constexpr unsigned kRollClosed = 1u << 15;       // count in bits 0-14, team size in bits 16-30
-constexpr unsigned long long kRollCallTicks = 50000;  // 0.5 ms of the 100 MHz counter
+constexpr unsigned kRollClosed = 1u << 15;       // the count is in bits 0-14
+// How long blocks wait for the others: about what an incomplete team takes
+// longer than a complete one (512x512, 30 iterations: 0.24 ms complete, 1.75
+// by tickets with half of the blocks or all but one; 128x128, 40 iterations:
+// 0.17 and 0.7).  Beside another stream's products that leave CUs only now and
+// then, a 512x512 step takes 0.82 ms; with half the wait, and without the late
+// blocks, it took 1.95.
+constexpr unsigned long long kRollCallTicks = 100000;  // 1 ms of the 100 MHz counter
 constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
 
-// Sign in (one thread per block); returns this block's rank, or -1 when the
-// roll is closed.
-__device__ inline int roll_call_sign(unsigned* roll) {
-    const unsigned w = __hip_atomic_fetch_add(roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return (w & kRollClosed) ? -1 : (int)(w & (kRollClosed - 1));
+// Sign in (one thread per block), then wait until all nb blocks have: true
+// once they have, false when the roll is closed.  The word decides: a close
+// only succeeds on a word whose count is below nb, and once the count has
+// reached nb no block closes it.
+__device__ inline void roll_call_sign(unsigned* roll) {
+    __hip_atomic_fetch_add(roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Team size once decided: all nb blocks, or those signed in when the roll was
-// closed.  The word decides: a close only succeeds on a word whose count is
-// below nb, and once the count has reached nb no block closes it.
-__device__ inline int roll_call_wait(unsigned* roll, int nb) {
+__device__ inline bool roll_call_wait(unsigned* roll, int nb) {
     const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
     for (;;) {
         unsigned w = __hip_atomic_load(roll, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (w & kRollClosed) return (int)(w >> 16);
-        const unsigned n = w & (kRollClosed - 1);
-        if ((int)n >= nb) return nb;
+        if (w & kRollClosed) return false;
+        if ((int)w >= nb) return true;
         if (__builtin_amdgcn_s_memrealtime() - t0 > kRollCallTicks)
-            __hip_atomic_compare_exchange_strong(roll, &w, w | kRollClosed | (n << 16), __ATOMIC_RELAXED,
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_compare_exchange_strong(roll, &w, w | kRollClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
         else
             __builtin_amdgcn_s_sleep(1);
     }
 }
 
-// Grid barrier of the blocks of a team (also the persistent solve): every
-// block adds 1 to *bar and waits until it reaches target.  The add is a
+// Grid barrier of the persistent solve's blocks: every block adds 1 to *bar and waits until it reaches target.  The add is a
 // release (the block's writes reach the device-coherent level first); the
 // wait polls with relaxed agent-scope loads, which read the coherent value
 // without invalidating caches, and a single acquire fence follows.  The wait
@@ -1458,30 +1460,65 @@ __device__ inline bool grid_barrier(unsigned* bar, unsigned target, int* err) {
     return ok != 0;
 }
 
-// All CG iterations by a team of co-resident blocks: the spmv and axpy phases
-// of the multi-kernel form, separated by grid barriers instead of kernel
-// boundaries.  Block `rank` of `team` serves tiles rank, rank + team, ... with
-// the same per-tile code.  Every block owns at least one tile and so takes
-// the same stop decisions as the others: all blocks pass the same barriers.
-// Returns false when a barrier timed out.
-template <int TX, int TY, int WP, bool STENCIL>
-__device__ inline bool cg_team(const DevCloth& c, const StepScalars& s, unsigned* bar, int rank, int team,
-                               SpmvShared<TX, TY>& sh, float* ws, float& bc) {
+// All CG iterations in one cooperative launch, for any topology: the spmv and
+// axpy phases of the multi-kernel form, separated by grid barriers instead of
+// kernel boundaries.  Each resident block serves tiles blockIdx.x,
+// + gridDim.x, ... with the same per-tile code.  Every block owns at least one
+// tile and so takes the same stop decisions as the others: all blocks pass the
+// same barriers.
+template <int TX, int TY, int WP>
+__global__ __launch_bounds__(TX* TY) void k_cg_persistent(DevCloth c, StepScalars s, unsigned* bar) {
+    __shared__ SpmvShared<TX, TY> sh;
+    __shared__ float ws[TX * TY / 64];
+    __shared__ float bc;
+    const unsigned nb = gridDim.x;
     unsigned target = 0;
     for (int k = 0; k < s.max_it; k++) {
         bool stop = false;
-        for (int vb = rank; vb < c.nt && !stop; vb += team)
-            stop = spmv_phase<TX, TY, WP, STENCIL, STENCIL>(c, s, k, false, sh, vb);
+        for (int vb = blockIdx.x; vb < c.nt && !stop; vb += gridDim.x)
+            stop = spmv_phase<TX, TY, WP>(c, s, k, false, sh, vb);
         if (stop) break;
-        target += (unsigned)team;
-        if (!grid_barrier(bar, target, c.ctl + 4)) return false;
-        for (int vb = rank; vb < c.nt && !stop; vb += team)
+        target += nb;
+        if (!grid_barrier(bar, target, c.ctl + 4)) break;
+        for (int vb = blockIdx.x; vb < c.nt && !stop; vb += gridDim.x)
             stop = axpy_phase<TX, TY>(c, s, k, false, ws, bc, vb);
         if (stop) break;
-        target += (unsigned)team;
-        if (!grid_barrier(bar, target, c.ctl + 4)) return false;
+        target += nb;
+        if (!grid_barrier(bar, target, c.ctl + 4)) break;
     }
-    return true;
+}
+
+// The same phases of a cloth in the stencil form, G tiles per ticket (what a
+// block of a complete team would have, for as few tickets as serve it), by
+// however many blocks there are (of at least TX * TY threads each, the first
+// of which work).  A phase that stops does so in every tile, and the block
+// that has its tile 0 writes the control words and, with finish, the status.
+template <int TX, int TY, int G>
+__device__ inline void cg_tickets(const DevCloth& c, const StepScalars& s, bool finish, SpmvShared<TX, TY>& sh, float* ws,
+                                  float& bc, Ticket& t) {
+    unsigned* const q = c.sync + kSyncTickets;
+    const unsigned pieces = (unsigned)(c.nt + G - 1) / G;  // at most 256, of 2 * 100000 phases
+    const unsigned total = 2u * (unsigned)s.max_it * pieces;
+    for (;;) {
+        const int what = ticket_take(q, pieces, total, c.ctl, c.ctl + 4, t);
+        if (what == kTicketOver) return;
+        if (what == kTicketLast) break;
+        const int phase = (int)(t.n / pieces), v0 = (int)(t.n % pieces) * G;
+        bool stop = false;
+#pragma unroll 1
+        for (int vb = v0; vb < min(v0 + G, c.nt) && !stop; vb++) {
+            if (vb > v0) __syncthreads();  // (the shared memory of the tile before)
+            stop = (phase & 1) ? axpy_phase<TX, TY>(c, s, phase >> 1, false, ws, bc, vb)
+                               : spmv_phase<TX, TY, kStencil, true, true>(c, s, phase >> 1, false, sh, vb);
+        }
+        ticket_done(q);
+        if (!stop) continue;
+        if (v0 != 0) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // (thread 0 has written what all read now)
+        break;
+    }
+    __syncthreads();
+    if (finish) cg_finish_block(c, s, &bc);
 }
 
 // Region r of block b: blocks go to XCDs round-robin and each XCD takes a
@@ -1514,8 +1551,9 @@ struct ResidentShared {
     float bc;       // alpha or beta of the exchange just read
     int go;         // kGo, kStop, kBreakdown or kTimeout, after the same exchange
     int late;       // a halo vertex's z did not come
-    int team, rank;
+    int team;
 };
+constexpr int kTeamAll = 0, kTeamOpen = 1, kTeamOver = 2;
 constexpr int kGo = 0, kStop = 1, kBreakdown = 2, kTimeout = 4;
 
 // Up to here two assembly blocks per tile have a CU each.
@@ -1559,15 +1597,16 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
             SpmvShared<TX, TY> sp;
             float ws[NWT];
             float bc;
+            Ticket ticket;
         } t;
     };
     __shared__ Shared lds;
     SH& sh = lds.r;
     const int tid = threadIdx.x, lx = tid % TX, ly = tid / TX;
     // sign in, unless the solve is already done (a second solve of one
-    // assembly); all blocks read ctl[0] before any can finish
-    int rank = 0;
-    if (tid == 0) rank = c.ctl[0] ? -1 : roll_call_sign(c.sync + 1);
+    // assembly, or a block that starts after the others have finished it)
+    int done = 0;
+    if (tid == 0 && !(done = c.ctl[0])) roll_call_sign(c.sync + 1);
 
     const int N = c.N, nx = c.nx, ny = c.ny, ntx = c.ntx;
     const int reg = region_of_block(blockIdx.x, nb);
@@ -1737,23 +1776,18 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
     if (tid == 0) {
         sh.go = stopped() ? kStop : kGo;
         sh.late = 0;
-        sh.rank = rank;
-        sh.team = rank < 0 ? 0 : roll_call_wait(c.sync + 1, nb);
+        sh.team = done ? kTeamOver : roll_call_wait(c.sync + 1, nb) ? kTeamAll : kTeamOpen;
     }
     __syncthreads();
     const int team = sh.team;
-    rank = sh.rank;
-    if (rank < 0) return;
-    if (team < nb) {
+    if (team == kTeamOver) return;
+    if (team == kTeamOpen) {
         __syncthreads();  // (the shared words above have been read)
         if (VT == 1 && c.asm_rows) {  // every block for itself, all the same
             for (int k = tid; k < c.nt; k += NT) c.del_part[k] = row_partial(c, k);
             __syncthreads();
         }
-        if (tid >= TX * TY) return;
-        if (!cg_team<TX, TY, kStencil, true>(c, s, c.sync + 2, rank, team, lds.t.sp, lds.t.ws, lds.t.bc)) return;
-        __syncthreads();
-        if (finish && rank == 0) cg_finish_block(c, s, &lds.t.bc);
+        if (tid < TX * TY) cg_tickets<TX, TY, VT>(c, s, finish != 0, lds.t.sp, lds.t.ws, lds.t.bc, lds.t.ticket);
         return;
     }
 
@@ -1890,15 +1924,17 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
         go = sh.late ? kTimeout : last ? sh.go & kTimeout : sh.go;
     }
 
-    // the next solve's base: past the tags that were used, which every block
+    // The next solve's tags start past those that were used, which every block
     // has written over the older ones in the words (a solve that stops at once
-    // uses none; were the base to move on all the same, it could come round to
-    // tags that the words still hold)
-    if (blockIdx.x == 0 && tid == 0) c.sync[3] = base + 2u * (unsigned)it + (go == kGo || go == kStop ? 0u : 2u);
+    // uses none; were the start to move on all the same, it could come round to
+    // tags that the words still hold).
     if (go == kTimeout) {  // an exchange timed out: report it, leave dv as it was
         if (tid == 0) {
             __hip_atomic_fetch_or(c.ctl + 4, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (blockIdx.x == 0) c.ctl[0] = 1;
+            if (blockIdx.x == 0) {
+                c.ctl[0] = 1;
+                c.sync[3] = base + 2u * (unsigned)it + 2u;
+            }
         }
         return;
     }
@@ -1908,6 +1944,7 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
         // status bits follow as cg_finish_block derives them
         c.scal[0] = delta0;
         c.scal[it] = delta;
+        c.sync[3] = base + 2u * (unsigned)(go == kBreakdown ? it + 1 : it);
         c.ctl[0] = 1;
         c.ctl[1] = it;
         int st = c.ctl[2] | (go == kBreakdown ? OC_SOLVE_BREAKDOWN : 0);
@@ -1918,16 +1955,6 @@ __global__ __launch_bounds__(TX* HY) void k_cg_resident(DevCloth c, StepScalars 
         }
         c.ctl[2] = st;
     }
-}
-
-// All CG iterations of any topology in one cooperative launch (each resident
-// block serves tiles blockIdx.x, + gridDim.x, ...).
-template <int TX, int TY, int WP>
-__global__ __launch_bounds__(TX* TY) void k_cg_persistent(DevCloth c, StepScalars s, unsigned* bar) {
-    __shared__ SpmvShared<TX, TY> sh;
-    __shared__ float ws[TX * TY / 64];
-    __shared__ float bc;
-    (void)cg_team<TX, TY, WP, false>(c, s, bar, blockIdx.x, gridDim.x, sh, ws, bc);
 }
 
 __global__ void k_reset_barrier(unsigned* bar) {

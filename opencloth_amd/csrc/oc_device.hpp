@@ -137,6 +137,58 @@ __device__ inline void xch_store(uint64_t* p, unsigned i, unsigned tag, float v)
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Phases of `pieces` pieces of work each, for blocks that need not all be
+// running: a block takes the next ticket (phase by phase), waits until the
+// phases before its own are complete, does the piece and says so.  A ticket's
+// holder only waits for holders of earlier tickets, which are running, so any
+// number of blocks gets through, a single one too, and blocks that start late
+// take part from then on.  q[0]: tickets taken, q[kTicketDone]: pieces done (a
+// cache line of its own), both zero at the start.  *stop, set while a piece is done, ends the work in the next
+// phase at the latest.  A wait is bounded; on time-out *err is set and the
+// block leaves, so every wave exits.  A launch has fewer than 2^31 pieces.
+enum { kTicketWork, kTicketLast, kTicketOver };
+struct Ticket {
+    unsigned n;
+    int what;
+};
+constexpr unsigned kTicketPolls = 1u << 22;  // seconds
+// The block's next ticket t: a piece of work (t.n counts over all phases);
+// the one after the last piece, which a single block gets, once all are done;
+// or nothing more to do.  What other blocks wrote in earlier phases is visible.
+__device__ inline int ticket_take(unsigned* q, unsigned pieces, unsigned total, int* stop, int* err, Ticket& t) {
+    __syncthreads();  // t and the last piece's shared memory are free
+    if (threadIdx.x == 0) {
+        const unsigned n = __hip_atomic_fetch_add(q, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int what = n < total ? kTicketWork : n == total ? kTicketLast : kTicketOver;
+        auto stopped = [&]() { return stop && __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+        if (what != kTicketOver) {
+            unsigned polls = 0;
+            while (__hip_atomic_load(q + kTicketDone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n / pieces * pieces) {
+                if (stopped()) break;
+                if (++polls > kTicketPolls) {
+                    __hip_atomic_fetch_or(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    what = kTicketOver;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(8);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (stopped()) what = kTicketOver;
+        }
+        t.n = n;
+        t.what = what;
+    }
+    __syncthreads();
+    return t.what;
+}
+// The block's piece is done: its writes first (every wave's, then the release
+// takes them to the device-coherent level).
+__device__ inline void ticket_done(unsigned* q) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(q + kTicketDone, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Wave tree: lane l += lane l+off for off = 32..1; lane 0 ends with the sum
 // (the other lanes' values are not the tree's).  Offsets 32 and 16 by gfx950's
 // lane-swap instructions, the rest by row shifts inside 16 lanes: register

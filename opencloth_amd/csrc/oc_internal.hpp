@@ -233,8 +233,9 @@ struct DevCloth {
     // resident solve: tiles per block (0: not used), the exchange words
     // (resident_words of them) with xslots slots per set of partials and
     // xstride words from one copy of the partials to the next, and its
-    // control words: [0] epoch base of the tags, [1] roll call, [2] barrier
-    // counter of a partial team, [3] the next solve's epoch base
+    // control words: [0] epoch base of the tags, [1] roll call, [3] the next
+    // solve's epoch base, [kSyncTickets ...] the tickets of
+    // an incomplete team
     int res_vt;
     int xslots, xstride;
     uint64_t* xch;
@@ -245,6 +246,10 @@ struct DevCloth {
     float* row_part;
     int asm_rows;
 };
+
+// Control words of launches whose blocks wait for each other: a line of 128
+// bytes, then the tickets (oc_device.hpp), two counters in lines of their own.
+constexpr int kSyncTickets = 32, kTicketDone = 32, kSyncWords = 96;
 
 // Resident solve (k_cg_resident): one block per region of kTileX x (kTileY
 // tiles) vertices, one block per CU.  Registers hold a thread's pair blocks

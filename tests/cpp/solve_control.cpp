@@ -75,7 +75,7 @@ int main() {
             int ctl[8] = {done, done ? 2 : 0, 0, 0, 0, 0, 0, 0};
             float scal[2 * (its + 2)] = {9.0f, 4.0f, 1.0f, 0.0f}, part[(its + 1) * nt] = {};
             for (int k = 0; k < nt; k++) part[its * nt + k] = 0.5f;
-            unsigned sync[64] = {100u, 7u, 7u, 160u};
+            unsigned sync[oc::kSyncWords] = {100u, 7u, 7u, 160u};
             oc::DevCloth c;
             std::memset((void*)&c, 0, sizeof(c));
             c.nt = nt;
@@ -111,7 +111,7 @@ int main() {
             for (int t = 1; t < kThreads; t++) other += g_passed[t] != g_passed[0];
             const int status = done ? 0 : OC_SOLVE_NOT_CONVERGED;
             const bool right = ctl[0] == 0 && ctl[1] == 0 && ctl[2] == 0 && ctl[3] == status &&
-                               (!res || (sync[0] == 160u && sync[1] == 0u && sync[2] == 0u));
+                               (!res || (sync[0] == 160u && sync[1] == 0u && sync[oc::kSyncTickets] == 0u));
             std::printf("done %d resident %d: %d %d %d\n", done, res, g_passed[0], other, right ? 1 : 0);
         }
     return 0;
