@@ -87,8 +87,11 @@ oc::VerletScalars vscalars(const oc_verlet_s* v) {
 // win back at 4 to 8 us each (21x21, 7 steps 59 us one by one, 8 steps 46 us
 // in one launch); it is not recorded into graphs.
 constexpr int kResidentSteps = 4;
+// Steps of one launch: some 7 ms of the largest cloths, for which no other
+// stream's work gets the CUs.
+constexpr int kResidentMost = 1024;
 bool resident(const oc_verlet_s* v, int nsteps) {
-    if (!v->region || nsteps < kResidentSteps || nsteps >= (1 << 24)) return false;
+    if (!v->region || nsteps < kResidentSteps) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return oc::hip_ok(hipStreamIsCapturing(v->stream, &cap)) && cap == hipStreamCaptureStatusNone;
 }
@@ -258,16 +261,17 @@ int oc_verlet_step(oc_verlet v, int32_t nsteps, const oc_ellipsoid* e) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     if (nsteps < 0) return set_error(OC_ERR_INVALID_ARGUMENT, "nsteps < 0");
     const oc::VerletScalars s = vscalars(v);
-    if (resident(v, nsteps)) {
-        const unsigned span = 2u * (unsigned)nsteps + 2u;
+    while (resident(v, nsteps)) {
+        const int n = std::min(nsteps, kResidentMost);
+        const unsigned span = 2u * (unsigned)n + 2u;
         if (v->tag > UINT32_MAX - span) {  // all tags used: begin again on a clean exchange
             OC_HIP(hipMemsetAsync(v->xch, 0, sizeof(uint64_t) * 8 * (size_t)v->topo.N, v->stream));
             v->tag = 0;
         }
-        OC_HIP(oc::launch_verlet_resident(view(v), s, v->pos[v->cur], v->pos[v->last], v->region, nsteps, v->tag, e,
+        OC_HIP(oc::launch_verlet_resident(view(v), s, v->pos[v->cur], v->pos[v->last], v->region, n, v->tag, e,
                                           v->stream));
         v->tag += span;
-        return OC_OK;
+        nsteps -= n;
     }
     for (int k = 0; k < nsteps; k++) {
         oc::DevVerlet d = view(v);
