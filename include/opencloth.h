@@ -281,8 +281,9 @@ int oc_verlet_compute_forces(oc_verlet verlet, float* f_out);
  * Replaces StepPhysics of the Verlet demo (VL:557-562).  From four steps on,
  * a cloth in the reference's form of up to 512x512 runs them in one
  * cooperative launch (not while its stream is captured); should a wait
- * between the launch's blocks ever time out, the next oc_verlet_get_state
- * returns OC_ERR_DEVICE. */
+ * between the launch's blocks ever time out, the state is lost, and the calls
+ * that use it return OC_ERR_DEVICE until oc_verlet_set_state has been given
+ * both arrays. */
 int oc_verlet_step(oc_verlet verlet, int32_t nsteps, const oc_ellipsoid* ellipsoid);
 
 /* ---- grid Verlet: the GPU demos' kernel ---------------------------------- */

@@ -95,14 +95,19 @@ bool resident(const oc_verlet_s* v, int nsteps) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return oc::hip_ok(hipStreamIsCapturing(v->stream, &cap)) && cap == hipStreamCaptureStatusNone;
 }
-// Reported once, after the stream's work is done.
+// The blocks that ended without a word from the others have not stored their
+// part of the state, and those that had finished have: the error stays until
+// the caller has given both arrays of a new state.
 int resident_error(oc_verlet_s* v) {
     if (!v->err || !*(volatile int*)v->err) return OC_OK;
-    *v->err = 0;
-    return set_error(OC_ERR_DEVICE, "a wait between blocks of resident steps timed out");
+    return set_error(OC_ERR_DEVICE, "a wait between blocks of resident steps timed out; the state is lost");
 }
 
 }  // namespace
+
+namespace oc {
+int* verlet_error_word(oc_verlet_s* v) { return v->err; }
+}  // namespace oc
 
 extern "C" {
 
@@ -240,6 +245,7 @@ int oc_verlet_set_state(oc_verlet v, const float* x, const float* x_last) {
     const size_t N = (size_t)v->topo.N;
     OC_HIP(v->io.write({{x ? v->pos[v->cur] : nullptr, N, const_cast<float*>(x)},
                         {x_last ? v->pos[v->last] : nullptr, N, const_cast<float*>(x_last)}}, v->stream));
+    if (v->err && x && x_last) *v->err = 0;  // (the stream's work is done)
     return OC_OK;
 }
 
@@ -247,6 +253,7 @@ int oc_verlet_get_state(oc_verlet v, float* x, float* x_last) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     const size_t N = (size_t)v->topo.N;
     OC_HIP(v->io.read({{v->pos[v->cur], N, x}, {v->pos[v->last], N, x_last}}, v->stream));
+    if (!x && !x_last && v->tag) OC_HIP(hipStreamSynchronize(v->stream));  // (for the error word)
     return resident_error(v);
 }
 
@@ -254,12 +261,14 @@ int oc_verlet_compute_forces(oc_verlet v, float* f_out) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     OC_HIP(oc::launch_verlet_forces(view(v), vscalars(v), v->stream));
     if (f_out) OC_HIP(v->io.read({{v->f, (size_t)v->topo.N, f_out}}, v->stream));
-    return OC_OK;
+    return resident_error(v);
 }
 
 int oc_verlet_step(oc_verlet v, int32_t nsteps, const oc_ellipsoid* e) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     if (nsteps < 0) return set_error(OC_ERR_INVALID_ARGUMENT, "nsteps < 0");
+    const int rc = resident_error(v);  // (of steps that are done by now)
+    if (rc != OC_OK) return rc;
     const oc::VerletScalars s = vscalars(v);
     while (resident(v, nsteps)) {
         const int n = std::min(nsteps, kResidentMost);

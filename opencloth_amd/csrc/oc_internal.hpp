@@ -414,6 +414,7 @@ struct VerletScalars {
     float mass, gx, gy, gz, damping, dt;
     int flags;
 };
+int* verlet_error_word(::oc_verlet_s* v);  // NULL without resident steps
 hipError_t launch_verlet_forces(const DevVerlet& c, const VerletScalars& s, hipStream_t st);
 hipError_t launch_verlet_step(const DevVerlet& c, const VerletScalars& s, hipStream_t st);
 // Side of the square regions of a resident launch on the current device, 0

@@ -2,6 +2,9 @@
 //   launches: a call of many steps is split over launches of bounded length,
 //             with the same bits as shorter calls (the program counts the
 //             library's launches on their way to the runtime)
+//   lost:     after a wait between blocks that ended without its word (the
+//             program sets the error word itself), every call that uses the
+//             state says so until the caller has given a new one
 #include <dlfcn.h>
 
 #include <cmath>
@@ -102,9 +105,32 @@ static void launches() {
     }
 }
 
+static void lost() {
+    Cloth c(40, 30), fresh(40, 30);
+    int* const err = oc::verlet_error_word(c.v);
+    check("error word", 0, 0, err != nullptr);
+    if (!err) return;
+    auto says = [&](const char* name, int rc) { check(name, rc, OC_ERR_DEVICE, rc == OC_ERR_DEVICE); };
+    bool ok = oc_verlet_step(c.v, 8, &c.ball) == OC_OK && c.get();
+    *err = 1;
+    for (int k = 0; k < 2; k++) {  // not only once
+        says("get_state", oc_verlet_get_state(c.v, c.x.data(), c.xl.data()));
+        says("get_state of nothing", oc_verlet_get_state(c.v, nullptr, nullptr));
+        says("forces", oc_verlet_compute_forces(c.v, c.x.data()));
+        says("step", oc_verlet_step(c.v, 8, nullptr));
+        says("one step", oc_verlet_step(c.v, 1, nullptr));
+        ok = ok && (k ? oc_verlet_set_state(c.v, nullptr, c.x0.data()) : oc_verlet_set_state(c.v, c.x0.data(), nullptr)) == OC_OK;
+    }
+    // (half a state at a time is none; both arrays are)
+    ok = ok && oc_verlet_set_state(c.v, c.x0.data(), c.x0.data()) == OC_OK && oc_verlet_step(c.v, 20, &c.ball) == OC_OK &&
+         c.get() && oc_verlet_step(fresh.v, 20, &fresh.ball) == OC_OK && fresh.get();
+    check("a new state", 0, 0, ok && c.same(fresh));
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "launches") launches();
+    else if (what == "lost") lost();
     else return 99;
     std::printf("wrong %d\n", g_wrong);
     return g_wrong;

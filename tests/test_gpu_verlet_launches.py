@@ -1,5 +1,6 @@
 """The resident Verlet steps from inside (tests/cpp/verlet_resident.cpp): how a
-call of many steps is split over launches."""
+call of many steps is split over launches, and what the calls say after a wait
+between blocks has ended without its word."""
 import os
 import subprocess
 
@@ -34,3 +35,7 @@ def run(exe, what):
 
 def test_long_calls_are_split(exe):
     assert len(run(exe, "launches")) == 2
+
+
+def test_a_lost_state_is_reported_until_it_is_replaced(exe):
+    assert len(run(exe, "lost")) == 1 + 2 * 5 + 1
