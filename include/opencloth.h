@@ -279,9 +279,10 @@ int oc_verlet_compute_forces(oc_verlet verlet, float* f_out);
 /* nsteps of ComputeForces + IntegrateVerlet (VL:428-444) fused per vertex,
  * then the ellipsoid pass (x_last = x on contact, VL:509-533) when given.
  * Replaces StepPhysics of the Verlet demo (VL:557-562).  From four steps on,
- * a cloth in the reference's form of up to 512x512 runs them in one
- * cooperative launch (not while its stream is captured); should a wait
- * between the launch's blocks ever time out, the state is lost, and the calls
+ * a cloth in the reference's form of up to 512x512 runs them in launches of
+ * up to 1024 steps (not while its stream is captured), whose blocks wait up to
+ * 1 ms for each other and otherwise go on, slower, with those that get a CU;
+ * should a later wait between them ever time out, the state is lost, and the calls
  * that use it return OC_ERR_DEVICE until oc_verlet_set_state has been given
  * both arrays. */
 int oc_verlet_step(oc_verlet verlet, int32_t nsteps, const oc_ellipsoid* ellipsoid);

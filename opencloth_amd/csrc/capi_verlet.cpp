@@ -41,6 +41,8 @@ struct oc_verlet_s {
     float* cst = nullptr;
     int region = 0;            // side of the resident steps' regions, 0: none
     uint64_t* xch = nullptr;   // their exchange words
+    unsigned* sync = nullptr;  // and control words
+    int set = 0;               // the next launch's
     int* err = nullptr;        // and their pinned error word
     unsigned tag = 0;          // the last launch's tags end here
 };
@@ -67,6 +69,7 @@ oc::DevVerlet view(const oc_verlet_s* v) {
     d.cst = v->cst;
     d.stencil_asm = v->asm_mask ? 1 : 0;
     d.xch = v->xch;
+    d.sync = v->sync;
     d.err = v->err;
     return d;
 }
@@ -83,13 +86,11 @@ oc::VerletScalars vscalars(const oc_verlet_s* v) {
     return s;
 }
 
-// A cooperative launch takes some 16 us more than the others, which its steps
-// win back at 4 to 8 us each (21x21, 7 steps 59 us one by one, 8 steps 46 us
-// in one launch); it is not recorded into graphs.
+// A launch for all steps takes longer to begin than one for a single step,
+// and wins back 4 to 8 us with each (21x21: three steps 37 us one by one, four
+// 36 us in one launch; 512x512: 56 and 50).  Its tags come from the host, so
+// it is not recorded into graphs.
 constexpr int kResidentSteps = 4;
-// Steps of one launch: some 7 ms of the largest cloths, for which no other
-// stream's work gets the CUs.
-constexpr int kResidentMost = 1024;
 bool resident(const oc_verlet_s* v, int nsteps) {
     if (!v->region || nsteps < kResidentSteps) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -106,7 +107,23 @@ int resident_error(oc_verlet_s* v) {
 }  // namespace
 
 namespace oc {
+
 int* verlet_error_word(oc_verlet_s* v) { return v->err; }
+
+int verlet_steps_resident(oc_verlet_s* v, int nsteps, const oc_ellipsoid* e, int blocks) {
+    if (!v->region) return set_error(OC_ERR_INVALID_ARGUMENT, "no resident steps for this cloth");
+    const unsigned span = 2u * (unsigned)nsteps + 2u;
+    if (v->tag > UINT32_MAX - span) {  // all tags used: begin again on a clean exchange
+        OC_HIP(hipMemsetAsync(v->xch, 0, sizeof(uint64_t) * 8 * (size_t)v->topo.N, v->stream));
+        v->tag = 0;
+    }
+    OC_HIP(launch_verlet_resident(view(v), vscalars(v), v->pos[v->cur], v->pos[v->last], v->region, nsteps, v->tag, v->set,
+                                  e, blocks, v->stream));
+    v->tag += span;
+    v->set = 1 - v->set;
+    return OC_OK;
+}
+
 }  // namespace oc
 
 extern "C" {
@@ -145,7 +162,8 @@ int oc_verlet_create(int32_t nx, int32_t ny, const float* x0, const float* x_las
     const size_t cst = st_asm ? align_up(sizeof(float) * oc::kCstPlanes * N) : 0;
     const int region = st_asm ? oc::verlet_resident_region(nx, ny, t.asm_mask.data()) : 0;
     const size_t xch = region ? align_up(sizeof(uint64_t) * 8 * N) : 0;
-    const size_t total = 4 * vec + align_up(N) + as + am + 3 * sp + amask + cst + xch;
+    const size_t sync = region ? align_up(sizeof(unsigned) * 2 * oc::kSyncWords) : 0;
+    const size_t total = 4 * vec + align_up(N) + as + am + 3 * sp + amask + cst + xch + sync;
     if (hipMalloc(&v->arena, total) != hipSuccess) {
         delete v;
         return set_error(OC_ERR_OUT_OF_MEMORY, "hipMalloc failed");
@@ -179,6 +197,7 @@ int oc_verlet_create(int32_t nx, int32_t ny, const float* x0, const float* x_las
         *v->err = 0;
         v->region = region;
         v->xch = (uint64_t*)p;
+        v->sync = (unsigned*)(p + xch);
     }
     std::vector<float> L0(S, 0.0f), ks(S, 0.0f), kd(S, 0.0f);
     for (int s = 0; s < t.S; s++) {
@@ -267,21 +286,14 @@ int oc_verlet_compute_forces(oc_verlet v, float* f_out) {
 int oc_verlet_step(oc_verlet v, int32_t nsteps, const oc_ellipsoid* e) {
     if (!v) return set_error(OC_ERR_INVALID_ARGUMENT, "verlet is NULL");
     if (nsteps < 0) return set_error(OC_ERR_INVALID_ARGUMENT, "nsteps < 0");
-    const int rc = resident_error(v);  // (of steps that are done by now)
+    int rc = resident_error(v);  // (of steps that are done by now)
     if (rc != OC_OK) return rc;
-    const oc::VerletScalars s = vscalars(v);
     while (resident(v, nsteps)) {
-        const int n = std::min(nsteps, kResidentMost);
-        const unsigned span = 2u * (unsigned)n + 2u;
-        if (v->tag > UINT32_MAX - span) {  // all tags used: begin again on a clean exchange
-            OC_HIP(hipMemsetAsync(v->xch, 0, sizeof(uint64_t) * 8 * (size_t)v->topo.N, v->stream));
-            v->tag = 0;
-        }
-        OC_HIP(oc::launch_verlet_resident(view(v), s, v->pos[v->cur], v->pos[v->last], v->region, n, v->tag, e,
-                                          v->stream));
-        v->tag += span;
+        const int n = std::min(nsteps, oc::kVerletMost);
+        if ((rc = oc::verlet_steps_resident(v, n, e, 0)) != OC_OK) return rc;
         nsteps -= n;
     }
+    const oc::VerletScalars s = vscalars(v);
     for (int k = 0; k < nsteps; k++) {
         oc::DevVerlet d = view(v);
         OC_HIP(oc::launch_verlet_step(d, s, v->stream));

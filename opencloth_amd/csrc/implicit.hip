@@ -1401,36 +1401,7 @@ __global__ __launch_bounds__(TX* TY) void k_cg_axpy(DevCloth c, StepScalars s, i
 // 2.4 us among 256 (store to the coherence point, then polled loads of 512
 // words); the rest at 512x512, 2.9 us, is the arithmetic: 16 waves per CU
 // issue about 200 instructions each per iteration.
-constexpr unsigned kRollClosed = 1u << 15;       // the count is in bits 0-14
-// How long blocks wait for the others: about what an incomplete team takes
-// longer than a complete one (512x512, 30 iterations: 0.24 ms complete, 1.75
-// by tickets with half of the blocks or all but one; 128x128, 40 iterations:
-// 0.17 and 0.7).  Beside another stream's products that leave CUs only now and
-// then, a 512x512 step takes 0.82 ms; with half the wait, and without the late
-// blocks, it took 1.95.
-constexpr unsigned long long kRollCallTicks = 100000;  // 1 ms of the 100 MHz counter
 constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
-
-// Sign in (one thread per block), then wait until all nb blocks have: true
-// once they have, false when the roll is closed.  The word decides: a close
-// only succeeds on a word whose count is below nb, and once the count has
-// reached nb no block closes it.
-__device__ inline void roll_call_sign(unsigned* roll) {
-    __hip_atomic_fetch_add(roll, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline bool roll_call_wait(unsigned* roll, int nb) {
-    const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
-    for (;;) {
-        unsigned w = __hip_atomic_load(roll, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (w & kRollClosed) return false;
-        if ((int)w >= nb) return true;
-        if (__builtin_amdgcn_s_memrealtime() - t0 > kRollCallTicks)
-            __hip_atomic_compare_exchange_strong(roll, &w, w | kRollClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-        else
-            __builtin_amdgcn_s_sleep(1);
-    }
-}
 
 // Grid barrier of the persistent solve's blocks: every block adds 1 to *bar and waits until it reaches target.  The add is a
 // release (the block's writes reach the device-coherent level first); the

@@ -405,9 +405,11 @@ struct DevVerlet {
     const uint32_t* asm_mask;
     const float* cst;
     int stencil_asm;
-    // resident steps: two sets of 4 words per vertex, and a host word set
-    // when a wait for one ended without it
+    // resident steps: two sets of 4 words per vertex, two sets of control
+    // words ([1] roll call, [kSyncTickets ...] tickets), and a host word set
+    // when a wait ended without its word
     uint64_t* xch;
+    unsigned* sync;
     int* err;
 };
 struct VerletScalars {
@@ -420,11 +422,18 @@ hipError_t launch_verlet_step(const DevVerlet& c, const VerletScalars& s, hipStr
 // Side of the square regions of a resident launch on the current device, 0
 // when the cloth (mask: its asm_mask) does not fit it.
 int verlet_resident_region(int nx, int ny, const uint32_t* mask);
-// nsteps >= 2 steps of c.x and c.xl with the collider (e may be NULL) in one
-// cooperative launch; the results go to x and xl, which may be c.x and c.xl.
-// The tags base + 2 .. base + 2 nsteps (base even) must not be in c.xch.
+// Steps of one launch: some 7 ms of the largest cloths, for which no other
+// stream's work gets the CUs.
+constexpr int kVerletMost = 1024;
+// 2 to kVerletMost steps of x and xl (c.x and c.xl) in place with the collider
+// (e may be NULL) in one launch.  The tags base + 2 .. base + 2 nsteps (base
+// even) must not be in c.xch.  set: 0 and 1 in turn, from launch to launch.
+// blocks: 0, or fewer than there are regions, to run the incomplete team's
+// code.
 hipError_t launch_verlet_resident(const DevVerlet& c, const VerletScalars& s, float* x, float* xl, int region, int nsteps,
-                                  unsigned base, const oc_ellipsoid* e, hipStream_t st);
+                                  unsigned base, int set, const oc_ellipsoid* e, int blocks, hipStream_t st);
+// The same of a handle with resident steps.
+int verlet_steps_resident(::oc_verlet_s* v, int nsteps, const oc_ellipsoid* e, int blocks);
 
 // Grid Verlet (grid_verlet.hip): the reference's GPU Verlet kernel on a
 // width x height grid with a fixed 12-neighbour stencil.  Two position sets

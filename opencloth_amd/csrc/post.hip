@@ -122,25 +122,32 @@ struct VerletShared {
     float wv[3][WY][WX];
 };
 
-// Force on the tile's vertex (VL:448-484): gravity on free vertices, damping
+// A vertex's next position (VL:428-444).
+__device__ __forceinline__ V3 verlet_next(const VerletScalars& s, V3 xi, V3 xl, V3 F) {
+    const float c2 = (s.dt * s.dt) / s.mass;
+    V3 xn = {xi.x + (xi.x - xl.x) + c2 * F.x, xi.y + (xi.y - xl.y) + c2 * F.y, xi.z + (xi.z - xl.z) + c2 * F.z};
+    if ((s.flags & OC_FLAG_GROUND_CLAMP) && xn.y < 0.0f) xn.y = 0.0f;
+    return xn;
+}
+
+// Force on vertex t of a tile (VL:448-484): gravity on free vertices, damping
 // on all, springs in list order (pinned vertices: damping only).  Springs are
 // evaluated from this vertex's side (x1 = x_i), which is bitwise the negated
-// p1-side force, so it is always added.  FORCES: write the force; otherwise
-// integrate (VL:428-444) into the next positions.
+// p1-side force, so it is always added.  out(i, x_i, F) takes it; a tile past
+// the last has no vertices.
 // STENCIL: the topology has the stencil assembly form; a vertex's springs
 // come from its ownership mask in stencil order (the slot order on such
 // topologies) and their constants from the owner planes at the pair's lower
 // vertex, so no slot table or spring-id gather is read.
-template <int TX, int TY, int WA, bool FORCES, bool STENCIL>
-__global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s) {
+template <int TX, int TY, int WA, bool STENCIL, class Out>
+__device__ __forceinline__ void verlet_tile(const DevVerlet& c, const VerletScalars& s, VerletShared<TX, TY>& sh, int tile,
+                                            int t, const Out& out) {
     constexpr int NT = TX * TY, H = kHalo;
     constexpr int WX = TX + 2 * H, WY = TY + 2 * H;
     constexpr int NWIN = (WX * WY + NT - 1) / NT;
-    __shared__ VerletShared<TX, TY> sh;
-    const int ntx = (c.nx + TX - 1) / TX, nt = ntx * ((c.ny + TY - 1) / TY);
-    const int tile = tile_of_block(blockIdx.x, nt);
+    const int ntx = (c.nx + TX - 1) / TX;
     const int bx = tile % ntx, by = tile / ntx;
-    const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
+    const int lx = t % TX, ly = t / TX;
     const int gi = bx * TX + lx, gj = by * TY + ly;
     const bool own = gi < c.nx && gj < c.ny;
     const int N = c.N, i = gj * c.nx + gi;
@@ -159,7 +166,7 @@ __global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s)
     const int x0 = bx * TX - H, y0 = by * TY - H;
 #pragma unroll
     for (int n = 0; n < NWIN; n++) {
-        const int idx = threadIdx.x + n * NT;
+        const int idx = t + n * NT;
         if (idx < WX * WY) {
             const int wx = idx % WX, wy = idx / WX;
             const int gx = x0 + wx, gy = y0 + wy;
@@ -213,17 +220,25 @@ __global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s)
             F = add3(F, spring_force(xi, xj, vi, vj, c.L0[sp], c.ks[sp], c.kd[sp]));
         }
     }
-    if (FORCES) {
-        st3(c.f, N, i, F);
-        return;
-    }
-    const float c2 = (s.dt * s.dt) / s.mass;
-    const V3 xl = ld3(c.xl, N, i);
-    V3 xn = {xi.x + (xi.x - xl.x) + c2 * F.x, xi.y + (xi.y - xl.y) + c2 * F.y,
-             xi.z + (xi.z - xl.z) + c2 * F.z};
-    if ((s.flags & OC_FLAG_GROUND_CLAMP) && xn.y < 0.0f) xn.y = 0.0f;
-    st3(c.xn, N, i, xn);
+    out(i, xi, F);
 }
+
+// One step of all vertices, or (FORCES) their forces.
+template <int TX, int TY, int WA, bool FORCES, bool STENCIL>
+__global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s) {
+    __shared__ VerletShared<TX, TY> sh;
+    const int nt = ((c.nx + TX - 1) / TX) * ((c.ny + TY - 1) / TY);
+    verlet_tile<TX, TY, WA, STENCIL>(c, s, sh, tile_of_block(blockIdx.x, nt), threadIdx.x, [&](int i, V3 xi, V3 F) {
+        if constexpr (FORCES)
+            st3(c.f, c.N, i, F);
+        else
+            st3(c.xn, c.N, i, verlet_next(s, xi, ld3(c.xl, c.N, i), F));
+    });
+}
+
+// The Verlet step has no reduction, so its tile shape is free: 32x8 measured
+// faster than the implicit kernels' 64x8 at 512x512 (15.5 against 17.4 us).
+constexpr int kVerletTileX = 32, kVerletTileY = 8;
 
 // ---------------------------------------------------------------------------
 // resident Verlet: many steps in one launch, the cloth in registers and LDS
@@ -242,9 +257,12 @@ __global__ __launch_bounds__(TX* TY) void k_verlet(DevVerlet c, VerletScalars s)
 // these publish that only after they have read its step n, so two sets of
 // words are enough.  The tag's low bit tells that the collider moved the
 // vertex (its previous position is then the position itself; else the reader
-// knows it).  Blocks wait for each other, so the launch is cooperative; a
-// wait is bounded, and one that ends without its word sets *err and every
-// block leaves.
+// knows it).  Blocks wait for each other, so all must run: there is one per CU
+// at most, and they call the roll first.  Where other work holds CUs for too
+// long, the roll is closed and every block, those that start later too, takes
+// tiles of whole steps in memory by tickets, so the steps are done in any case.
+// After a complete roll every wait ends; each is bounded all the same, and one
+// that ends without its word sets *err and every block leaves.
 //
 // Measured per step of 200, with the collider, a launch each for step and
 // collider before: 512x512 14.2 -> 6.5 us, 256x256 12 -> 4.6, 21x21 8.4 ->
@@ -262,14 +280,69 @@ struct VerletRegion {
     static constexpr size_t lds = sizeof(float) * (6 * NW + 18 * NT + 3 * NT);
 };
 
+// What steps by tickets take: the arguments of k_verlet_resident again, as
+// arguments of their own.  (Shared, they stay in scalar registers from the
+// kernel's start, and what a resident step needs is moved out of them.)
+struct VerletTickets {
+    DevVerlet c;
+    VerletScalars s;
+    float* x;
+    float* xl;
+    oc_ellipsoid e;
+    int has_e, nsteps;
+    unsigned* q;
+};
+
+// The steps by tickets, G tiles per ticket (a thread per vertex), from the
+// state x, xl to c.xn, c.f and back; after an odd number a last phase copies.
+template <int T>
+__device__ inline void verlet_tickets(const VerletTickets& a, float* lds, Ticket& t) {
+    constexpr int TX = kVerletTileX, TY = kVerletTileY, G = T * T / (TX * TY);
+    static_assert(G >= 1 && G * sizeof(VerletShared<TX, TY>) <= VerletRegion<T>::lds, "a window per tile");
+    VerletShared<TX, TY>* const sh = reinterpret_cast<VerletShared<TX, TY>*>(lds) + threadIdx.x / (TX * TY);
+    const int nt = ((a.c.nx + TX - 1) / TX) * ((a.c.ny + TY - 1) / TY), N = a.c.N;
+    const unsigned pieces = (unsigned)(nt + G - 1) / G, total = (unsigned)(a.nsteps + (a.nsteps & 1)) * pieces;
+    while (ticket_take(a.q, pieces, total, nullptr, a.c.err, t) == kTicketWork) {
+        const int n = (int)(t.n / pieces), tile = (int)(t.n % pieces) * G + (int)threadIdx.x / (TX * TY);
+        const bool odd = n & 1;
+        DevVerlet d = a.c;
+        d.x = odd ? a.c.xn : a.x;
+        d.xl = odd ? a.c.f : a.xl;
+        float* const to = odd ? a.x : a.c.xn;
+        float* const tol = odd ? a.xl : a.c.f;
+        verlet_tile<TX, TY, 1, true>(d, a.s, *sh, tile, threadIdx.x % (TX * TY), [&](int i, V3 xi, V3 F) {
+            V3 p = xi, last = ld3(d.xl, N, i);
+            if (n < a.nsteps) {
+                bool moved = false;
+                p = verlet_next(a.s, xi, last, F);
+                if (a.has_e) p = ellipsoid_push(a.e, p, moved);
+                last = moved ? p : xi;
+            }
+            st3(to, N, i, p);
+            st3(tol, N, i, last);
+        });
+        ticket_done(a.q);
+    }
+}
+
+// set: which of the two sets of control words (c.sync) this launch uses; it
+// clears the other, which the launch before has left.  nb: the regions.
 template <int T>
 __global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletScalars s, float* xo, float* xlo, int nsteps,
-                                                          unsigned base, oc_ellipsoid e, int has_e) {
+                                                          unsigned base, oc_ellipsoid e, int has_e, int set, int nb,
+                                                          VerletTickets rest) {
     using R = VerletRegion<T>;
     constexpr int NT = R::NT, H = R::H, W = R::W, NW = R::NW, NS = R::NS;
     static_assert(R::NJ > 0 && 4 * R::NJ <= 18 * NT, "one extra spring per thread, room for their list");
     extern __shared__ float lds[];
-    __shared__ int lost, jobs;
+    __shared__ int lost, jobs, all;
+    __shared__ Ticket ticket;
+    unsigned* const ctl = c.sync + set * kSyncWords;
+    if (threadIdx.x == 0) {
+        roll_call_sign(ctl + 1);
+        unsigned* const other = c.sync + (1 - set) * kSyncWords;
+        if (blockIdx.x == 0) other[1] = other[kSyncTickets] = other[kSyncTickets + kTicketDone] = 0;
+    }
     float* const wx = lds;           // 3 planes of the window: positions
     float* const wv = lds + 3 * NW;  // velocities
     float* const fo = lds + 6 * NW;  // 18 planes of NT: force of own spring o, component c at plane 3 o + c
@@ -398,9 +471,28 @@ __global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletSca
         hdst[q] = comp * NW + py * W + px;
     }
     const bool rim = own && (lx < H || lx >= T - H || ly < H || ly >= T - H);
-    const float c2 = (s.dt * s.dt) / s.mass;
     auto win = [&](const float* p, int a) { return V3{p[a], p[NW + a], p[2 * NW + a]}; };
 
+    if (tid == 0) all = roll_call_wait(ctl + 1, nb);
+    __syncthreads();
+    if (!__builtin_amdgcn_readfirstlane(all)) {
+        verlet_tickets<T>(rest, lds, ticket);
+        return;
+    }
+
+    // What the steps take from outside is too much for the scalar registers.
+    // One wave per SIMD (T = 16) loses least by testing the mask's bits anew
+    // (here) and loading the collider's numbers in every step: 21x21 3.62 us a
+    // step, 3.71 with the bits' 24 conditions and the numbers kept and spilled;
+    // with four (T = 32), it is the other way round: 512x512 6.44 and 6.35.
+    oc_ellipsoid ball = e;
+    if constexpr (T == 32) {
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            if (k % 4 < 3) asm volatile("" : "+s"(ball.inverse[k]));
+#pragma unroll
+        for (int k = 0; k < 3; k++) asm volatile("" : "+s"(ball.center[k]));
+    }
     for (int n = 0; n < nsteps; n++) {
         __syncthreads();  // the window is complete
         if (lost) return;
@@ -426,9 +518,10 @@ __global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletSca
         F = {F.x + s.damping * vi.x, F.y + s.damping * vi.y, F.z + s.damping * vi.z};
         if (!pinned) {
             unsigned q = second;
+            const unsigned bits = T == 16 ? here(mi) : mi;
 #pragma unroll
             for (int k = 0; k < kStencil; k++) {
-                if (!((mi >> k) & 1u)) continue;
+                if (!((bits >> k) & 1u)) continue;
                 const int o = owned_index(k);
                 if (stencil_owner(k)) {
                     F = add3(F, f[o]);
@@ -436,18 +529,17 @@ __global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletSca
                     const float* p = part[o] >= 0 ? fo + part[o] : fs + ~part[o];
                     F = sub3(F, V3{p[0], p[NT], p[2 * NT]});
                 }
-                if ((mi >> (16 + k)) & 1u) {
+                if ((bits >> (16 + k)) & 1u) {
                     const float* p = fs + (q & 0xFFFFu);
                     F = add3(F, V3{p[0], p[NT], p[2 * NT]});
                     q >>= 16;
                 }
             }
         }
-        V3 xn = {xi.x + (xi.x - xl.x) + c2 * F.x, xi.y + (xi.y - xl.y) + c2 * F.y, xi.z + (xi.z - xl.z) + c2 * F.z};
-        if ((s.flags & OC_FLAG_GROUND_CLAMP) && xn.y < 0.0f) xn.y = 0.0f;
+        V3 xn = verlet_next(s, xi, xl, F);
         xl = xi;
         bool moved = false;
-        if (has_e) xn = ellipsoid_push(e, xn, moved);
+        if (has_e) xn = ellipsoid_push(ball, xn, moved);
         if (moved) xl = xn;
         xi = xn;
         if (n + 1 == nsteps) break;
@@ -488,10 +580,6 @@ __global__ __launch_bounds__(T* T) void k_verlet_resident(DevVerlet c, VerletSca
     }
 }
 
-// The Verlet step has no reduction, so its tile shape is free: 32x8 measured
-// faster than the implicit kernels' 64x8 at 512x512 (15.5 against 17.4 us).
-constexpr int kVerletTileX = 32, kVerletTileY = 8;
-
 template <bool FORCES>
 hipError_t launch_verlet(const DevVerlet& c, const VerletScalars& s, hipStream_t st) {
     constexpr int TX = kVerletTileX, TY = kVerletTileY;
@@ -519,12 +607,11 @@ hipError_t launch_provot(const DevCloth& c, float slack, hipStream_t st) {
     return hipGetLastError();
 }
 
-// CUs, if a region's block fits one and cooperative launches are there.
+// CUs, if a region's block fits one.
 template <int T>
 static int verlet_blocks_fit() {
-    int dev = 0, coop = 0, cus = 0, per_cu = 0, lds = 0;
-    if (!hip_ok(hipGetDevice(&dev)) || !hip_ok(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev)) ||
-        !coop || !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) ||
+    int dev = 0, cus = 0, per_cu = 0, lds = 0;
+    if (!hip_ok(hipGetDevice(&dev)) || !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) ||
         !hip_ok(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) ||
         VerletRegion<T>::lds + 64 > (size_t)lds ||
         !hip_ok(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_verlet_resident<T>, T * T, VerletRegion<T>::lds)))
@@ -561,17 +648,21 @@ int verlet_resident_region(int nx, int ny, const uint32_t* mask) {
 }
 
 hipError_t launch_verlet_resident(const DevVerlet& c, const VerletScalars& s, float* x, float* xl, int T, int nsteps,
-                                  unsigned base, const oc_ellipsoid* e, hipStream_t st) {
-    if ((T != 16 && T != 32) || nsteps < 2 || (base & 1u) || !c.stencil_asm) return hipErrorInvalidValue;
-    DevVerlet ca = c;
-    VerletScalars sa = s;
-    oc_ellipsoid el = e ? *e : oc_ellipsoid{};
-    int has_e = e != nullptr;
-    void* args[] = {&ca, &sa, &x, &xl, &nsteps, &base, &el, &has_e};
-    const void* k = T == 16 ? reinterpret_cast<const void*>(k_verlet_resident<16>)
-                            : reinterpret_cast<const void*>(k_verlet_resident<32>);
-    const size_t lds = T == 16 ? VerletRegion<16>::lds : VerletRegion<32>::lds;
-    return hipLaunchCooperativeKernel(k, dim3(verlet_regions(c.nx, c.ny, T)), dim3(T * T), args, (unsigned)lds, st);
+                                  unsigned base, int set, const oc_ellipsoid* e, int blocks, hipStream_t st) {
+    const int nb = verlet_regions(c.nx, c.ny, T == 16 ? 16 : 32);
+    if ((T != 16 && T != 32) || nsteps < 2 || nsteps > kVerletMost || (base & 1u) || !c.stencil_asm || x != c.x ||
+        xl != c.xl || (set & ~1) || blocks < 0 || blocks > nb)
+        return hipErrorInvalidValue;
+    const oc_ellipsoid el = e ? *e : oc_ellipsoid{};
+    const dim3 grid(blocks ? blocks : nb), block(T * T);
+    const VerletTickets rest = {c, s, x, xl, el, e != nullptr, nsteps, c.sync + set * kSyncWords + kSyncTickets};
+    if (T == 16)
+        hipLaunchKernelGGL(k_verlet_resident<16>, grid, block, VerletRegion<16>::lds, st, c, s, x, xl, nsteps, base, el,
+                           e != nullptr, set, nb, rest);
+    else
+        hipLaunchKernelGGL(k_verlet_resident<32>, grid, block, VerletRegion<32>::lds, st, c, s, x, xl, nsteps, base, el,
+                           e != nullptr, set, nb, rest);
+    return hipGetLastError();
 }
 
 hipError_t launch_verlet_forces(const DevVerlet& c, const VerletScalars& s, hipStream_t st) {

@@ -2,6 +2,9 @@
 //   launches: a call of many steps is split over launches of bounded length,
 //             with the same bits as shorter calls (the program counts the
 //             library's launches on their way to the runtime)
+//   teams:    steps of resident launches against single steps, with every
+//             block and with fewer than there are regions, so that the roll
+//             never fills and the steps are done by tickets
 //   lost:     after a wait between blocks that ended without its word (the
 //             program sets the error word itself), every call that uses the
 //             state says so until the caller has given a new one
@@ -127,10 +130,33 @@ static void lost() {
     check("a new state", 0, 0, ok && c.same(fresh));
 }
 
+static void teams() {
+    const int sizes[][2] = {{21, 21}, {33, 17}, {130, 100}, {256, 256}, {257, 250}, {512, 512}};
+    for (const auto& n : sizes) {
+        Cloth one(n[0], n[1]), team(n[0], n[1]);
+        const int T = n[0] * n[1] > 256 * 256 || n[0] > 256 ? 32 : 16;
+        const int nb = ((n[0] + T - 1) / T) * ((n[1] + T - 1) / T);
+        // (0: all of them; teams in turn, so that each set of control words is used after the other)
+        for (int blocks : {0, 1, nb / 2, 0, 0, nb - 1, 1}) {
+            if (blocks == 0 && nb < 1) continue;
+            for (int steps : {2, 5, 4}) {
+                const oc_ellipsoid* const e = steps == 4 ? nullptr : &one.ball;
+                bool ok = oc::verlet_steps_resident(team.v, steps, e, blocks) == OC_OK;
+                for (int k = 0; k < steps; k++) ok = ok && oc_verlet_step(one.v, 1, e) == OC_OK;
+                ok = ok && one.get() && team.get();
+                check(("team of " + std::to_string(blocks)).c_str(), n[0], n[1], ok && one.same(team));
+            }
+        }
+        check("calls", n[0], n[1], oc_verlet_step(one.v, 12, &one.ball) == OC_OK && oc_verlet_step(team.v, 3, &one.ball) == OC_OK &&
+                                       oc_verlet_step(team.v, 9, &one.ball) == OC_OK && one.get() && team.get() && one.same(team));
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "launches") launches();
     else if (what == "lost") lost();
+    else if (what == "teams") teams();
     else return 99;
     std::printf("wrong %d\n", g_wrong);
     return g_wrong;

@@ -1,6 +1,7 @@
 """The resident Verlet steps from inside (tests/cpp/verlet_resident.cpp): how a
-call of many steps is split over launches, and what the calls say after a wait
-between blocks has ended without its word."""
+call of many steps is split over launches, complete and incomplete teams of
+blocks (the resident route is the one that runs: it refuses other cloths), and
+what the calls say after a wait between blocks has ended without its word."""
 import os
 import subprocess
 
@@ -39,3 +40,8 @@ def test_long_calls_are_split(exe):
 
 def test_a_lost_state_is_reported_until_it_is_replaced(exe):
     assert len(run(exe, "lost")) == 1 + 2 * 5 + 1
+
+
+def test_complete_and_incomplete_teams(exe):
+    lines = run(exe, "teams")
+    assert len(lines) == 6 * (7 * 3 + 1)
