@@ -50,6 +50,7 @@ struct oc_cloth_s {
     float* alt_v = nullptr;  // then the two sets swap
     int32_t* spring_cst = nullptr;  // stencil assembly form: owner-plane index per spring
     bool assembled = false;
+    bool captured = false;  // steps have been recorded into a graph
     // differentiable rollouts: checkpoints, one segment of states, adjoint vectors
     oc::RolloutStore roll;
 };
@@ -172,7 +173,14 @@ int cloth_step(oc_cloth_s* c, int nsteps, float* partials) {
     // also records the solve's status, is a launch of its own.  A cold start
     // is not fused: its assembly zeroes dv, which neighbouring blocks of a
     // fused assembly would still be reading for the update.
+    // Each fused update ends in the other pair of x and v.  A graph's replay
+    // starts and ends where its capture did, so from the first capture on, of
+    // an even number of steps, whose updates would be an odd number, the first
+    // is a launch of its own.
     const bool fuse = s.warm && s.max_it >= 1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hip_ok(hipStreamIsCapturing(c->stream, &cap)) && cap != hipStreamCaptureStatusNone) c->captured = true;
+    const bool apart = fuse && c->captured && nsteps % 2 == 0;
     d.asm_rows = assembles_rows(d, s);
     bool pending = false;  // a solve whose update has not been launched yet
     hipError_t e = hipSuccess;
@@ -189,7 +197,7 @@ int cloth_step(oc_cloth_s* c, int nsteps, float* partials) {
             break;
         }
         if ((e = launch_cg(d, s, c->stream, false)) != hipSuccess) break;
-        if (fuse) {
+        if (fuse && !(apart && k == 0)) {
             pending = true;
             continue;
         }
