@@ -43,18 +43,19 @@ float k_prime(float k, int ns) {
 // does not change the result, and neighbouring lanes then read neighbouring
 // particles (the reference lists column constraints column by column, which
 // in list order would put a whole grid row between neighbouring lanes).
-void bucket(int n, int arity, const std::vector<int32_t>& p, const std::vector<int>& col, int ncol,
+void bucket(int N, int n, int arity, const std::vector<int32_t>& p, const std::vector<int>& col, int ncol,
             std::vector<int32_t>& order, std::vector<int32_t>& ptr) {
     ptr.assign((size_t)ncol + 1, 0);
     for (int c = 0; c < n; c++) ptr[col[c] + 1]++;
     for (int k = 0; k < ncol; k++) ptr[k + 1] += ptr[k];
+    // by first particle (in list order), then by group, each by counting
+    std::vector<int32_t> at((size_t)N + 1, 0), by_first((size_t)n);
+    for (int c = 0; c < n; c++) at[p[(size_t)arity * c] + 1]++;
+    for (int i = 0; i < N; i++) at[i + 1] += at[i];
+    for (int c = 0; c < n; c++) by_first[at[p[(size_t)arity * c]]++] = c;
     std::vector<int32_t> fill(ptr.begin(), ptr.end());
     order.assign((size_t)n, 0);
-    for (int c = 0; c < n; c++) order[fill[col[c]]++] = c;
-    for (int k = 0; k < ncol; k++)
-        std::stable_sort(order.begin() + ptr[k], order.begin() + ptr[k + 1], [&](int32_t x, int32_t y) {
-            return p[(size_t)arity * x] < p[(size_t)arity * y];
-        });
+    for (int32_t c : by_first) order[fill[col[c]]++] = c;
 }
 
 // Greedy colouring in list order.  Returns the colour count, -1 past 64.
@@ -90,7 +91,7 @@ int levels(int N, int n, int arity, const std::vector<int32_t>& p, std::vector<i
         for (int a = 0; a < arity; a++) last[p[(size_t)arity * c + a]] = l;
         nlev = std::max(nlev, l + 1);
     }
-    bucket(n, arity, p, lev, nlev, order, ptr);
+    bucket(N, n, arity, p, lev, nlev, order, ptr);
     return nlev;
 }
 
@@ -219,8 +220,8 @@ int oc_pbd_create(int32_t n_vertices, const float* x0, const uint8_t* pinned,
         const oc::PbdFamily bf{n_bending, 3, p->n_bcol, bp.data(), bcol.data()};
         const bool small = N <= oc::kPbdSmall;
         if (!oc::build_pbd_plan(N, x0, df, bf, small ? oc::kPbdSmall : oc::kPbdOwned, local, 4.0f, &plan)) {
-            bucket(n_distance, 2, dp, dcol, p->n_dcol, d_order, p->d_ptr);
-            bucket(n_bending, 3, bp, bcol, p->n_bcol, b_order, p->b_ptr);
+            bucket(N, n_distance, 2, dp, dcol, p->n_dcol, d_order, p->d_ptr);
+            bucket(N, n_bending, 3, bp, bcol, p->n_bcol, b_order, p->b_ptr);
         }
     }
     // rest lengths and k' of every constraint, in list order (PBD:148-178)

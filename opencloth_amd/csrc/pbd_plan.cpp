@@ -124,7 +124,7 @@ bool make_plan(int N, const float* x0, const PbdFamily& dist, const PbdFamily& b
             for (int c = ncol - 1; c >= 0 && ok; c--) {
                 const int f = c >= dist.ncol ? 1 : 0, ar = fam[f]->arity;
                 const size_t n0 = B.ids.size();
-                for (size_t k = 0; k < n0; k++) {
+                for (size_t k = 0; k < n0 && ok; k++) {
                     const int32_t e = con[(size_t)c * N + B.ids[k]];
                     if (e < 0 || seen[f][e] == b) continue;
                     seen[f][e] = b;
@@ -136,13 +136,16 @@ bool make_plan(int N, const float* x0, const PbdFamily& dist, const PbdFamily& b
                             B.ids.push_back(q);
                         }
                     }
+                    if ((int)B.ids.size() > max_local) ok = false;  // (for all blocks: the plan is refused)
                 }
+                work += (int64_t)B.cons[c].size();
+            }
+            for (int c = 0; c < ncol && ok; c++) {
+                const int f = c >= dist.ncol ? 1 : 0, ar = fam[f]->arity;
                 std::sort(B.cons[c].begin(), B.cons[c].end(), [&](int32_t x, int32_t y) {
                     const int32_t px = fam[f]->p[(size_t)ar * x], py = fam[f]->p[(size_t)ar * y];
                     return px != py ? px < py : x < y;
                 });
-                work += (int64_t)B.cons[c].size();
-                if ((int)B.ids.size() > max_local) ok = false;
             }
             std::sort(B.ids.begin() + own[b].size(), B.ids.end());
         }
