@@ -24,7 +24,7 @@ using oc::set_error;
 }  // namespace
 
 struct oc_vgrid_s {
-    int nx = 0, ny = 0, N = 0;
+    int nx = 0, ny = 0, N = 0, few = 0;
     oc_vgrid_params prm{};
     oc::StateIo io;
     hipStream_t stream = nullptr;
@@ -91,6 +91,7 @@ int oc_vgrid_create(int32_t width, int32_t height, const float* x0, const float*
     g->nx = width;
     g->ny = height;
     g->N = width * height;
+    g->few = oc::vgrid_few(width, height);
     g->prm = *params;
     const size_t N = g->N;
     const size_t vec = align_up(sizeof(float) * 3 * N), pl = align_up(sizeof(float) * N);
@@ -181,6 +182,7 @@ int oc_vgrid_step(oc_vgrid g, int32_t nsteps, float* vbo) {
     const oc::VgridScalars s = scalars(g);
     for (int k = 0; k < nsteps; k++) {
         oc::DevVgrid d;
+        d.few = g->few;
         d.nx = g->nx;
         d.ny = g->ny;
         d.N = g->N;

@@ -44,7 +44,14 @@ struct VgridShared {
     float wv[3][WY][WX];
 };
 
-template <int TX, int TY, bool VBO>
+// FEW: a few waves per SIMD, whose time is a vertex's own chain.  The springs'
+// forces go without a branch, so that their chains overlap (at 256x256, a wave
+// per SIMD, where a spring's chain is some 600 cycles: 8.1 us with a branch
+// around each, 7.0 without), and what the end of the step reads is loaded with
+// the window.  That takes 80 registers instead of 30; with more waves than
+// that leaves room for, which overlap as well, the branches are the better
+// form (1000x1000: 27.2 us, 28.6 without).
+template <int TX, int TY, bool VBO, bool FEW>
 __global__ __launch_bounds__(TX* TY) void k_vgrid(DevVgrid c, VgridScalars s) {
     constexpr int NT = TX * TY, H = 2;
     constexpr int WX = TX + 2 * H, WY = TY + 2 * H;
@@ -56,13 +63,11 @@ __global__ __launch_bounds__(TX* TY) void k_vgrid(DevVgrid c, VgridScalars s) {
     const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
     const int gi = bx * TX + lx, gj = by * TY + ly;
     const int N = c.N;
-    // what the end of the step reads, under way with the window's loads
     const bool own = gi < c.nx && gj < c.ny;
     const int i = own ? gj * c.nx + gi : 0;
-    const bool pinned = c.pin[i] != 0;
-    const V3 xl = ld3(c.xl, N, i);
-    float w = 0.0f;
-    if (VBO) w = c.w[i];
+    const bool early_pin = FEW ? c.pin[i] != 0 : false;
+    const V3 early_xl = FEW ? ld3(c.xl, N, i) : V3{0.0f, 0.0f, 0.0f};
+    const float early_w = FEW && VBO ? c.w[i] : 0.0f;
     const int x0 = bx * TX - H, y0 = by * TY - H;
 #pragma unroll
     for (int n = 0; n < NWIN; n++) {
@@ -92,25 +97,27 @@ __global__ __launch_bounds__(TX* TY) void k_vgrid(DevVgrid c, VgridScalars s) {
     const V3 vi = {sh.wv[0][cy][cx], sh.wv[1][cy][cx], sh.wv[2][cy][cx]};
     V3 F = {s.gx * s.mass + vi.x * s.damping, s.gy * s.mass + vi.y * s.damping,
             s.gz * s.mass + vi.z * s.damping};
-    // all springs' forces without a branch, so that their chains overlap (a
-    // wave per SIMD at 256x256, where a spring's chain, some 600 cycles, is
-    // the time: 8.1 us with a branch around each, 7.0 without); a spring
-    // beyond the grid's edge reads the window's zeros and is not added
-    V3 f[12];
+    V3 f[12];  // (FEW: a spring beyond the grid's edge reads the window's zeros and is not added)
 #pragma unroll
     for (int k = 0; k < 12; k++) {
-        const int wy = cy + vg_dy(k), wx = cx + vg_dx(k), cls = k >> 2;
+        const int dx = vg_dx(k), dy = vg_dy(k), cls = k >> 2;
+        if (!FEW && (gi + dx < 0 || gi + dx >= c.nx || gj + dy < 0 || gj + dy >= c.ny)) continue;
+        const int wy = cy + dy, wx = cx + dx;
         const V3 xj = {sh.wx[0][wy][wx], sh.wx[1][wy][wx], sh.wx[2][wy][wx]};
         const V3 vj = {sh.wv[0][wy][wx], sh.wv[1][wy][wx], sh.wv[2][wy][wx]};
         f[k] = spring_force(xi, xj, vi, vj, s.rest[k], s.ks[cls], s.kd[cls]);
+        if (!FEW) F = add3(F, f[k]);
     }
 #pragma unroll
-    for (int k = 0; k < 12; k++) {
+    for (int k = 0; FEW && k < 12; k++) {
         const int dx = vg_dx(k), dy = vg_dy(k);
         const bool have = gi + dx >= 0 && gi + dx < c.nx && gj + dy >= 0 && gj + dy < c.ny;
         const V3 g = add3(F, f[k]);
         F = {have ? g.x : F.x, have ? g.y : F.y, have ? g.z : F.z};
     }
+    const bool pinned = FEW ? early_pin : c.pin[i] != 0;
+    const V3 xl = FEW ? early_xl : ld3(c.xl, N, i);
+    const float w = FEW ? early_w : VBO ? c.w[i] : 0.0f;
     const V3 a = pinned ? V3{0.0f, 0.0f, 0.0f} : V3{F.x / s.mass, F.y / s.mass, F.z / s.mass};
     V3 xc = xi;
     if (xc.y < 0.0f) xc.y = 0.0f;
@@ -129,12 +136,26 @@ constexpr int kVgridTileX = 32, kVgridTileY = 8;
 
 hipError_t launch_vgrid(const DevVgrid& c, const VgridScalars& s, hipStream_t st) {
     constexpr int TX = kVgridTileX, TY = kVgridTileY;
-    const int nt = ((c.nx + TX - 1) / TX) * ((c.ny + TY - 1) / TY);
-    if (c.vbo)
-        hipLaunchKernelGGL((k_vgrid<TX, TY, true>), dim3(nt), dim3(TX * TY), 0, st, c, s);
+    const dim3 grid(((c.nx + TX - 1) / TX) * ((c.ny + TY - 1) / TY)), block(TX * TY);
+    if (c.few && c.vbo)
+        hipLaunchKernelGGL((k_vgrid<TX, TY, true, true>), grid, block, 0, st, c, s);
+    else if (c.few)
+        hipLaunchKernelGGL((k_vgrid<TX, TY, false, true>), grid, block, 0, st, c, s);
+    else if (c.vbo)
+        hipLaunchKernelGGL((k_vgrid<TX, TY, true, false>), grid, block, 0, st, c, s);
     else
-        hipLaunchKernelGGL((k_vgrid<TX, TY, false>), dim3(nt), dim3(TX * TY), 0, st, c, s);
+        hipLaunchKernelGGL((k_vgrid<TX, TY, false, false>), grid, block, 0, st, c, s);
     return hipGetLastError();
+}
+
+// Up to four waves per SIMD: 512x512 9.8 us a step against 9.95 with branches,
+// 576x576 12.8 and 12.5, 640x640 14.7 and 14.2.
+int vgrid_few(int nx, int ny) {
+    int dev = 0, cus = 0;
+    if (!hip_ok(hipGetDevice(&dev)) || !hip_ok(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)))
+        return 0;
+    const int64_t tiles = (int64_t)((nx + kVgridTileX - 1) / kVgridTileX) * ((ny + kVgridTileY - 1) / kVgridTileY);
+    return tiles <= 4 * (int64_t)cus;  // (a tile has a wave for each SIMD of a CU)
 }
 
 }  // namespace oc

@@ -447,7 +447,11 @@ struct DevVgrid {
     const uint8_t* pin;
     const float* w;   // w of the position buffer, carried into the vertex buffer
     float* vbo;       // NULL or N float4 (16-byte aligned)
+    int few;          // a few waves per SIMD (vgrid_few)
 };
+// Whether a grid leaves so few waves on the current device that its step's
+// time is a vertex's chain.
+int vgrid_few(int nx, int ny);
 struct VgridScalars {
     float mass, gx, gy, gz, damping, dt;
     float rest[12];  // rest length of stencil position k
