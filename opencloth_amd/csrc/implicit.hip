@@ -2173,8 +2173,12 @@ int persistent_cg_grid(const DevCloth& c) {
     return std::min(grid, c.nt);
 }
 
+// In a single iteration the blocks of a larger cloth do not win back what it
+// takes to load what they keep and to exchange sums once (a step of one
+// iteration, resident and with two launches: 512x512 53.7 and 48.4 us, 320x400
+// 42.2 and 37.9, but 256x256 31.8 and 33.1; of two: 320x400 48.1 and 49.5).
 static bool solves_resident(const DevCloth& c, const StepScalars& s) {
-    return c.res_vt && s.max_it > 0 && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION);
+    return c.res_vt && s.max_it > (c.nt > kRowTiles ? 1 : 0) && !(s.flags & OC_FLAG_CG_SINGLE_REDUCTION);
 }
 
 bool assembles_rows(const DevCloth& c, const StepScalars& s) {
