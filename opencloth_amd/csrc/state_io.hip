@@ -9,7 +9,8 @@
 // large ones (56 GB/s when device memory is copied to pinned memory; 24.6 MB
 // of 1023x1001 vertices in 640 us, 5.3 ms before) and the page faults of the
 // caller's fresh arrays.  Up to one slot both arrays of a state go in a
-// single launch with one synchronisation; beyond it, the host copy of one
+// single launch with one synchronisation, and one array alone by a copy where
+// that is quicker; beyond it, the host copy of one
 // slot overlaps the transfer of the next, and larger transfers have more host
 // threads with slots of their own.
 #include <algorithm>
@@ -29,6 +30,12 @@ constexpr size_t kSlot = 21846 * 48;          // bytes: about 1 MiB, whole verti
 // with arrays whose pages are there threads gain and lose nothing.
 constexpr size_t kPerThread = 2u << 20;
 constexpr int kThreads = 4;
+// One array of xyz of more than this, up to a slot, is transposed by the host
+// and copied: above 16 KiB the runtime's copy takes 9 us with its
+// synchronisation, where a launch that packs takes 14 (one array of 4096
+// vertices: 11 us, packed 16; of 16384: 17 and 21; below, 12 to 14 for the
+// copy alone).  Two arrays would be two copies.
+constexpr size_t kCopy = 16384;
 
 int threads_of(size_t total) { return (int)std::min<size_t>(kThreads, 1 + total / kPerThread); }
 
@@ -210,6 +217,20 @@ hipError_t StateIo::move(bool read, const IoArray* in, int n, hipStream_t st) {
     }
     if (na == 0 && !zeroed) return hipSuccess;
     hipError_t r = hipSuccess;
+    if (na == 1 && !a[0].w && a[0].bytes(a[0].n) > kCopy && total <= kSlot) {
+        if ((r = reserve(total)) != hipSuccess) return r;
+        const size_t m = a[0].n, bytes = a[0].bytes(m);
+        float *const s = (float*)pinned_, *const h = a[0].host;
+        for (size_t i = 0; !read && i < m; i++)
+            for (int k = 0; k < 3; k++) s[k * m + i] = h[3 * i + k];
+        r = read ? hipMemcpyAsync(s, a[0].planes, bytes, hipMemcpyDeviceToHost, st)
+                 : hipMemcpyAsync(a[0].planes, s, bytes, hipMemcpyHostToDevice, st);
+        const hipError_t rs = hipStreamSynchronize(st);
+        if (r == hipSuccess) r = rs;
+        for (size_t i = 0; read && r == hipSuccess && i < m; i++)
+            for (int k = 0; k < 3; k++) h[3 * i + k] = s[k * m + i];
+        return r;
+    }
     if (na > 0 && total <= kSlot) {
         if ((r = reserve(total)) != hipSuccess) return r;
         const Part p0 = part_of(a[0], 0, a[0].n), p1 = na > 1 ? part_of(a[1], 0, a[1].n) : Part{};
