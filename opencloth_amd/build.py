@@ -16,6 +16,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libopencloth.so")
+# The kernels use gfx950's instructions (lane swaps of 32 and 16); other values
+# are for variants of that target, not for other GPUs.
 ARCH = os.environ.get("OPENCLOTH_ARCH", "gfx950")
 
 # -ffp-contract=off: no FMA contraction, so the per-spring arithmetic follows

@@ -1396,11 +1396,12 @@ __global__ __launch_bounds__(TX* TY) void k_cg_axpy(DevCloth c, StepScalars s, i
 // for a block that never starts.
 //
 // Measured per iteration (30 to 40 iterations, two launches per iteration
-// before): 512x512 16.3 -> 7.1 us, 256x256 about 9 -> 4.3, 128x128 9.7 -> 3.9,
-// 21x21 7.1 -> 3.6.  An exchange takes 1.0 us between a few blocks and 1.7 to
+// before): 512x512 16.3 -> 7.7 us, 256x256 about 9 -> 4.4, 128x128 9.7 -> 3.9,
+// 21x21 7.1 -> 3.4.  An exchange takes 1.0 us between a few blocks and 1.7 to
 // 2.4 us among 256 (store to the coherence point, then polled loads of 512
-// words); the rest at 512x512, 2.9 us, is the arithmetic: 16 waves per CU
-// issue about 200 instructions each per iteration.
+// words); the rest at 512x512, about 3 us, is the arithmetic: 16 waves per CU
+// issue about 340 vector instructions each per iteration, 29% of the issue
+// slots of the whole solve.
 constexpr int kPollLimit = 1 << 21;              // polls of one exchange (seconds)
 
 // Grid barrier of the persistent solve's blocks: every block adds 1 to *bar and waits until it reaches target.  The add is a

@@ -563,7 +563,9 @@ hipError_t launch_pbd_tiled(const DevPbd& c, const PbdScalars& s, int iterations
 // Tile shape of the implicit kernels (one workgroup per tile; a multiple of
 // 64 threads).  The reduction order depends on it; oc_cloth_tile_shape
 // reports it.  64x8 measured fastest at 512x512 among 32x8, 32x16, 32x32,
-// 64x4, 64x8, 64x16, 128x4 and 128x8.
+// 64x4, 64x8, 64x16, 128x4 and 128x8, with a launch per kernel and iteration.
+// The width is no longer free: the resident solve and the half-tile assembly
+// take a row of a tile for one wave and refuse to compile with another width.
 #ifndef OC_TILE_X
 #define OC_TILE_X 64
 #endif

@@ -265,10 +265,11 @@ constexpr int kVerletTileX = 32, kVerletTileY = 8;
 // that ends without its word sets *err and every block leaves.
 //
 // Measured per step of 200, with the collider, a launch each for step and
-// collider before: 512x512 14.2 -> 6.5 us, 256x256 12 -> 4.6, 21x21 8.4 ->
-// 3.9.  About 1 us of it is the exchange; the rest is the chain through a step
+// collider before: 512x512 14.2 -> 6.3 us, 256x256 12 -> 4.5, 21x21 8.4 ->
+// 3.6.  About 1 us of it is the exchange; the rest is the chain through a step
 // (six springs with a square root and two divisions each, the sum over
-// twelve, three barriers), at 512x512 with four waves per SIMD to issue.
+// twelve, three barriers), at 512x512 with four waves per SIMD to issue (635
+// vector instructions per wave and step, 69% of the issue slots).
 constexpr int kVerletPolls = 1 << 21;  // seconds
 
 template <int T>
@@ -639,8 +640,8 @@ static bool verlet_seconds_fit(int nx, int ny, const uint32_t* mask) {
 }
 
 // The smaller regions while each has a CU of its own (a wave per SIMD: 256x256
-// 4.6 us per step, in 32x32 regions 5.2; 128x128 4.1 and 5.2), then the larger
-// ones (512x512 6.5 us, in 1024 small regions, four per CU, 7.0).
+// 4.5 us per step, in 32x32 regions 5.2; 128x128 3.8 and 5.2), then the larger
+// ones (512x512 6.3 us, in 1024 small regions, four per CU, 7.0).
 int verlet_resident_region(int nx, int ny, const uint32_t* mask) {
     if (verlet_regions(nx, ny, 16) <= verlet_blocks_fit<16>() && verlet_seconds_fit<16>(nx, ny, mask)) return 16;
     if (verlet_regions(nx, ny, 32) <= verlet_blocks_fit<32>() && verlet_seconds_fit<32>(nx, ny, mask)) return 32;
